@@ -15,7 +15,23 @@
 //             torch's
 //
 // One (token, kv_head) row per D/8 lanes, 16 bytes (8 fp16) per lane; the
-// int8 row maximum is a xor-shuffle reduction inside those lanes.
+// int8 row maximum is a DPP reduction inside those lanes. A workgroup holds
+// whole tokens (or, above 256 lanes a token, a 256-lane part of one), so a
+// lane finds its token and head without an integer division; K, V and the
+// slot are loaded together, before anything waits.
+//
+// What bounds it: HBM (read and write) for large writes, the launch and one
+// round trip for a decode step's. The form with two 64-bit divisions a lane, K
+// and V one after the other and ~15 VALU instructions per int8 element was
+// bound by issue. The bytes go out with non-temporal stores (16,384 fp16 rows
+// 28.9 us without); the rows come in with plain loads, since the projection
+// that made them has just left them in a cache (non-temporal loads: 2-6% faster
+// on rows from HBM, up to 8% slower on cached ones). Graph-timed at the
+// Llama-3-8B shape (8 kv heads, head_dim 128), before -> after:
+//   16,384 tokens: fp16 29.1 -> 25.0 us, fp8 25.2 -> 20.7, int8 with fp32
+//     scales 32.1 -> 22.4 (4.6 TB/s; a large device copy runs at 4.7);
+//   64 tokens: fp16 2.42 -> 2.29, fp8 3.20 -> 2.33, int8 3.89 -> 2.90 (an empty
+//     kernel in a graph takes 1.6).
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -27,6 +43,7 @@ namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
 struct WParams {
   const uint8_t *key;
@@ -36,13 +53,29 @@ struct WParams {
   uint8_t *ks;
   uint8_t *vs;
   const int64_t *slots;
-  int64_t rows;            // num_tokens * num_kv_heads
-  int32_t hkv, block_size;
+  uint32_t tokens;
+  uint32_t lanes;      // lanes of one token: num_kv_heads * head_dim / 8
+  uint32_t tpb;        // tokens per group of 256 lanes (1 when a token takes several groups)
+  uint32_t parts;      // groups per token (1 when a group holds whole tokens)
+  uint32_t groups;     // all groups; workgroup i takes groups i, i + gridDim.x, ...
+  uint32_t inv_lanes;  // ceil(2^16 / lanes): x / lanes = x * inv_lanes >> 16 for x < 256, lanes <= 256
+  int32_t block_size;
+  int32_t log2_block;  // -1: block_size is not a power of two
   int64_t max_slot;        // num_blocks * block_size
   int64_t skt, skh, svt, svh;  // bytes
   int64_t scn, sct, sch;       // bytes
   int64_t ssn, sst;            // bytes
 };
+
+// Index times stride, added to base: 32 x 32 -> 64 bits (one v_mad_u64_u32) or
+// 64-bit throughout.
+template <bool WIDE>
+__device__ __forceinline__ uint64_t at(uint64_t base, uint64_t index, int64_t stride) {
+  if constexpr (WIDE) return base + index * (uint64_t)stride;
+  return base + (uint64_t)(uint32_t)index * (uint32_t)stride;
+}
+
+constexpr int64_t kMaxGrid = 1 << 14;  // workgroups of a launch; more groups than that loop
 
 // fp16 bit pattern -> e5m2 byte, round to nearest even on the dropped byte.
 __device__ __forceinline__ uint32_t half_to_e5m2(uint32_t h) {
@@ -52,85 +85,175 @@ __device__ __forceinline__ uint32_t half_to_e5m2(uint32_t h) {
   return sign | ((mag + 0x7fu + ((mag >> 8) & 1u)) >> 8);
 }
 
+// Two fp16 patterns, rounded so that bytes 1 and 3 are their e5m2 bytes: the
+// same sum as half_to_e5m2 on 16-bit halves (for anything but NaN it cannot
+// carry out of the magnitude, so the sign stays).
+__device__ __forceinline__ uint32_t round_halves_e5m2(uint32_t w) {
+  const u16x2 h = __builtin_bit_cast(u16x2, w);
+  const u16x2 odd = __builtin_bit_cast(u16x2, (w >> 8) & 0x00010001u);
+  return __builtin_bit_cast(uint32_t, h + u16x2{0x7f, 0x7f} + odd);
+}
+
 __device__ __forceinline__ float half_bits_to_float(uint32_t h) {
   return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
 }
 
-template <int KV, int SC, int D>
+// x combined by max with the value of the lane that DPP control CTRL names (the
+// lanes of a row are all active), on the bits of non-negative floats, which
+// order as integers do: one v_max_u32 each.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_max(uint32_t x) {
+  const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, true);
+  return x > y ? x : y;
+}
+
+// Maximum of a non-negative float over the LANES (4, 8, 16 or 32) neighbouring lanes of a row.
+template <int LANES>
+__device__ __forceinline__ float row_max(float f) {
+  uint32_t x = __builtin_bit_cast(uint32_t, f);
+  x = dpp_max<0xB1>(x);                              // quad_perm 1,0,3,2
+  x = dpp_max<0x4E>(x);                              // quad_perm 2,3,0,1
+  if constexpr (LANES >= 8) x = dpp_max<0x141>(x);   // row_half_mirror: the other quad of 8
+  if constexpr (LANES >= 16) x = dpp_max<0x140>(x);  // row_mirror: the other 8 of 16
+  f = __builtin_bit_cast(float, x);
+  if constexpr (LANES >= 32) f = fmaxf(f, __shfl_xor(f, 16));
+  return f;
+}
+
+// 16 bytes of fp16 -> 8 e5m2 bytes.
+__device__ __forceinline__ u32x2 to_e5m2(u32x4 w) {
+  // a NaN anywhere in the lane (its magnitude above infinity's) takes the
+  // form that tests each value
+  u16x2 m = __builtin_bit_cast(u16x2, w.x & 0x7fff7fffu);
+  m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, w.y & 0x7fff7fffu));
+  m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, w.z & 0x7fff7fffu));
+  m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2, w.w & 0x7fff7fffu));
+  if (__builtin_expect(m[0] > 0x7c00u || m[1] > 0x7c00u, 0)) {
+    uint32_t b[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) b[i] = half_to_e5m2(i & 1 ? w[i / 2] >> 16 : w[i / 2] & 0xffffu);
+    return u32x2{b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24),
+                 b[4] | (b[5] << 8) | (b[6] << 16) | (b[7] << 24)};
+  }
+  // v_perm: bytes 1, 3 of the first word, then of the second
+  return u32x2{__builtin_amdgcn_perm(round_halves_e5m2(w.y), round_halves_e5m2(w.x), 0x07050301u),
+               __builtin_amdgcn_perm(round_halves_e5m2(w.w), round_halves_e5m2(w.z), 0x07050301u)};
+}
+
+// a / 127 correctly rounded, for a = |fp16| or 1e-6f (every such value is
+// checked against the division in tests/test_cache_write_math.py): the product
+// with 1/127 corrected once by its exact remainder; infinity as it is.
+__device__ __forceinline__ float div127(float a) {
+  constexpr float kInv = 1.0f / 127.0f;
+  const float q = a * kInv;
+  return a < __builtin_inff() ? __builtin_fmaf(__builtin_fmaf(-q, 127.0f, a), kInv, q) : a;
+}
+
+// 16 bytes of fp16 -> 8 int8 bytes and the row's scale.
+template <int SC, int LANES>
+__device__ __forceinline__ u32x2 to_int8(u32x4 w, float &scale) {
+  float x[8];
+  float amax = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    x[i] = half_bits_to_float(i & 1 ? w[i / 2] >> 16 : w[i / 2] & 0xffffu);
+    // (emits nothing: keeps the products below from becoming v_fma_mix, which
+    // takes the fp16 value itself at half the rate)
+    asm("" : "+v"(x[i]));
+    amax = fmaxf(amax, fabsf(x[i]));
+  }
+  amax = fmaxf(row_max<LANES>(amax), 1e-6f);
+  scale = div127(amax);
+  if constexpr (SC == PA_SCALE_FP16) scale = (float)(_Float16)scale;
+  // round_half_even(x / scale) with the IEEE quotient's rounding: x times the
+  // scale's reciprocal (v_rcp_f32, 1 ulp) is within 2 * 2^-23 of x / scale,
+  // relatively, so for a quotient up to 127.5 the two round to different
+  // integers only within 2^-15 of a half-integer. x * inv + 1.5 * 2^23 rounds
+  // the product to an integer, half to even, and leaves it in the low mantissa
+  // byte. A lane takes the division form when an element is within 2^-14 of a
+  // half-integer, when one is NaN (__builtin_elementwise_maximum hands it on),
+  // or when the row's largest quotient is 127.4 or more (infinities, and fp16
+  // scales that rounded far down or to zero).
+  const float inv = __builtin_amdgcn_rcpf(scale);
+  constexpr float kMagic = 12582912.0f;
+  uint32_t t[8];
+  float off = __builtin_elementwise_maximum(__builtin_fmaf(amax, inv, -126.9f), 0.0f);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float r = __builtin_fmaf(x[i], inv, kMagic);
+    t[i] = __builtin_bit_cast(uint32_t, r);
+    off = __builtin_elementwise_maximum(off, fabsf(__builtin_fmaf(x[i], inv, kMagic - r)));
+  }
+  if (__builtin_expect(!(off < 0.5f - 0x1p-14f), 0)) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float r = rintf(x[i] / scale);
+      // a zero row with fp16 scales underflows the scale to 0: 0/0 is NaN,
+      // which the reference's cast to int8 stores as 0
+      const float q = (r != r) ? 0.f : fminf(fmaxf(r, -127.f), 127.f);
+      t[i] = (uint32_t)(int32_t)q;
+    }
+  }
+  // the low bytes, four to a word
+  const uint32_t a = __builtin_amdgcn_perm(t[1], t[0], 0x0c0c0400u), b = __builtin_amdgcn_perm(t[3], t[2], 0x04000c0cu);
+  const uint32_t c = __builtin_amdgcn_perm(t[5], t[4], 0x0c0c0400u), d = __builtin_amdgcn_perm(t[7], t[6], 0x04000c0cu);
+  return u32x2{a | b, c | d};
+}
+
+// WIDE: some stride is 4 GiB or more, or block_size is not a power of two (64-bit
+// products and divisions); otherwise strides and block ids fit 32 bits.
+template <int KV, int SC, int D, bool WIDE>
 __global__ void __launch_bounds__(256) cache_write_kernel(const WParams p) {
   constexpr int kLanesPerRow = D / 8;  // 8 fp16 (16 bytes) per lane
-  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t row = gid / kLanesPerRow;
-  const int piece = (int)(gid % kLanesPerRow);
-  bool live = row < p.rows;
-  const int64_t t = live ? row / p.hkv : 0;
-  const int h = live ? (int)(row % p.hkv) : 0;
-  const int64_t slot = live ? p.slots[t] : -1;
-  live = live && slot >= 0 && slot < p.max_slot;  // uniform across the row's lanes
-  const int64_t blk = live ? slot / p.block_size : 0;
-  const int64_t off = live ? slot % p.block_size : 0;
-  const int64_t cbase = blk * p.scn + off * p.sct + h * p.sch;
+  const uint32_t tid = threadIdx.x;
+  for (uint32_t g = blockIdx.x; g < p.groups; g += gridDim.x) {
+    uint32_t t, lane;  // token, lane in the token
+    if (p.lanes <= 256) {
+      const uint32_t tb = tid * p.inv_lanes >> 16;
+      if (tb >= p.tpb) return;
+      t = g * p.tpb + tb;
+      lane = tid - tb * p.lanes;
+    } else {
+      t = g / p.parts;
+      lane = (g % p.parts) * 256u + tid;
+    }
+    // (all these tests are uniform over a row's lanes)
+    if (lane >= p.lanes || t >= p.tokens) continue;
+    const uint32_t h = lane / kLanesPerRow, piece = lane % kLanesPerRow;
+
+    const int64_t slot = p.slots[t];
+    u32x4 w[2];
+    w[0] = *reinterpret_cast<const u32x4 *>(
+        p.key + at<WIDE>(at<WIDE>(piece * 16, h, p.skh), t, p.skt));
+    w[1] = *reinterpret_cast<const u32x4 *>(
+        p.value + at<WIDE>(at<WIDE>(piece * 16, h, p.svh), t, p.svt));
+    // both rows are in flight with the slot: without this (it emits nothing)
+    // the compiler moves their loads behind the slot's arrival
+    asm volatile("" : : "v"(w[0]), "v"(w[1]));
+    if (slot < 0 || slot >= p.max_slot) continue;
+    uint64_t blk, off;
+    if constexpr (WIDE) {
+      blk = (uint64_t)slot / (uint32_t)p.block_size;
+      off = (uint64_t)slot % (uint32_t)p.block_size;
+    } else {
+      blk = (uint64_t)slot >> p.log2_block;
+      off = (uint32_t)slot & (uint32_t)(p.block_size - 1);
+    }
+    constexpr int kPiece = (KV == PA_KV_FP16 || KV == PA_KV_BF16) ? 16 : 8;  // bytes a lane stores
+    const uint64_t cbase = at<WIDE>(at<WIDE>(at<WIDE>(piece * kPiece, h, p.sch), off, p.sct), blk, p.scn);
 
 #pragma unroll
-  for (int which = 0; which < 2; ++which) {
-    const uint8_t *src = (which ? p.value : p.key) + t * (which ? p.svt : p.skt) +
-                         h * (which ? p.svh : p.skh) + piece * 16;
-    uint8_t *dst = which ? p.vc : p.kc;
-    u32x4 w = {0u, 0u, 0u, 0u};
-    if (live) w = *reinterpret_cast<const u32x4 *>(src);
-    uint32_t hv[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      hv[2 * i] = w[i] & 0xffffu;
-      hv[2 * i + 1] = w[i] >> 16;
-    }
-    if constexpr (KV == PA_KV_FP16 || KV == PA_KV_BF16) {
-      if (live) *reinterpret_cast<u32x4 *>(dst + cbase + piece * 16) = w;
-    } else if constexpr (KV == PA_KV_FP8_E5M2) {
-      uint32_t b[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) b[i] = half_to_e5m2(hv[i]);
-      const u32x2 o = {b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24),
-                       b[4] | (b[5] << 8) | (b[6] << 16) | (b[7] << 24)};
-      if (live) *reinterpret_cast<u32x2 *>(dst + cbase + piece * 8) = o;
-    } else {
-      float x[8];
-      float amax = 0.f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        x[i] = half_bits_to_float(hv[i]);
-        amax = fmaxf(amax, fabsf(x[i]));
-      }
-#pragma unroll
-      for (int o = kLanesPerRow / 2; o >= 1; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
-      amax = fmaxf(amax, 1e-6f);
-      // IEEE division (the default for float `/` in HIP device code)
-      float scale = amax / 127.0f;
-      if constexpr (SC == PA_SCALE_FP16) scale = (float)(_Float16)scale;
-      // round_half_even(x / scale) with the IEEE quotient's rounding: x times
-      // the row's reciprocal is within 1.5 ulp of the correctly rounded
-      // quotient, so the two can round to different integers only next to a
-      // half-integer; those (rare) elements take the IEEE division
-      const float inv = 1.0f / scale;
-      uint32_t b[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float q0 = x[i] * inv;
-        const float frac = q0 - floorf(q0);
-        const float tol = fabsf(q0) * 0x1p-20f + 0x1p-40f;
-        float r = rintf(q0);
-        if (fabsf(frac - 0.5f) <= tol) r = rintf(x[i] / scale);
-        // a zero row with fp16 scales underflows the scale to 0: 0/0 is NaN,
-        // which the reference's cast to int8 stores as 0
-        const float q = (r != r) ? 0.f : fminf(fmaxf(r, -127.f), 127.f);
-        b[i] = (uint32_t)(int32_t)q & 0xffu;
-      }
-      const u32x2 o = {b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24),
-                       b[4] | (b[5] << 8) | (b[6] << 16) | (b[7] << 24)};
-      if (live) {
-        *reinterpret_cast<u32x2 *>(dst + cbase + piece * 8) = o;
+    for (int which = 0; which < 2; ++which) {
+      uint8_t *dst = (which ? p.vc : p.kc) + cbase;
+      if constexpr (KV == PA_KV_FP16 || KV == PA_KV_BF16) {
+        __builtin_nontemporal_store(w[which], reinterpret_cast<u32x4 *>(dst));
+      } else if constexpr (KV == PA_KV_FP8_E5M2) {
+        __builtin_nontemporal_store(to_e5m2(w[which]), reinterpret_cast<u32x2 *>(dst));
+      } else {
+        float scale;
+        __builtin_nontemporal_store(to_int8<SC, kLanesPerRow>(w[which], scale), reinterpret_cast<u32x2 *>(dst));
         if (piece == 0) {
-          uint8_t *s = (which ? p.vs : p.ks) + blk * p.ssn + off * p.sst;
+          uint8_t *s = (which ? p.vs : p.ks) + at<WIDE>(at<WIDE>(0, off, p.sst), blk, p.ssn);
           if constexpr (SC == PA_SCALE_FP16) {
             reinterpret_cast<_Float16 *>(s)[h] = (_Float16)scale;
           } else {
@@ -142,13 +265,24 @@ __global__ void __launch_bounds__(256) cache_write_kernel(const WParams p) {
   }
 }
 
+template <int KV, int SC, int D>
+void launch_d(const WParams &p, dim3 grid, hipStream_t st) {
+  const int64_t big = int64_t(1) << 32;
+  const bool wide = p.log2_block < 0 || p.skt >= big || p.skh >= big || p.svt >= big || p.svh >= big ||
+                    p.scn >= big || p.sct >= big || p.sch >= big || p.ssn >= big || p.sst >= big;
+  if (wide)
+    hipLaunchKernelGGL((cache_write_kernel<KV, SC, D, true>), grid, dim3(256), 0, st, p);
+  else
+    hipLaunchKernelGGL((cache_write_kernel<KV, SC, D, false>), grid, dim3(256), 0, st, p);
+}
+
 template <int KV, int SC>
-hipError_t launch_w(const WParams &p, int d, int grid, hipStream_t st) {
+hipError_t launch_w(const WParams &p, int d, dim3 grid, hipStream_t st) {
   switch (d) {
-    case 32: hipLaunchKernelGGL((cache_write_kernel<KV, SC, 32>), dim3(grid), dim3(256), 0, st, p); break;
-    case 64: hipLaunchKernelGGL((cache_write_kernel<KV, SC, 64>), dim3(grid), dim3(256), 0, st, p); break;
-    case 128: hipLaunchKernelGGL((cache_write_kernel<KV, SC, 128>), dim3(grid), dim3(256), 0, st, p); break;
-    default: hipLaunchKernelGGL((cache_write_kernel<KV, SC, 256>), dim3(grid), dim3(256), 0, st, p); break;
+    case 32: launch_d<KV, SC, 32>(p, grid, st); break;
+    case 64: launch_d<KV, SC, 64>(p, grid, st); break;
+    case 128: launch_d<KV, SC, 128>(p, grid, st); break;
+    default: launch_d<KV, SC, 256>(p, grid, st); break;
   }
   return hipGetLastError();
 }
@@ -193,9 +327,11 @@ extern "C" int pa_cache_write(const pa_cache_write_args *a, void *stream) {
     return pa_fail(PA_ERR_INVALID, "scale_dtype must be PA_SCALE_NONE for kv_dtype %d", a->kv_dtype);
   }
   const int64_t rows = (int64_t)a->num_tokens * a->num_kv_heads;
-  const int64_t lanes = rows * (a->head_dim / 8);
-  const int64_t grid = (lanes + 255) / 256;
-  if (grid > 0x7fffffff) return pa_fail(PA_ERR_UNSUPPORTED, "too many rows (%lld)", (long long)rows);
+  const int64_t lanes = (int64_t)a->num_kv_heads * (a->head_dim / 8);  // of one token
+  const int64_t tpb = lanes <= 256 ? 256 / lanes : 1, parts = (lanes + 255) / 256;
+  const int64_t groups = (a->num_tokens + tpb - 1) / tpb * parts;
+  if (lanes > 0xffffff00u || groups > 0x7fffffff)
+    return pa_fail(PA_ERR_UNSUPPORTED, "too many rows (%lld)", (long long)rows);
   if (rows == 0) return pa_ok();
 
   WParams p;
@@ -206,9 +342,16 @@ extern "C" int pa_cache_write(const pa_cache_write_args *a, void *stream) {
   p.ks = static_cast<uint8_t *>(a->k_scale);
   p.vs = static_cast<uint8_t *>(a->v_scale);
   p.slots = a->slot_mapping;
-  p.rows = rows;
-  p.hkv = a->num_kv_heads;
+  p.tokens = (uint32_t)a->num_tokens;
+  p.lanes = (uint32_t)lanes;
+  p.tpb = (uint32_t)tpb;
+  p.parts = (uint32_t)parts;
+  p.groups = (uint32_t)groups;
+  p.inv_lanes = lanes <= 256 ? (65536u + (uint32_t)lanes - 1) / (uint32_t)lanes : 0;
   p.block_size = a->block_size;
+  p.log2_block = -1;
+  if ((a->block_size & (a->block_size - 1)) == 0)
+    for (p.log2_block = 0; (1 << p.log2_block) < a->block_size;) ++p.log2_block;
   p.max_slot = (int64_t)a->num_blocks * a->block_size;
   p.skt = a->stride_kt * 2;
   p.skh = a->stride_kh * 2;
@@ -219,14 +362,15 @@ extern "C" int pa_cache_write(const pa_cache_write_args *a, void *stream) {
   p.sch = a->stride_ch * elem;
   p.ssn = a->stride_sn * sb;
   p.sst = a->stride_st * sb;
+  const dim3 grid((uint32_t)(groups < kMaxGrid ? groups : kMaxGrid));
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int d = a->head_dim;
   hipError_t e;
-  if (a->kv_dtype == PA_KV_FP16) e = launch_w<PA_KV_FP16, PA_SCALE_NONE>(p, d, (int)grid, st);
-  else if (a->kv_dtype == PA_KV_BF16) e = launch_w<PA_KV_BF16, PA_SCALE_NONE>(p, d, (int)grid, st);
-  else if (a->kv_dtype == PA_KV_FP8_E5M2) e = launch_w<PA_KV_FP8_E5M2, PA_SCALE_NONE>(p, d, (int)grid, st);
-  else if (a->scale_dtype == PA_SCALE_FP32) e = launch_w<PA_KV_INT8, PA_SCALE_FP32>(p, d, (int)grid, st);
-  else e = launch_w<PA_KV_INT8, PA_SCALE_FP16>(p, d, (int)grid, st);
+  if (a->kv_dtype == PA_KV_FP16) e = launch_w<PA_KV_FP16, PA_SCALE_NONE>(p, d, grid, st);
+  else if (a->kv_dtype == PA_KV_BF16) e = launch_w<PA_KV_BF16, PA_SCALE_NONE>(p, d, grid, st);
+  else if (a->kv_dtype == PA_KV_FP8_E5M2) e = launch_w<PA_KV_FP8_E5M2, PA_SCALE_NONE>(p, d, grid, st);
+  else if (a->scale_dtype == PA_SCALE_FP32) e = launch_w<PA_KV_INT8, PA_SCALE_FP32>(p, d, grid, st);
+  else e = launch_w<PA_KV_INT8, PA_SCALE_FP16>(p, d, grid, st);
   if (e != hipSuccess) return pa_fail(PA_ERR_HIP, "cache write launch failed: %s", hipGetErrorString(e));
   return pa_ok();
 }

@@ -194,3 +194,58 @@ def test_repeated_writes_through_the_argument_cache(kv_dtype):
     assert torch.equal(_raw(c.k_cache.cpu()), _raw(ref.k_cache))  # c untouched
     with pytest.raises(ValueError, match="int64"):
         reshape_and_cache(key.cuda(), key.cuda(), c2, slots.to(torch.int32).cuda())
+
+
+@pytest.mark.parametrize("hkv,d,page,tokens", [
+    (3, 64, 16, 21),      # 24 lanes a token: 10 tokens and 16 idle lanes a workgroup
+    (5, 32, 32, 300),     # 20 lanes a token
+    (7, 128, 16, 19),     # 112 lanes a token, two tokens a workgroup
+    (9, 256, 16, 5),      # 288 lanes: a token over two workgroups, the second partly idle
+    (40, 128, 16, 3),     # 640 lanes: two and a half workgroups
+    (2, 128, 24, 77),     # a page that is no power of two: the 64-bit form
+    (8, 256, 16, 16390),  # more groups than the grid holds: workgroups loop
+])
+@pytest.mark.parametrize("kv_dtype,scale_dtype", [("fp16", None), ("fp8_e5m2", None), ("int8", torch.float16),
+                                                  ("int8", torch.float32)])
+def test_write_geometry_edges(kv_dtype, scale_dtype, hkv, d, page, tokens):
+    """Bytes equal the oracle's where a token's lanes do not divide the workgroup, exceed it, or
+    the launch loops; rows are slices of one tensor, as a fused projection leaves them."""
+    if tokens > 1000 and kv_dtype not in ("fp8_e5m2",):
+        tokens = tokens if scale_dtype == torch.float32 else 40  # one looping case per arithmetic
+    blocks = -(-tokens // page) + 2
+    shape = ModelShape(hkv, hkv, d, "e")
+    kw = {} if scale_dtype is None else {"scale_dtype": scale_dtype}
+    c = allocate(shape, 1, [blocks * page], block_size=page, kv_dtype=kv_dtype, seed=51, device="cuda",
+                 fill_device="cuda", **kw)
+    ref = _cpu_copy(c)
+    g = torch.Generator(device="cuda").manual_seed(52)
+    rows = torch.randn((tokens, 2 * hkv, d), generator=g, device="cuda").half()
+    rows[0, 0] = 0                                                  # the 1e-6 floor
+    rows[1, 0] *= 2.0 ** -20                                        # fp16 scales round far down
+    slots = torch.randperm(blocks * page, generator=g, device="cuda")[:tokens]
+    slots[2] = -1
+    reshape_and_cache(rows[:, :hkv], rows[:, hkv:], c, slots)
+    oracle.write_kv(rows[:, :hkv].cpu(), rows[:, hkv:].cpu(), ref, slots.cpu())
+    assert torch.equal(_raw(c.k_cache.cpu()), _raw(ref.k_cache))
+    assert torch.equal(_raw(c.v_cache.cpu()), _raw(ref.v_cache))
+    if scale_dtype is not None:
+        assert torch.equal(c.k_scale.cpu(), ref.k_scale) and torch.equal(c.v_scale.cpu(), ref.v_scale)
+
+
+@pytest.mark.parametrize("scale_dtype", [torch.float16, torch.float32])
+def test_int8_rows_with_nan_and_infinity(scale_dtype):
+    """A NaN is stored as 0 and does not enter the row's maximum; an infinity gives an infinite
+    scale and zeros (finite / inf, and inf / inf as a NaN)."""
+    c = allocate(ModelShape(1, 1, 64, "n"), 1, [16], kv_dtype="int8", scale_dtype=scale_dtype, seed=53,
+                 device="cuda", shuffle=False)
+    g = torch.Generator().manual_seed(54)
+    rows = torch.randn((3, 1, 64), generator=g).half()
+    clean = rows.clone()
+    clean[0, 0, 5] = 0
+    rows[0, 0, 5] = float("nan")
+    rows[1, 0, 9] = float("-inf")
+    reshape_and_cache(rows.cuda(), rows.cuda(), c, torch.arange(3, device="cuda"))
+    want, scale = oracle.quantize_kv(clean, "int8", scale_dtype)
+    assert torch.equal(c.k_cache[0, [0, 2]].cpu(), want[[0, 2]])
+    assert torch.equal(c.k_scale[0, [0, 2]].cpu(), scale[[0, 2]])
+    assert bool((c.k_cache[0, 1] == 0).all()) and bool(torch.isinf(c.k_scale[0, 1]).all())
