@@ -137,6 +137,9 @@ struct KParams {
   int32_t sbtb;              // elements
   float qk_scale;            // sm_scale * log2(e)
   int32_t io_bf16;           // q and out are bf16 (else fp16)
+  // Neighbouring kv heads that one wave takes as one of pack times the head
+  // dim: then hkv counts packs, and group and skh are a pack's.
+  int32_t pack;
 };
 
 struct RParams {
@@ -306,13 +309,16 @@ __device__ __forceinline__ void buf_load_bytes(uint32_t *w, __amdgpu_buffer_rsrc
   }
 }
 
-// The bits of one scale (fp16 scales in the low half).
-template <int SC>
-__device__ __forceinline__ uint32_t load_scale_bits(__amdgpu_buffer_rsrc_t r, uint32_t voff) {
-  if constexpr (SC == PA_SCALE_FP32) {
-    return __builtin_amdgcn_raw_buffer_load_b32(r, voff, 0, 0);
+// The bits of the scales of PK (1 or 2) neighbouring heads: fp32 scales one a
+// word, fp16 scales in word 0 (one: in the low half; two: low, high).
+template <int SC, int PK>
+__device__ __forceinline__ u32x2 load_scale_bits(__amdgpu_buffer_rsrc_t r, uint32_t voff) {
+  if constexpr (SC == PA_SCALE_FP32 && PK == 2) {
+    return __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0, 0);
+  } else if constexpr (SC == PA_SCALE_FP32 || PK == 2) {
+    return u32x2{__builtin_amdgcn_raw_buffer_load_b32(r, voff, 0, 0), 0u};
   } else {
-    return __builtin_amdgcn_raw_buffer_load_b16(r, voff, 0, 0);
+    return u32x2{__builtin_amdgcn_raw_buffer_load_b16(r, voff, 0, 0), 0u};
   }
 }
 
@@ -323,6 +329,16 @@ __device__ __forceinline__ uint32_t load_scale_bits(__amdgpu_buffer_rsrc_t r, ui
 // where a vector load's (vmcnt) would wait for them.
 typedef __attribute__((address_space(4))) const int32_t ro_i32;
 __device__ __forceinline__ const ro_i32 *ro(const int32_t *ptr) { return (const ro_i32 *)ptr; }
+
+// The kernel's parameters (its first argument), to be read from here on: what
+// an epilogue needs is then loaded in the epilogue instead of being held in
+// scalar registers through the tile loop.
+__device__ __forceinline__ const KParams &late_params() {
+  typedef __attribute__((address_space(4))) const KParams ro_params;
+  auto k = (ro_params *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(k));
+  return *(const KParams *)k;
+}
 
 // Compile-time geometry for one (KV dtype, head_dim) instance.
 //
@@ -352,7 +368,7 @@ struct Geo {
   static constexpr int kKLoads = kTT / kKRowsPerLoad;       // K loads per tile
   static constexpr int kKSlotStride = kRowBytes + 16;       // padded LDS row
   static constexpr int kKSlotBytes = kTT * kKSlotStride;    // per wave
-  static constexpr int kScales = 2 * kTT;                   // int8: K and V scales per tile
+  static constexpr int kScales = 2 * kTT;                   // int8: K and V scales per tile (and kv head)
   // double-buffer the tile registers unless, with the accumulators and the Q
   // operands, they would crowd out the rest (the budget is set by the
   // largest instance that measured best double-buffered: fp16 at D = 128)
@@ -361,12 +377,12 @@ struct Geo {
 };
 
 // Registers of one tile of one wave.
-template <int KV, int D>
+template <int KV, int D, int PK>
 struct Tile {
   using G = Geo<KV, D>;
   u32x4 k[G::kKLoads];               // K: 16 bytes of row (i*rows_per_load + lane/lanes_per_row)
   uint32_t v[G::kVRows][G::kVWords]; // V row 4c + (e & 3) of sub-tile e >> 2, elems kE*r16..
-  float sc[G::kScales / 64];         // int8: scale j*64 + lane of the tile's (K|V, sub-tile, row)
+  float sc[PK];                      // int8: scale `lane` of packed head j's (K|V, sub-tile, row)
 };
 
 // The loop-invariant parts of a wave's tile addresses (one kv head): bases
@@ -381,15 +397,15 @@ struct TileAddr {
   uint32_t s_mask[4];      // int8 scale: all ones in lane group lane / 16, else zero
 };
 
-template <int KV, int SC, int D>
+template <int KV, int SC, int D, int PK>
 __device__ __forceinline__ TileAddr<KV, D> tile_addr(const KParams &p, int kvh, int lane) {
   using G = Geo<KV, D>;
   TileAddr<KV, D> a;
   const uint32_t skt = (uint32_t)p.skt;
   a.k = p.k + (int64_t)kvh * p.skh;
   a.v = p.v + (int64_t)kvh * p.skh;
-  a.ks = p.ks + (int64_t)kvh * (SC == PA_SCALE_FP32 ? 4 : 2);
-  a.vs = p.vs + (int64_t)kvh * (SC == PA_SCALE_FP32 ? 4 : 2);
+  a.ks = p.ks + (int64_t)kvh * (SC == PA_SCALE_FP32 ? 4 : 2) * PK;
+  a.vs = p.vs + (int64_t)kvh * (SC == PA_SCALE_FP32 ? 4 : 2) * PK;
   a.k_lane = (uint32_t)((lane / G::kKLanesPerRow) & 15) * skt + 16u * (lane % G::kKLanesPerRow);
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -398,6 +414,14 @@ __device__ __forceinline__ TileAddr<KV, D> tile_addr(const KParams &p, int kvh, 
 #pragma unroll
   for (int g = 0; g < 4; ++g) a.s_mask[g] = (lane >> 4) == g ? ~0u : 0u;
   return a;
+}
+
+// The packed kv head (of PK = 2) that query column r16 belongs to: `group`
+// columns, the first half of them the first head's.
+template <int PK>
+__device__ __forceinline__ int packed_head(int r16, int group) {
+  static_assert(PK <= 2, "one comparison tells the heads apart");
+  return PK > 1 && 2 * r16 >= group ? 1 : 0;
 }
 
 template <int KV, int D>
@@ -421,8 +445,8 @@ struct WaveState {
 // once the loads issued before them (the tile about to be computed) have
 // arrived: one tile in flight per wave instead of two (the block-table
 // reads still go ahead).
-template <int KV, int SC, int D>
-__device__ __forceinline__ void load_tile(Tile<KV, D> &r, const KParams &p, const TileAddr<KV, D> &ta,
+template <int KV, int SC, int D, int PK>
+__device__ __forceinline__ void load_tile(Tile<KV, D, PK> &r, const KParams &p, const TileAddr<KV, D> &ta,
                                           const ro_i32 *bt_row, int n0, int hi, int lane,
                                           bool wait_prev = false) {
   using G = Geo<KV, D>;
@@ -482,18 +506,26 @@ __device__ __forceinline__ void load_tile(Tile<KV, D> &r, const KParams &p, cons
     // lane group g = lane / 16 holds scale (K | V)[g / 2] of sub-tile g % 2:
     // four loads, each with a uniform buffer, combined by bit masks (a
     // select between the loads would become one load from a per-lane buffer)
-    const uint32_t k0 = load_scale_bits<SC>(rks[0], ta.s_lane);
-    const uint32_t k1 = load_scale_bits<SC>(rks[1], ta.s_lane);
-    const uint32_t v0 = load_scale_bits<SC>(rvs[0], ta.s_lane);
-    const uint32_t v1 = load_scale_bits<SC>(rvs[1], ta.s_lane);
-    const uint32_t bits = (k0 & ta.s_mask[0]) | (k1 & ta.s_mask[1]) | (v0 & ta.s_mask[2]) | (v1 & ta.s_mask[3]);
-    r.sc[0] = SC == PA_SCALE_FP32 ? __builtin_bit_cast(float, bits)
-                                  : (float)__builtin_bit_cast(_Float16, (uint16_t)bits);
+    const u32x2 k0 = load_scale_bits<SC, PK>(rks[0], ta.s_lane);
+    const u32x2 k1 = load_scale_bits<SC, PK>(rks[1], ta.s_lane);
+    const u32x2 v0 = load_scale_bits<SC, PK>(rvs[0], ta.s_lane);
+    const u32x2 v1 = load_scale_bits<SC, PK>(rvs[1], ta.s_lane);
+    auto pick = [&](int w) {
+      return (k0[w] & ta.s_mask[0]) | (k1[w] & ta.s_mask[1]) | (v0[w] & ta.s_mask[2]) | (v1[w] & ta.s_mask[3]);
+    };
+    const uint32_t bits = pick(0);
+    if constexpr (SC == PA_SCALE_FP32) {
+      r.sc[0] = __builtin_bit_cast(float, bits);
+      if constexpr (PK == 2) r.sc[1] = __builtin_bit_cast(float, pick(1));
+    } else {
+      r.sc[0] = (float)__builtin_bit_cast(_Float16, (uint16_t)bits);
+      if constexpr (PK == 2) r.sc[1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(bits >> 16));
+    }
   }
 }
 
-template <int KV, int SC, int D>
-__device__ __forceinline__ void compute_tile(WaveState<KV, D> &st, const Tile<KV, D> &r,
+template <int KV, int SC, int D, int PK>
+__device__ __forceinline__ void compute_tile(WaveState<KV, D> &st, const Tile<KV, D, PK> &r,
                                              const KParams &p, int n0, int hi, int lane,
                                              float *sc_lds, uint8_t *k_lds) {
   using G = Geo<KV, D>;
@@ -521,7 +553,7 @@ __device__ __forceinline__ void compute_tile(WaveState<KV, D> &st, const Tile<KV
     // (entries 0 .. kTT-1 are K scales, the rest V scales; fp32 scales
     // stored times 2^24, fp16 scales as they are)
 #pragma unroll
-    for (int j = 0; j < G::kScales / 64; ++j)
+    for (int j = 0; j < PK; ++j)
       sc_lds[j * 64 + lane] = SC == PA_SCALE_FP32 ? r.sc[j] * kInt8Unit : r.sc[j];
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -532,20 +564,26 @@ __device__ __forceinline__ void compute_tile(WaveState<KV, D> &st, const Tile<KV
   f32x4 sacc[NS];
 #pragma unroll
   for (int u = 0; u < NS; ++u) {
-    f32x4 a = {0.f, 0.f, 0.f, 0.f};
+    f32x4 a[PK] = {};  // one sum per packed head: what one head's K holds (infinities) stays its own
     // int8: every element of this lane's operand is in row r16 of the
-    // sub-tile, so one scale serves them all (fp32 scales: ks8 = s * 2^24,
-    // kc8 = -128 * s; fp16 scales: the pair ks2 = (s, s))
-    float ks8 = 0.f, kc8 = 0.f;
-    uint32_t ks2 = 0;
+    // sub-tile, so one scale (of each packed head) serves them all (fp32
+    // scales: ks8 = s * 2^24, kc8 = -128 * s; fp16 scales: the pair ks2 = (s, s))
+    float ks8s[PK] = {}, kc8s[PK] = {};
+    uint32_t ks2s[PK] = {};
     if constexpr (KV == PA_KV_INT8) {
-      ks8 = sc_lds[16 * u + r16];
-      kc8 = ks8 * (-1.0f / 131072.0f);
-      if constexpr (SC == PA_SCALE_FP16) ks2 = cvt_pk_f16(ks8, ks8);
+#pragma unroll
+      for (int j = 0; j < PK; ++j) {
+        ks8s[j] = sc_lds[64 * j + 16 * u + r16];
+        kc8s[j] = ks8s[j] * (-1.0f / 131072.0f);
+        if constexpr (SC == PA_SCALE_FP16) ks2s[j] = cvt_pk_f16(ks8s[j], ks8s[j]);
+      }
     }
 #pragma unroll
     for (int ks = 0; ks < G::kKSteps; ++ks) {
       f16x8 kop;
+      const int kh = ks * PK / G::kKSteps;  // packed head of these 32 elements
+      [[maybe_unused]] const float ks8 = ks8s[kh], kc8 = kc8s[kh];
+      [[maybe_unused]] const uint32_t ks2 = ks2s[kh];
       const uint8_t *src = k_lds + (16 * u + r16) * G::kKSlotStride + (32 * ks + 8 * c) * G::kElem;
       if constexpr (KV == PA_KV_BF16) {
         kop = bf16x8_to_f16x8(*reinterpret_cast<const u32x4 *>(src));
@@ -575,9 +613,14 @@ __device__ __forceinline__ void compute_tile(WaveState<KV, D> &st, const Tile<KV
                        bytes_to_halves<KV>(w.y, w.y, pair_sel<KV>(0, 1)),
                        bytes_to_halves<KV>(w.y, w.y, pair_sel<KV>(2, 3)));
       }
-      a = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop, st.qop[ks], a, 0, 0, 0);
+      a[kh] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop, st.qop[ks], a[kh], 0, 0, 0);
     }
-    sacc[u] = a;
+    sacc[u] = a[0];
+    if constexpr (PK == 2) {
+      const bool second = packed_head<PK>(r16, p.group) != 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sacc[u][i] = second ? a[1][i] : a[0][i];
+    }
   }
   // the next tile's rows overwrite the slot only after these reads
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -647,7 +690,9 @@ __device__ __forceinline__ void compute_tile(WaveState<KV, D> &st, const Tile<KV
       if constexpr (KV == PA_KV_INT8) {
 #pragma unroll
         for (int h2 = 0; h2 < 2; ++h2) {
-          const f32x4 vq = *reinterpret_cast<const f32x4 *>(sc_lds + 16 * (NS + 2 * pp + h2) + 4 * c);
+          // (this lane's V elements lie in packed head r16 * PK / 16)
+          const f32x4 vq = *reinterpret_cast<const f32x4 *>(sc_lds + 64 * (r16 * PK / 16) +
+                                                            16 * (NS + 2 * pp + h2) + 4 * c);
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             vs[4 * h2 + i] = vq[i];
@@ -698,26 +743,29 @@ __device__ __forceinline__ void compute_tile(WaveState<KV, D> &st, const Tile<KV
 }
 
 // Q^T B-operands of query heads qh0 .. qh0 + nh - 1 of sequence b (lane
-// column r16 = head, padded columns are zero).
-template <int KV, int D>
+// column r16 = head, padded columns are zero). With PK packed kv heads a
+// column is zero outside its own kv head's D / PK elements of the row.
+template <int KV, int D, int PK>
 __device__ __forceinline__ void load_q(WaveState<KV, D> &st, const KParams &p, int b, int qh0,
                                        int nh, int r16, int c) {
   using G = Geo<KV, D>;
   const bool hv = r16 < nh;
+  const int sub = PK > 1 ? packed_head<PK>(r16, p.group) : 0;
   const uint16_t *qrow = reinterpret_cast<const uint16_t *>(p.q) + (int64_t)b * p.sqb +
                          (int64_t)(qh0 + (hv ? r16 : 0)) * p.sqh;
-  // 8 q values from head dim d0 on, as fp16 (bf16 rounded to fp16 first,
-  // the reference's q.to(fp16)); zeros for padded heads
-  auto q8 = [&](int d0) {
+  // 8 q values of k-step ks, as fp16 (bf16 rounded to fp16 first, the
+  // reference's q.to(fp16)); zeros for padded heads
+  auto q8 = [&](int ks) {
     f16x8 qv = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (hv) {
-      const u32x4 w = *reinterpret_cast<const u32x4 *>(qrow + d0);
+    const int kh = ks * PK / G::kKSteps;
+    if (hv && (PK == 1 || sub == kh)) {
+      const u32x4 w = *reinterpret_cast<const u32x4 *>(qrow + 32 * ks - kh * (D / PK) + 8 * c);
       qv = p.io_bf16 ? bf16x8_to_f16x8(w) : __builtin_bit_cast(f16x8, w);
     }
     return qv;
   };
 #pragma unroll
-  for (int ks = 0; ks < G::kKSteps; ++ks) st.qop[ks] = q8(32 * ks + 8 * c);
+  for (int ks = 0; ks < G::kKSteps; ++ks) st.qop[ks] = q8(ks);
 }
 
 template <int KV, int D>
@@ -729,15 +777,24 @@ __device__ __forceinline__ void reset_state(WaveState<KV, D> &st) {
   for (int sl = 0; sl < G::kE; ++sl) st.acc[sl] = f32x4{0.f, 0.f, 0.f, 0.f};
 }
 
+// Whether the lanes of group c (accumulator elements d0 = 4 * kE * c .. of the
+// row) hold elements of query column r16's own kv head. Packed heads share the
+// PV products, so the other head's elements of a column mean nothing.
+template <int PK>
+__device__ __forceinline__ bool own_elements(int r16, int c, int group) {
+  return PK == 1 || packed_head<PK>(r16, group) == c * PK / 4;
+}
+
 // One lane's share of a finished row of head h: y[0 .. 4*kE) = O[h][d0 ..)
 // (already normalised), L the row's sum of 2^(s - M). Written to `out` of
 // sequence b (direct) or as a partial row at element offsets part_off /
-// lse_off (the lse by the c == 0 lane).
-template <int D>
+// lse_off (the lse by the head's first lane).
+template <int D, int PK>
 __device__ __forceinline__ void store_result(const KParams &p, const float *y, float L, float M,
-                                             int b, int h, int d0, int c, bool direct,
+                                             int b, int h, int d0, bool direct,
                                              int64_t part_off, int64_t lse_off) {
   constexpr int kRegs = 4 * (D / 16);
+  d0 %= D / PK;  // element of the head
   if (!direct) {
     float *dst = p.part_out + part_off + (int64_t)h * p.sph + d0;
 #pragma unroll
@@ -745,7 +802,7 @@ __device__ __forceinline__ void store_result(const KParams &p, const float *y, f
       f32x4 t4 = {y[4 * v4], y[4 * v4 + 1], y[4 * v4 + 2], y[4 * v4 + 3]};
       *reinterpret_cast<f32x4 *>(dst + 4 * v4) = t4;
     }
-    if (c == 0) p.part_lse[lse_off + (int64_t)h * p.slh] = (L > 0.f) ? M + __log2f(L) : -INFINITY;
+    if (d0 == 0) p.part_lse[lse_off + (int64_t)h * p.slh] = (L > 0.f) ? M + __log2f(L) : -INFINITY;
   } else {
     uint8_t *dst = p.out + ((int64_t)b * p.sob + (int64_t)h * p.soh + d0) * 2;
     if (p.io_bf16) {
@@ -773,12 +830,12 @@ __device__ __forceinline__ void store_result(const KParams &p, const float *y, f
 // The same result written straight from the accumulators, a few registers at
 // a time: acc[sl][i] (sl = 0 .. kE-1) are the kE contiguous head-dim elements
 // from 4*kE*c + kE*i, scaled by `inv` on the way out.
-template <int D>
+template <int D, int PK>
 __device__ __forceinline__ void store_acc(const KParams &p, const f32x4 *acc, float inv, float L,
                                           float M, int b, int h, int c, bool direct,
                                           int64_t part_off, int64_t lse_off) {
   constexpr int kE = D / 16;
-  const int d0 = 4 * kE * c;
+  const int d0 = 4 * kE * c % (D / PK);  // element of the head
   if (!direct) {
     float *dst = p.part_out + part_off + (int64_t)h * p.sph + d0;
 #pragma unroll
@@ -795,7 +852,7 @@ __device__ __forceinline__ void store_acc(const KParams &p, const f32x4 *acc, fl
         for (int sl = 0; sl < kE; ++sl) dst[kE * i + sl] = acc[sl][i] * inv;
       }
     }
-    if (c == 0) p.part_lse[lse_off + (int64_t)h * p.slh] = (L > 0.f) ? M + __log2f(L) : -INFINITY;
+    if (d0 == 0) p.part_lse[lse_off + (int64_t)h * p.slh] = (L > 0.f) ? M + __log2f(L) : -INFINITY;
   } else {
     // kE (even) elements of group i = kE / 2 dwords at byte offset 2 * kE * i
     uint32_t *dst = reinterpret_cast<uint32_t *>(
@@ -869,7 +926,7 @@ enum { kUnsplit = 0, kPartials = 1, kAuto = 2 };
 
 // Two workgroups (8 waves) per CU must fit in the register file: the
 // double-buffered tiles are sized for that budget.
-template <int KV, int SC, int D, int MODE>
+template <int KV, int SC, int D, int MODE, int PK>
 __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
 paged_decode_kernel(const KParams p) {
   using G = Geo<KV, D>;
@@ -882,7 +939,7 @@ paged_decode_kernel(const KParams p) {
   __shared__ __attribute__((aligned(16))) uint8_t sm_raw[kMergeBytes > kSlotsBytes ? kMergeBytes : kSlotsBytes];
   __shared__ float sm_m[kWaves][16];
   __shared__ float sm_l[kWaves][16];
-  __shared__ __attribute__((aligned(16))) float sm_sc[kWaves][G::kScales];
+  __shared__ __attribute__((aligned(16))) float sm_sc[kWaves][G::kScales * PK];
   auto sm_acc = reinterpret_cast<float (*)[kRegs][64]>(sm_raw);
 
   const int lane = threadIdx.x & 63;
@@ -927,10 +984,10 @@ paged_decode_kernel(const KParams p) {
 
   WaveState<KV, D> st;
   reset_state(st);
-  load_q(st, p, b, qh0, nh, r16, c);
+  load_q<KV, D, PK>(st, p, b, qh0, nh, r16, c);
 
   const ro_i32 *bt_row = ro(p.bt) + (int64_t)b * p.sbtb;
-  const TileAddr<KV, D> addr = tile_addr<KV, SC, D>(p, kvh, lane);
+  const TileAddr<KV, D> addr = tile_addr<KV, SC, D, PK>(p, kvh, lane);
   float *sc_lds = sm_sc[wave];
   uint8_t *k_lds = sm_raw + wave * G::kKSlotBytes;
   const int ntiles = (hi > lo) ? (hi - lo + G::kTT - 1) / G::kTT : 0;
@@ -939,27 +996,27 @@ paged_decode_kernel(const KParams p) {
   auto n0_of = [&](int i) { return lo + (wave + kWaves * i) * G::kTT; };
   if (cnt > 0) {
     if constexpr (G::kPrefetch) {
-      Tile<KV, D> ta, tb;
-      load_tile<KV, SC, D>(ta, p, addr, bt_row, n0_of(0), hi, lane);
+      Tile<KV, D, PK> ta, tb;
+      load_tile<KV, SC, D, PK>(ta, p, addr, bt_row, n0_of(0), hi, lane);
       int i = 0;
       for (; i + 2 < cnt; i += 2) {
-        load_tile<KV, SC, D>(tb, p, addr, bt_row, n0_of(i + 1), hi, lane);
-        compute_tile<KV, SC, D>(st, ta, p, n0_of(i), hi, lane, sc_lds, k_lds);
-        load_tile<KV, SC, D>(ta, p, addr, bt_row, n0_of(i + 2), hi, lane);
-        compute_tile<KV, SC, D>(st, tb, p, n0_of(i + 1), hi, lane, sc_lds, k_lds);
+        load_tile<KV, SC, D, PK>(tb, p, addr, bt_row, n0_of(i + 1), hi, lane);
+        compute_tile<KV, SC, D, PK>(st, ta, p, n0_of(i), hi, lane, sc_lds, k_lds);
+        load_tile<KV, SC, D, PK>(ta, p, addr, bt_row, n0_of(i + 2), hi, lane);
+        compute_tile<KV, SC, D, PK>(st, tb, p, n0_of(i + 1), hi, lane, sc_lds, k_lds);
       }
       if (i + 1 < cnt) {
-        load_tile<KV, SC, D>(tb, p, addr, bt_row, n0_of(i + 1), hi, lane);
-        compute_tile<KV, SC, D>(st, ta, p, n0_of(i), hi, lane, sc_lds, k_lds);
-        compute_tile<KV, SC, D>(st, tb, p, n0_of(i + 1), hi, lane, sc_lds, k_lds);
+        load_tile<KV, SC, D, PK>(tb, p, addr, bt_row, n0_of(i + 1), hi, lane);
+        compute_tile<KV, SC, D, PK>(st, ta, p, n0_of(i), hi, lane, sc_lds, k_lds);
+        compute_tile<KV, SC, D, PK>(st, tb, p, n0_of(i + 1), hi, lane, sc_lds, k_lds);
       } else {
-        compute_tile<KV, SC, D>(st, ta, p, n0_of(i), hi, lane, sc_lds, k_lds);
+        compute_tile<KV, SC, D, PK>(st, ta, p, n0_of(i), hi, lane, sc_lds, k_lds);
       }
     } else {
       for (int i = 0; i < cnt; ++i) {
-        Tile<KV, D> t;
-        load_tile<KV, SC, D>(t, p, addr, bt_row, n0_of(i), hi, lane);
-        compute_tile<KV, SC, D>(st, t, p, n0_of(i), hi, lane, sc_lds, k_lds);
+        Tile<KV, D, PK> t;
+        load_tile<KV, SC, D, PK>(t, p, addr, bt_row, n0_of(i), hi, lane);
+        compute_tile<KV, SC, D, PK>(st, t, p, n0_of(i), hi, lane, sc_lds, k_lds);
       }
     }
   }
@@ -1003,9 +1060,10 @@ paged_decode_kernel(const KParams p) {
   const float inv = (L > 0.f) ? 1.0f / L : 0.f;
   float y[kRegs];
   regroup<D>(y, o, inv);
-  if (r16 >= nh) return;
-  store_result<D>(p, y, L, M, b, qh0 + r16, 4 * G::kE * c, c, direct,
-                  (int64_t)b * p.spb + (int64_t)split * p.sps, (int64_t)b * p.slb + split);
+  if (r16 >= nh || !own_elements<PK>(r16, c, p.group)) return;
+  const KParams &e = late_params();
+  store_result<D, PK>(e, y, L, M, b, qh0 + r16, 4 * G::kE * c, direct,
+                      (int64_t)b * e.spb + (int64_t)split * e.sps, (int64_t)b * e.slb + split);
 }
 
 // ----------------------------------------------------------------------------
@@ -1272,6 +1330,7 @@ __global__ void __launch_bounds__(flat_waves<KV>() * 64) __attribute__((amdgpu_w
 paged_decode_flat_kernel(const FlatArgs fa) {
   const KParams &p = fa.p;
   using G = Geo<KV, D>;
+  constexpr int PK = 1;
   static_assert(G::kTT == kSplitAlign, "flat tiles are the kernel's tiles");
   // the workgroup's W waves take W neighbouring kv heads of one range, so
   // together they read a contiguous W-head stretch of every token row (4
@@ -1349,11 +1408,11 @@ paged_decode_flat_kernel(const FlatArgs fa) {
 
   WaveState<KV, D> st;
   reset_state(st);
-  load_q(st, p, cc.b, qh0, nh, r16, c);
+  load_q<KV, D, PK>(st, p, cc.b, qh0, nh, r16, c);
 
   float *sc_lds = sm_sc[wave];
   uint8_t *k_lds = sm_k + wave * G::kKSlotBytes;
-  const TileAddr<KV, D> addr = tile_addr<KV, SC, D>(p, kvh, lane);
+  const TileAddr<KV, D> addr = tile_addr<KV, SC, D, PK>(p, kvh, lane);
 
   // block-table row of sequence b, in 32 bits (batch * stride_btb < 2^31 is
   // checked on the host): the 64-bit product cost 8 scalar instructions per
@@ -1377,14 +1436,14 @@ paged_decode_flat_kernel(const FlatArgs fa) {
       const float inv = (L > 0.f) ? 1.0f / L : 0.f;
       if (r16 < nh) {
         const int slot = cc.b + j;
-        store_acc<D>(p, st.acc, inv, L, st.m, cc.b, qh0 + r16, c, seg_t0 == 0 && seq_end,
+        store_acc<D, PK>(p, st.acc, inv, L, st.m, cc.b, qh0 + r16, c, seg_t0 == 0 && seq_end,
                      (int64_t)slot * p.spb, (int64_t)slot * p.slb);
       }
       if (i + 1 < n) {
         cursor_next(cc, ro(p.seq_lens), p.batch, p.max_tokens);
         seg_t0 = 0;
         reset_state(st);
-        load_q(st, p, cc.b, qh0, nh, r16, c);
+        load_q<KV, D, PK>(st, p, cc.b, qh0, nh, r16, c);
       }
     } else {
       ++cc.t;
@@ -1396,35 +1455,35 @@ paged_decode_flat_kernel(const FlatArgs fa) {
     // tiles of rows up to 64 bytes (4 KB) keep two in flight at any length:
     // one in flight per wave leaves too few bytes in flight for HBM
     const bool shallow = G::kRowBytes > 64 && n > kDeepTiles;
-    Tile<KV, D> ta, tb;
-    load_tile<KV, SC, D>(ta, p, addr, bt_of(lc.b), n0_of(lc), lc.len, lane);
+    Tile<KV, D, PK> ta, tb;
+    load_tile<KV, SC, D, PK>(ta, p, addr, bt_of(lc.b), n0_of(lc), lc.len, lane);
     int i = 0;
     for (; i + 2 < n; i += 2) {
       cursor_next(lc, ro(p.seq_lens), p.batch, p.max_tokens);
-      load_tile<KV, SC, D>(tb, p, addr, bt_of(lc.b), n0_of(lc), lc.len, lane, shallow);
-      compute_tile<KV, SC, D>(st, ta, p, n0_of(cc), cc.len, lane, sc_lds, k_lds);
+      load_tile<KV, SC, D, PK>(tb, p, addr, bt_of(lc.b), n0_of(lc), lc.len, lane, shallow);
+      compute_tile<KV, SC, D, PK>(st, ta, p, n0_of(cc), cc.len, lane, sc_lds, k_lds);
       post(i);
       cursor_next(lc, ro(p.seq_lens), p.batch, p.max_tokens);
-      load_tile<KV, SC, D>(ta, p, addr, bt_of(lc.b), n0_of(lc), lc.len, lane, shallow);
-      compute_tile<KV, SC, D>(st, tb, p, n0_of(cc), cc.len, lane, sc_lds, k_lds);
+      load_tile<KV, SC, D, PK>(ta, p, addr, bt_of(lc.b), n0_of(lc), lc.len, lane, shallow);
+      compute_tile<KV, SC, D, PK>(st, tb, p, n0_of(cc), cc.len, lane, sc_lds, k_lds);
       post(i + 1);
     }
     if (i + 1 < n) {
       cursor_next(lc, ro(p.seq_lens), p.batch, p.max_tokens);
-      load_tile<KV, SC, D>(tb, p, addr, bt_of(lc.b), n0_of(lc), lc.len, lane, shallow);
-      compute_tile<KV, SC, D>(st, ta, p, n0_of(cc), cc.len, lane, sc_lds, k_lds);
+      load_tile<KV, SC, D, PK>(tb, p, addr, bt_of(lc.b), n0_of(lc), lc.len, lane, shallow);
+      compute_tile<KV, SC, D, PK>(st, ta, p, n0_of(cc), cc.len, lane, sc_lds, k_lds);
       post(i);
-      compute_tile<KV, SC, D>(st, tb, p, n0_of(cc), cc.len, lane, sc_lds, k_lds);
+      compute_tile<KV, SC, D, PK>(st, tb, p, n0_of(cc), cc.len, lane, sc_lds, k_lds);
       post(i + 1);
     } else {
-      compute_tile<KV, SC, D>(st, ta, p, n0_of(cc), cc.len, lane, sc_lds, k_lds);
+      compute_tile<KV, SC, D, PK>(st, ta, p, n0_of(cc), cc.len, lane, sc_lds, k_lds);
       post(i);
     }
   } else {
     for (int i = 0; i < n; ++i) {
-      Tile<KV, D> t;
-      load_tile<KV, SC, D>(t, p, addr, bt_of(cc.b), n0_of(cc), cc.len, lane);
-      compute_tile<KV, SC, D>(st, t, p, n0_of(cc), cc.len, lane, sc_lds, k_lds);
+      Tile<KV, D, PK> t;
+      load_tile<KV, SC, D, PK>(t, p, addr, bt_of(cc.b), n0_of(cc), cc.len, lane);
+      compute_tile<KV, SC, D, PK>(st, t, p, n0_of(cc), cc.len, lane, sc_lds, k_lds);
       post(i);
     }
   }
@@ -1699,6 +1758,38 @@ int ilog2(int x) {
   return r;
 }
 
+// Whether the classic kernel takes two kv heads as one of twice the head dim
+// (KParams::pack): rows of 64 one-byte elements, heads next to each other in a
+// token, both groups within the 16 MFMA columns, and enough workgroups left
+// when each takes two heads. A row of 64 bytes is half a cache line and its
+// tile 4 KB, so the per-tile instructions (softmax, block table, waits) set the
+// pace, not HBM; two heads share them. The other type of row is bound by HBM
+// already: fp16 at this head dim 45.3 us packed, 44.8 not (B = 256, T = 2048).
+// Graph-timed at 14 q / 2 kv heads, one head / two per wave, whole calls in us:
+//   fp8, unsplit: B = 256, T = 2048 45.4 / 25.2; B = 256, T ~ U[32, 512] 10.4 / 7.9;
+//   int8, unsplit: B = 256, T = 2048 (fp32 scales) 48.8 / 32.9; B = 1024,
+//     T ~ U[32, 512] 31.7 / 24.3; B = 64, T = 4096, 4 splits 21.6 / 20.5;
+//   int8, B = 16, T = 32768: 16 splits (256 workgroups) 35.1 / 32.3, 8 splits
+//     (128) 46.3 / 51.6; fp8, B = 8, T = 65536: 32 splits 45.2 / 26.8, 16 (128)
+//     30.0 / 31.3; B = 192 unsplit (192 workgroups) 30.0 / 26.9.
+constexpr int kPackMinWorkgroups = 192;
+
+bool packs_heads(const pa_decode_args *a, const KParams &k) {
+  const bool one_byte = a->kv_dtype == PA_KV_FP8_E5M2 || a->kv_dtype == PA_KV_INT8;
+  if (a->flat_splits > 0 || !one_byte || a->head_dim != 64 || k.hkv % 2 != 0 || 2 * k.group > PA_MAX_GROUP)
+    return false;
+  // (the range check of a V row's buffer counts whole token strides, so the
+  // pair's row, and its scales, must lie inside one)
+  if (k.skh != 64 || k.skt < 128) return false;
+  if (a->kv_dtype == PA_KV_INT8) {
+    // a pair of scales is one load of 8 or 4 bytes
+    const int pair = a->scale_dtype == PA_SCALE_FP32 ? 8 : 4;
+    if (!aligned(a->k_scale, 4) || !aligned(a->v_scale, 4) || k.sst % 4 != 0 || k.ssn % 4 != 0 || k.sst < pair)
+      return false;
+  }
+  return (int64_t)a->batch * (k.hkv / 2) * a->num_splits >= kPackMinWorkgroups;
+}
+
 // Validates and fills the kernel parameter block. `need_partials` is true when
 // the decode kernel will write part_out / part_lse.
 int build_params(const pa_decode_args *a, bool need_partials, KParams *kp) {
@@ -1846,6 +1937,13 @@ int build_params(const pa_decode_args *a, bool need_partials, KParams *kp) {
   k.sbtb = a->stride_btb;
   k.qk_scale = a->sm_scale * kLog2e;
   k.io_bf16 = a->io_dtype == PA_IO_BF16;
+  k.pack = 1;
+  if (packs_heads(a, k)) {
+    k.pack = 2;
+    k.hkv /= 2;
+    k.group *= 2;
+    k.skh *= 2;
+  }
   return PA_OK;
 }
 
@@ -1863,10 +1961,10 @@ struct HostPlan {
   MergeTable mt;
 };
 
-template <int KV, int SC, int D>
+template <int KV, int SC, int D, int PK>
 hipError_t launch_decode_t(const KParams &k, int grid, int mode, hipStream_t st, const HostPlan *hp) {
   const dim3 g(grid), blk(kWaves * 64);
-  if (mode == kFlat) {
+  if constexpr (PK == 1) if (mode == kFlat) {
     constexpr int W = flat_waves<KV>();
     const int flat_grid = (k.hkv * k.head_tiles * k.flat_splits + W - 1) / W;
     if (hp != nullptr && hp->ranges) {
@@ -1877,12 +1975,14 @@ hipError_t launch_decode_t(const KParams &k, int grid, int mode, hipStream_t st,
       fa.ntab = 0;
       hipLaunchKernelGGL((paged_decode_flat_kernel<KV, SC, D>), dim3(flat_grid), dim3(W * 64), 0, st, fa);
     }
-  } else if (mode == kAuto) {
-    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kAuto>), g, blk, 0, st, k);
+    return hipGetLastError();
+  }
+  if (mode == kAuto) {
+    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kAuto, PK>), g, blk, 0, st, k);
   } else if (mode == kPartials) {
-    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kPartials>), g, blk, 0, st, k);
+    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kPartials, PK>), g, blk, 0, st, k);
   } else {
-    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kUnsplit>), g, blk, 0, st, k);
+    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kUnsplit, PK>), g, blk, 0, st, k);
   }
   return hipGetLastError();
 }
@@ -1890,17 +1990,20 @@ hipError_t launch_decode_t(const KParams &k, int grid, int mode, hipStream_t st,
 template <int KV, int SC>
 hipError_t launch_decode_d(const KParams &k, int d, int grid, int mode, hipStream_t st, const HostPlan *hp) {
   switch (d) {
-    case 32: return launch_decode_t<KV, SC, 32>(k, grid, mode, st, hp);
-    case 64: return launch_decode_t<KV, SC, 64>(k, grid, mode, st, hp);
-    case 128: return launch_decode_t<KV, SC, 128>(k, grid, mode, st, hp);
-    default: return launch_decode_t<KV, SC, 256>(k, grid, mode, st, hp);
+    case 32: return launch_decode_t<KV, SC, 32, 1>(k, grid, mode, st, hp);
+    case 64:
+      if constexpr (Geo<KV, 64>::kElem == 1)
+        if (k.pack == 2) return launch_decode_t<KV, SC, 128, 2>(k, grid, mode, st, hp);
+      return launch_decode_t<KV, SC, 64, 1>(k, grid, mode, st, hp);
+    case 128: return launch_decode_t<KV, SC, 128, 1>(k, grid, mode, st, hp);
+    default: return launch_decode_t<KV, SC, 256, 1>(k, grid, mode, st, hp);
   }
 }
 
 hipError_t launch_decode(const KParams &k, const pa_decode_args *a, int mode, hipStream_t st,
                          const HostPlan *hp = nullptr) {
   // the flat launch sizes its own grid from its workgroup width
-  const int grid = mode == kFlat ? 0 : a->batch * a->num_kv_heads * k.head_tiles * a->num_splits;
+  const int grid = mode == kFlat ? 0 : a->batch * k.hkv * k.head_tiles * a->num_splits;
   const int d = a->head_dim;
   if (a->kv_dtype == PA_KV_FP16) return launch_decode_d<PA_KV_FP16, PA_SCALE_NONE>(k, d, grid, mode, st, hp);
   if (a->kv_dtype == PA_KV_BF16) return launch_decode_d<PA_KV_BF16, PA_SCALE_NONE>(k, d, grid, mode, st, hp);

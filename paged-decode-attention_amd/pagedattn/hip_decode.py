@@ -115,6 +115,19 @@ UNSPLIT_MAX_KV_BYTES_PER_CU = {"fp16": 2 << 20, "bf16": 2 << 20, "fp8_e5m2": 768
 # T = 2048 45.0 / 48.5.
 UNSPLIT_MIN_ROW_BYTES = 128
 UNSPLIT_MAX_SHORT_ROW_BYTES_PER_CU = 192 << 10
+# The classic kernel takes two 64-element kv heads of a 1-byte cache as one row
+# of 128 (`packs_heads`), and then streams such rows faster than the flat split,
+# unsplit or cut into the splits that give every CU a workgroup (rounded up to a
+# power of two), unless one sequence is far longer than the others: up to
+# PACKED_SPLIT_MAX_RAGGED times the mean. Graph-timed at the Qwen2.5-0.5B shape
+# (256 CUs), flat (the better of F = 512 and 1024) / this rule in us: T ~ U[128,
+# 2047] B = 256 fp8 27.1 / 17.6, int8 33.2 / 27.2; T ~ U[200, 3000] B = 96 fp8
+# 22.0 / 16.3, int8 28.7 / 20.4 (4 splits); T ~ U[1000, 16000] B = 32 fp8 23.9 /
+# 18.8 (8 splits), int8 27.8 / 29.0; T = 4096 B = 256 fp8 56.4 / 45.6, int8 71.7
+# / 54.9; T ~ U[64, 1024] B = 1024 int8 69.4 / 37.8. With lengths log-uniform
+# over a factor of 64 (longest 4 times the mean) flat wins: B = 32 fp8 21.3 /
+# 27.4, B = 256 int8 31.8 / 44.1.
+PACKED_SPLIT_MAX_RAGGED = 2.25
 # Batches of short sequences that fill the CUs run unsplit, whatever their
 # size and merge or not: the flat split loses there, because its waves
 # switch sequences every few tiles. Per KV type, the longest sequence of a
@@ -223,6 +236,12 @@ def _nearly_uniform(lens) -> bool:
     return tmax > 0 and tmax <= 1.25 * int(lens.sum()) / lens.size
 
 
+def packs_heads(num_kv_heads: int, group: int, head_dim: int | None, kv_dtype: str | None) -> bool:
+    """Whether the classic kernel takes two kv heads of this geometry as one."""
+    return (head_dim == 64 and _KV_ELEM_BYTES.get(kv_dtype) == 1 and num_kv_heads % 2 == 0
+            and 2 * group <= _abi.PA_MAX_GROUP)
+
+
 def _fills_unsplit(lens, num_kv_heads: int, group: int, sm_count: int) -> bool:
     """A nearly uniform batch whose unsplit workgroups already give every CU one."""
     lens = _lens_array(lens)
@@ -312,6 +331,9 @@ class LaunchPlan:
     flat_splits == 0: the classic kernel with `num_splits` per-sequence
     splits (1 = unsplit), chunked from `max_seq_len`. `flat_seq_cost`: the
     tiles of weight the flat split charges each sequence (0 = equal tiles).
+    `packed_splits` > 0: launch the classic kernel with that many splits
+    instead, which takes pairs of heads and is faster; the other fields then
+    describe the launch without them.
     """
 
     num_splits: int
@@ -319,9 +341,12 @@ class LaunchPlan:
     flat_splits: int
     merge: bool = True
     flat_seq_cost: int = 0
+    packed_splits: int = 0
 
     def launch_kwargs(self) -> dict:
         """Keywords of `paged_decode_hip` that select this launch."""
+        if self.packed_splits:
+            return {"num_splits": self.packed_splits, "max_seq_len": self.max_seq_len}
         if self.flat_splits:
             return {"flat_splits": self.flat_splits, "flat_seq_cost": self.flat_seq_cost}
         return {"num_splits": self.num_splits, "max_seq_len": self.max_seq_len}
@@ -354,8 +379,40 @@ def plan_launch(batch: int, max_seq_len: int, num_kv_heads: int, group: int, sm_
         lengths or on `batch` sequences of `max_seq_len` tokens.
     A flat plan charges each sequence RAGGED_FLAT_SEQ_COST tiles
     (RAGGED_FLAT_SEQ_COST_KV for 1-byte KV) when the
-    lengths are known and not nearly uniform, else nothing.
+    lengths are known and not nearly uniform, else nothing. Where the classic
+    kernel would take pairs of heads, such a batch's plan also names the
+    splits to launch it with instead (`packed_splits_for`).
     """
+    plan = _plan_launch(batch, max_seq_len, num_kv_heads, group, sm_count, waves_per_simd, kv_dtype,
+                        head_dim, seq_lens)
+    packed = packed_splits_for(seq_lens, plan, num_kv_heads, group, sm_count, kv_dtype, head_dim)
+    return dataclasses.replace(plan, packed_splits=packed) if packed else plan
+
+
+def packed_splits_for(seq_lens, plan: LaunchPlan, num_kv_heads: int, group: int, sm_count: int,
+                      kv_dtype: str | None, head_dim: int | None) -> int:
+    """Splits of the classic kernel where it takes pairs of heads (`packs_heads`)
+    and beats `plan`: the fewest, as a power of two, that give every CU a
+    workgroup, chunks of at least MIN_SPLIT_TILES tiles. 0: `plan` stands (other
+    geometries, unknown lengths, short sequences, a batch with a sequence over
+    PACKED_SPLIT_MAX_RAGGED times the mean)."""
+    if seq_lens is None or not packs_heads(num_kv_heads, group, head_dim, kv_dtype):
+        return 0
+    lens = _lens_array(seq_lens)
+    batch, tmax = int(lens.size), plan.max_seq_len
+    if _tiles(tmax) <= UNSPLIT_MAX_TILES or tmax * batch > PACKED_SPLIT_MAX_RAGGED * int(lens.sum()):
+        return 0
+    pairs, splits = batch * (num_kv_heads // 2), 1
+    while splits * pairs < sm_count and _tiles(tmax) >= 2 * splits * MIN_SPLIT_TILES:
+        splits *= 2
+    if plan.flat_splits == 0 and splits > 2:
+        return 0  # a small batch of the classic split: more splits cost more than pairs save
+    return min(splits, _abi.PA_MAX_SPLITS)
+
+
+def _plan_launch(batch, max_seq_len, num_kv_heads, group, sm_count, waves_per_simd, kv_dtype, head_dim,
+                 seq_lens) -> LaunchPlan:
+    """`plan_launch` without packed heads."""
     cus = max(1, sm_count)
     known = seq_lens is not None
     lens = _lens_array(seq_lens) if known else None
@@ -836,6 +893,8 @@ def paged_decode_hip(
         plan = plan_launch(b, 0, shape.num_kv_heads, shape.gqa_group, _cu_count(q.device), wps,
                            kv_dtype=cache.kv_dtype, head_dim=d, seq_lens=lens)
         num_splits, flat_splits = plan.num_splits, plan.flat_splits
+        if plan.packed_splits:
+            num_splits, flat_splits = plan.packed_splits, 0
         if flat_seq_cost is None:
             flat_seq_cost = plan.flat_seq_cost
         if max_seq_len is None:

@@ -1,0 +1,114 @@
+"""The classic kernel on pairs of 64-element kv heads of a 1-byte cache (one wave takes both heads
+as a row of 128) against the oracle, and against the same heads taken one by one."""
+
+from __future__ import annotations
+
+import dataclasses
+
+import pytest
+import torch
+
+from helpers import max_abs, seeded_q
+from oracle import reference as oracle
+from pagedattn import ModelShape, allocate, decode_partials
+from pagedattn.hip_decode import paged_decode_hip
+
+pytestmark = pytest.mark.gpu
+
+KV = [("fp8_e5m2", None), ("int8", torch.float16), ("int8", torch.float32)]
+
+
+def _cache(hq, hkv, lens, kv_dtype, scale_dtype, page=16, seed=61):
+    kw = {} if scale_dtype is None else {"scale_dtype": scale_dtype}
+    return allocate(ModelShape(hq, hkv, 64, "p"), len(lens), lens, block_size=page, kv_dtype=kv_dtype, seed=seed,
+                    device="cuda", **kw)
+
+
+def _rows(c, sel):
+    return dataclasses.replace(c, block_table=c.block_table[sel].contiguous(), seq_lens=c.seq_lens[sel].contiguous())
+
+
+@pytest.mark.parametrize("kv_dtype,scale_dtype", KV)
+@pytest.mark.parametrize("hq,hkv,splits,page", [
+    (14, 2, 1, 16),   # 14 of 16 columns
+    (14, 2, 3, 32),
+    (16, 2, 2, 16),   # all 16 columns
+    (4, 4, 1, 64),    # two columns a pair, two pairs
+    (24, 4, 4, 16),
+])
+def test_pairs_match_the_oracle_and_single_heads(kv_dtype, scale_dtype, hq, hkv, splits, page):
+    batch = -(-192 // (hkv // 2 * splits))  # the smallest batch that packs
+    r = torch.Generator().manual_seed(62)
+    lens = torch.randint(1, 420, (batch,), generator=r).tolist()
+    lens[:5] = [1, 31, 32, 33, 0]
+    c = _cache(hq, hkv, lens, kv_dtype, scale_dtype, page)
+    q = seeded_q(batch, hq, 64, 63, device="cuda")
+    q[:, ::3] *= 3  # peaked heads next to flat ones
+    kw = {"num_splits": splits, "max_seq_len": max(lens)}
+    got = paged_decode_hip(q, c, **kw)
+    want = oracle.reference_decode(q, c, out_dtype=torch.float32)
+    assert bool((got[4] == 0).all())  # the empty sequence, for which the oracle has no value
+    want[4] = 0
+    assert max_abs(got, want) < 2e-3
+    # one sequence fewer: every head by itself
+    one = paged_decode_hip(q[1:].contiguous(), _rows(c, slice(1, None)), **kw)
+    assert max_abs(got[1:], one) < 2e-3
+    assert torch.equal(paged_decode_hip(q, c, **kw), got)
+    part, lse = decode_partials(q, c, splits, max_seq_len=max(lens))
+    part1, lse1 = decode_partials(q[1:].contiguous(), _rows(c, slice(1, None)), splits, max_seq_len=max(lens))
+    assert torch.equal(torch.isinf(lse[1:]), torch.isinf(lse1))
+    held = ~torch.isinf(lse1)
+    assert max_abs(lse[1:][held], lse1[held]) < 2e-3 and max_abs(part[1:], part1) < 2e-3
+
+
+@pytest.mark.parametrize("kv_dtype,scale_dtype", KV)
+def test_one_token_rows_are_the_dequantised_v_rows(kv_dtype, scale_dtype):
+    c = _cache(14, 2, [1] * 200, kv_dtype, scale_dtype)
+    out = paged_decode_hip(seeded_q(200, 14, 64, 64, device="cuda"), c, num_splits=1)
+    from pagedattn import dequantize_kv
+
+    first = c.block_table[:, 0].long()
+    # (index the raw bytes: fp8 tensors do not take every index kernel)
+    rows = c.v_cache.view(torch.uint8)[first, 0].view(c.v_cache.dtype)
+    v = dequantize_kv(rows, None if c.v_scale is None else c.v_scale[first, 0], kv_dtype)
+    assert torch.equal(out, v.repeat_interleave(7, dim=1))
+
+
+@pytest.mark.parametrize("what", ["k", "v"])
+def test_infinities_of_one_head_stay_in_it(what):
+    """An infinity in head 0's K or V (fp8 overflow) changes nothing of head 1's output."""
+    c = _cache(14, 2, [50] * 192, "fp8_e5m2", None)
+    q = seeded_q(192, 14, 64, 65, device="cuda")
+    clean = paged_decode_hip(q, c, num_splits=1)
+    store = (c.k_cache if what == "k" else c.v_cache).view(torch.uint8)
+    store[c.block_table[3, 1].long(), 2, 0, 5] = 0x7C  # +inf, head 0, sequence 3
+    got = paged_decode_hip(q, c, num_splits=1)
+    assert torch.equal(got[:, 7:], clean[:, 7:])
+    assert torch.equal(got[:3], clean[:3]) and torch.equal(got[4:], clean[4:])
+    assert not bool(torch.isfinite(got[3, :7]).all())
+
+
+@pytest.mark.parametrize("form", ["odd heads", "group 9", "head stride", "scale stride", "scale offset"])
+def test_forms_that_do_not_pair(form):
+    """Geometries outside the pairing rule give the oracle's result as before."""
+    lens = [5, 70, 33] * 70
+    if form == "odd heads":
+        c = _cache(6, 3, lens, "int8", torch.float16)
+    elif form == "group 9":
+        c = _cache(18, 2, lens, "int8", torch.float32)
+    else:
+        c = _cache(4, 2, lens, "int8", torch.float16)
+        if form == "head stride":  # heads 128 bytes apart
+            wide = [torch.zeros((*t.shape[:3], 128), dtype=t.dtype, device="cuda") for t in (c.k_cache, c.v_cache)]
+            for w, t in zip(wide, (c.k_cache, c.v_cache)):
+                w[..., :64] = t
+            c = dataclasses.replace(c, k_cache=wide[0][..., :64], v_cache=wide[1][..., :64])
+        else:  # three scales a token, or a first scale at an odd half word
+            wide = [torch.zeros((*t.shape[:2], 3), dtype=t.dtype, device="cuda") for t in (c.k_scale, c.v_scale)]
+            at = 0 if form == "scale stride" else 1
+            for w, t in zip(wide, (c.k_scale, c.v_scale)):
+                w[..., at:at + 2] = t
+            c = dataclasses.replace(c, k_scale=wide[0][..., at:at + 2], v_scale=wide[1][..., at:at + 2])
+    q = seeded_q(len(lens), c.shape.num_q_heads, 64, 66, device="cuda")
+    got = paged_decode_hip(q, c, num_splits=1)
+    assert max_abs(got, oracle.reference_decode(q, c, out_dtype=torch.float32)) < 2e-3
