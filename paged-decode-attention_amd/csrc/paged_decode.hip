@@ -107,6 +107,33 @@ constexpr int kDeepTiles = 16;
 // flat split's ranges, the merge's sequences); larger launches scan seq_lens
 // on the GPU instead.
 constexpr int kHostTab = PA_HOST_TABLE_MAX;
+constexpr uint32_t kMaxTiles = (1u << 26) - 1;  // 32-token tiles of the longest sequence (2^31 tokens)
+
+// Division of an n < 2^31 by a d that the host knows: floor(n / d) = n * mul >>
+// (32 + shift), mul = floor(2^(31 + l) / d) + 1, l = ceil(log2 d), shift = l -
+// 1 (Granlund and Montgomery's division by an invariant). A general 32-bit
+// division is ~25 dependent instructions in front of a kernel's first loads
+// and a 64-bit one ~150; with these the classic split's two kernels start
+// their loads 0.4 us earlier: whole calls at the Llama-3-8B shape, graph-timed,
+// B = 1, T = 2048 8.7 -> 8.3 us, B = 8, T <= 2500 17.0 -> 16.5, unsplit B = 24,
+// T <= 192 (Qwen2.5-0.5B shape) 4.66 -> 4.49.
+struct Div {
+  uint32_t d, mul, shift;
+};
+
+inline Div make_div(uint32_t d) {
+  Div v = {d, 0, 0};
+  if (d > 1) {
+    const uint32_t l = 32 - __builtin_clz(d - 1);
+    v.mul = (uint32_t)((uint64_t(1) << (31 + l)) / d + 1);
+    v.shift = l - 1;
+  }
+  return v;
+}
+
+__device__ __forceinline__ uint32_t div_by(uint32_t n, const Div &v) {
+  return v.d == 1 ? n : __umulhi(n, v.mul) >> v.shift;
+}
 
 struct KParams {
   const uint8_t *q;
@@ -142,17 +169,39 @@ struct KParams {
   int32_t pack;
 };
 
+// The classic split's division of a sequence: tiles of a split of max_seq_len
+// tokens (0: not given), and the divisors.
+struct SplitDiv {
+  int32_t max_seq_len, chunk_tiles;
+  Div by_splits, by_chunk;
+};
+
+// The classic kernel's arguments. (The flat kernel keeps the smaller ones: its
+// arguments are read cold on every eager launch.)
+struct ClassicArgs {
+  KParams p;
+  SplitDiv s;
+  Div by_head_tiles, by_hkv;
+};
+
 struct RParams {
   const float *part_out;
   const float *part_lse;
   uint8_t *out;
   int32_t io_bf16;  // out is bf16 (else fp16)
   const int32_t *seq_lens;  // AUTO and FLAT merges only
-  int32_t max_tokens, max_seq_len;  // AUTO and FLAT merges only
+  int32_t max_tokens;                       // AUTO and FLAT merges only
   int32_t num_heads, num_splits;    // FLAT: num_splits = flat splits
   int32_t batch;                    // FLAT only
   int32_t flat_cost;                // FLAT only: tiles charged per non-empty sequence
   int64_t spb, sph, sps, slb, slh, sob, soh;  // elements
+};
+
+// The merge of a classic split decode.
+struct AutoMergeArgs {
+  RParams r;
+  SplitDiv s;
+  Div by_heads;
 };
 
 // Reductions over the four lanes l, l^16, l^32, l^48 that hold one MFMA
@@ -445,10 +494,10 @@ struct WaveState {
 // once the loads issued before them (the tile about to be computed) have
 // arrived: one tile in flight per wave instead of two (the block-table
 // reads still go ahead).
-template <int KV, int SC, int D, int PK>
+template <int KV, int SC, int D, int PK, bool EARLY = false>
 __device__ __forceinline__ void load_tile(Tile<KV, D, PK> &r, const KParams &p, const TileAddr<KV, D> &ta,
                                           const ro_i32 *bt_row, int n0, int hi, int lane,
-                                          bool wait_prev = false) {
+                                          bool wait_prev = false, const int *early = nullptr) {
   using G = Geo<KV, D>;
   constexpr int NS = G::kNSub;
   static_assert(NS == 2 && G::kScales == 64, "one scale per lane covers the tile");
@@ -462,7 +511,10 @@ __device__ __forceinline__ void load_tile(Tile<KV, D, PK> &r, const KParams &p, 
 #pragma unroll
   for (int u = 0; u < NS; ++u) {
     const int t0 = min(n0 + 16 * u, (hi - 1) & ~15);
-    ph[u] = (uint32_t)min(max(bt_row[(uint32_t)t0 >> p.log2_page], 0), p.num_blocks - 1);
+    if constexpr (EARLY)  // the entries of n0 and n0 + 16, read ahead; a sub-tile past the end is n0's
+      ph[u] = (uint32_t)min(max(t0 > n0 ? early[1] : early[0], 0), p.num_blocks - 1);
+    else
+      ph[u] = (uint32_t)min(max(bt_row[(uint32_t)t0 >> p.log2_page], 0), p.num_blocks - 1);
     of[u] = (uint32_t)(t0 & page_mask);
     rows[u] = min(hi - t0, 16);  // valid rows of the sub-tile, >= 1
     const uint64_t row0 = (uint64_t)ph[u] * (uint32_t)p.skn + of[u] * skt;
@@ -897,20 +949,23 @@ struct SplitRange {
   int lo, hi, n;
 };
 
-__device__ __forceinline__ SplitRange split_range(int seq_len, int num_splits, int max_seq_len,
-                                                  int split) {
-  const int64_t own = ((int64_t)seq_len + kSplitAlign - 1) / kSplitAlign;
-  int64_t ntile_chunk = (own + num_splits - 1) / num_splits;
-  if (max_seq_len > 0) {
-    const int64_t longest = ((int64_t)max_seq_len + kSplitAlign - 1) / kSplitAlign;
-    ntile_chunk = max((longest + num_splits - 1) / num_splits, ntile_chunk);
+__device__ __forceinline__ SplitRange split_range(int seq_len, const SplitDiv &p, int split) {
+  static_assert(kSplitAlign == 32, "lengths are counted in 32-token tiles");
+  const uint32_t tiles = ((uint32_t)seq_len + 31) >> 5;  // < 2^27
+  uint32_t chunk = (uint32_t)p.chunk_tiles;
+  uint32_t n;
+  if (chunk != 0 && seq_len <= p.max_seq_len) {
+    n = div_by(tiles + chunk - 1, p.by_chunk);
+  } else {
+    // T = 0 still has one split
+    chunk = max(max(div_by(tiles + p.by_splits.d - 1, p.by_splits), chunk), 1u);
+    n = (tiles + chunk - 1) / chunk;
   }
-  const int64_t chunk = max(ntile_chunk, (int64_t)1) * kSplitAlign;  // T = 0 still has one split
-  const int64_t lo = min((int64_t)split * chunk, (int64_t)seq_len);
+  const uint32_t lo = min((uint32_t)split * chunk, tiles);
   SplitRange r;
-  r.lo = (int)lo;
-  r.hi = (int)min(lo + chunk, (int64_t)seq_len);
-  r.n = max(1, (int)((seq_len + chunk - 1) / chunk));
+  r.lo = (int)min(lo << 5, (uint32_t)seq_len);
+  r.hi = (int)min(min(lo + chunk, tiles) << 5, (uint32_t)seq_len);
+  r.n = max(1, (int)n);
   return r;
 }
 
@@ -928,7 +983,8 @@ enum { kUnsplit = 0, kPartials = 1, kAuto = 2 };
 // double-buffered tiles are sized for that budget.
 template <int KV, int SC, int D, int MODE, int PK>
 __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
-paged_decode_kernel(const KParams p) {
+paged_decode_kernel(const ClassicArgs ca) {
+  const KParams &p = ca.p;
   using G = Geo<KV, D>;
   constexpr int kRegs = 4 * G::kE;  // accumulator floats per lane
 
@@ -958,24 +1014,36 @@ paged_decode_kernel(const KParams p) {
     if (wg < full) wg = (wg % 8) * (full / 8) + wg / 8;
   }
   // wg = ((b * hkv + kvh) * head_tiles + ht) * num_splits + split
-  int x = wg;
-  const int split = x % p.num_splits;
-  x /= p.num_splits;
-  const int ht = x % p.head_tiles;
-  x /= p.head_tiles;
-  const int kvh = x % p.hkv;
-  const int b = x / p.hkv;
+  const int x1 = MODE == kUnsplit ? wg : div_by(wg, ca.s.by_splits);
+  const int split = MODE == kUnsplit ? 0 : wg - x1 * p.num_splits;
+  const int x2 = div_by(x1, ca.by_head_tiles);
+  const int ht = x1 - x2 * p.head_tiles;
+  const int b = div_by(x2, ca.by_hkv);
+  const int kvh = x2 - b * p.hkv;
 
   const int qh0 = kvh * p.group + ht * 16;
   const int nh = min(16, p.group - ht * 16);
 
-  int seq_len = p.seq_lens[b];
+  // The block-table entries of this wave's first tile are read together with
+  // the sequence's length, at the place where the tile will be unless the
+  // length is over max_seq_len (or that is not given; then they are read
+  // again): one round trip instead of two before the first K/V loads (0.08 us
+  // of the unsplit call at B = 24, T <= 192). The index is clamped to the row.
+  const ro_i32 *bt_row = ro(p.bt) + (int64_t)b * p.sbtb;
+  int guess_lo = 0;
+  if (MODE != kUnsplit) guess_lo = (int)min((uint32_t)split * (uint32_t)ca.s.chunk_tiles, kMaxTiles) << 5;
+  const uint32_t guess = (uint32_t)guess_lo + wave * G::kTT;
+  int early[2];
+#pragma unroll
+  for (int u = 0; u < 2; ++u)
+    early[u] = bt_row[min((guess + 16 * u) >> p.log2_page, (uint32_t)(p.max_blocks - 1))];
+  int seq_len = ro(p.seq_lens)[b];
   seq_len = max(0, min(seq_len, p.max_blocks << p.log2_page));
 
   int lo = 0, hi = seq_len;
   bool direct = true;  // write fp16 `out` (else a split partial)
   if (MODE != kUnsplit) {
-    const SplitRange r = split_range(seq_len, p.num_splits, p.max_seq_len, split);
+    const SplitRange r = split_range(seq_len, ca.s, split);
     if (MODE == kAuto && split >= r.n) return;  // an empty split: nothing to read or write
     lo = r.lo;
     hi = r.hi;
@@ -986,7 +1054,6 @@ paged_decode_kernel(const KParams p) {
   reset_state(st);
   load_q<KV, D, PK>(st, p, b, qh0, nh, r16, c);
 
-  const ro_i32 *bt_row = ro(p.bt) + (int64_t)b * p.sbtb;
   const TileAddr<KV, D> addr = tile_addr<KV, SC, D, PK>(p, kvh, lane);
   float *sc_lds = sm_sc[wave];
   uint8_t *k_lds = sm_raw + wave * G::kKSlotBytes;
@@ -995,9 +1062,14 @@ paged_decode_kernel(const KParams p) {
   const int cnt = ntiles > wave ? (ntiles - wave + kWaves - 1) / kWaves : 0;
   auto n0_of = [&](int i) { return lo + (wave + kWaves * i) * G::kTT; };
   if (cnt > 0) {
+    if (MODE != kUnsplit && lo != guess_lo) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        early[u] = bt_row[min((uint32_t)(n0_of(0) + 16 * u) >> p.log2_page, (uint32_t)(p.max_blocks - 1))];
+    }
     if constexpr (G::kPrefetch) {
       Tile<KV, D, PK> ta, tb;
-      load_tile<KV, SC, D, PK>(ta, p, addr, bt_row, n0_of(0), hi, lane);
+      load_tile<KV, SC, D, PK, true>(ta, p, addr, bt_row, n0_of(0), hi, lane, false, early);
       int i = 0;
       for (; i + 2 < cnt; i += 2) {
         load_tile<KV, SC, D, PK>(tb, p, addr, bt_row, n0_of(i + 1), hi, lane);
@@ -1437,7 +1509,7 @@ paged_decode_flat_kernel(const FlatArgs fa) {
       if (r16 < nh) {
         const int slot = cc.b + j;
         store_acc<D, PK>(p, st.acc, inv, L, st.m, cc.b, qh0 + r16, c, seg_t0 == 0 && seq_end,
-                     (int64_t)slot * p.spb, (int64_t)slot * p.slb);
+                         (int64_t)slot * p.spb, (int64_t)slot * p.slb);
       }
       if (i + 1 < n) {
         cursor_next(cc, ro(p.seq_lens), p.batch, p.max_tokens);
@@ -1627,8 +1699,13 @@ __device__ __forceinline__ void merge_into_out(const RParams &p, const float *ls
   write_merged<D>(p, acc, wsum, b, h, lane, active);
 }
 
-template <int D, int KIND>
-__global__ void __launch_bounds__(kMergeWaves * 64) split_reduce_kernel(const RParams p) {
+// ARGS: AutoMergeArgs for kMergeAuto, else RParams.
+template <int D, int KIND, typename ARGS>
+__global__ void __launch_bounds__(kMergeWaves * 64) split_reduce_kernel(const ARGS args) {
+  const RParams &p = [&]() -> const RParams & {
+    if constexpr (KIND == kMergeAuto) return args.r;
+    else return args;
+  }();
   __shared__ float sw_all[kMergeWaves][kReduceChunk];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -1643,16 +1720,18 @@ __global__ void __launch_bounds__(kMergeWaves * 64) split_reduce_kernel(const RP
   }
   const int bh = wg * kMergeWaves + wave;
   if (bh >= p.batch * p.num_heads) return;
-  const int b = bh / p.num_heads;
-  const int h = bh % p.num_heads;
+  int b;
+  if constexpr (KIND == kMergeAuto) b = div_by(bh, args.by_heads);
+  else b = bh / p.num_heads;
+  const int h = bh - b * p.num_heads;
   const float *lse = p.part_lse + (int64_t)b * p.slb + (int64_t)h * p.slh;
   const float *part = p.part_out + (int64_t)b * p.spb + (int64_t)h * p.sph;
   int64_t lse_step = 1;   // elements between consecutive partials
   int64_t part_step = p.sps;
   int S = p.num_splits;
-  if (KIND == kMergeAuto) {
-    const int seq_len = max(0, min(p.seq_lens[b], p.max_tokens));
-    S = split_range(seq_len, p.num_splits, p.max_seq_len, 0).n;
+  if constexpr (KIND == kMergeAuto) {
+    const int seq_len = max(0, min(ro(p.seq_lens)[b], p.max_tokens));
+    S = split_range(seq_len, args.s, 0).n;
     if (S <= 1) return;
   } else if (KIND == kMergeFlat) {
     // the decode's ranges: per = ceil(total / F) of weight each, where a
@@ -1756,6 +1835,16 @@ int ilog2(int x) {
   int r = 0;
   while ((1 << r) < x) ++r;
   return r;
+}
+
+SplitDiv split_div(int max_seq_len, int num_splits) {
+  const int64_t tiles = ((int64_t)max_seq_len + kSplitAlign - 1) / kSplitAlign;
+  SplitDiv s;
+  s.max_seq_len = max_seq_len;
+  s.chunk_tiles = (int)((tiles + num_splits - 1) / num_splits);
+  s.by_splits = make_div(num_splits);
+  s.by_chunk = make_div(std::max(1, s.chunk_tiles));
+  return s;
 }
 
 // Whether the classic kernel takes two kv heads as one of twice the head dim
@@ -1977,12 +2066,13 @@ hipError_t launch_decode_t(const KParams &k, int grid, int mode, hipStream_t st,
     }
     return hipGetLastError();
   }
+  const ClassicArgs ca = {k, split_div(k.max_seq_len, k.num_splits), make_div(k.head_tiles), make_div(k.hkv)};
   if (mode == kAuto) {
-    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kAuto, PK>), g, blk, 0, st, k);
+    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kAuto, PK>), g, blk, 0, st, ca);
   } else if (mode == kPartials) {
-    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kPartials, PK>), g, blk, 0, st, k);
+    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kPartials, PK>), g, blk, 0, st, ca);
   } else {
-    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kUnsplit, PK>), g, blk, 0, st, k);
+    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kUnsplit, PK>), g, blk, 0, st, ca);
   }
   return hipGetLastError();
 }
@@ -2035,7 +2125,6 @@ int check_reduce(const pa_reduce_args *r, RParams *rp) {
   rp->io_bf16 = r->io_dtype == PA_IO_BF16;
   rp->seq_lens = nullptr;
   rp->max_tokens = 0;
-  rp->max_seq_len = 0;
   rp->batch = r->batch;
   rp->flat_cost = 0;
   rp->num_heads = r->num_heads;
@@ -2050,15 +2139,15 @@ int check_reduce(const pa_reduce_args *r, RParams *rp) {
   return PA_OK;
 }
 
-template <int KIND>
-hipError_t launch_reduce(const RParams &rp, int batch, int d, hipStream_t st) {
-  const int grid = (batch * rp.num_heads + kMergeWaves - 1) / kMergeWaves;
+template <int KIND, typename ARGS>
+hipError_t launch_reduce(const ARGS &args, int batch, int num_heads, int d, hipStream_t st) {
+  const int grid = (batch * num_heads + kMergeWaves - 1) / kMergeWaves;
   const dim3 blk(kMergeWaves * 64);
   switch (d) {
-    case 32: hipLaunchKernelGGL((split_reduce_kernel<32, KIND>), dim3(grid), blk, 0, st, rp); break;
-    case 64: hipLaunchKernelGGL((split_reduce_kernel<64, KIND>), dim3(grid), blk, 0, st, rp); break;
-    case 128: hipLaunchKernelGGL((split_reduce_kernel<128, KIND>), dim3(grid), blk, 0, st, rp); break;
-    default: hipLaunchKernelGGL((split_reduce_kernel<256, KIND>), dim3(grid), blk, 0, st, rp); break;
+    case 32: hipLaunchKernelGGL((split_reduce_kernel<32, KIND, ARGS>), dim3(grid), blk, 0, st, args); break;
+    case 64: hipLaunchKernelGGL((split_reduce_kernel<64, KIND, ARGS>), dim3(grid), blk, 0, st, args); break;
+    case 128: hipLaunchKernelGGL((split_reduce_kernel<128, KIND, ARGS>), dim3(grid), blk, 0, st, args); break;
+    default: hipLaunchKernelGGL((split_reduce_kernel<256, KIND, ARGS>), dim3(grid), blk, 0, st, args); break;
   }
   return hipGetLastError();
 }
@@ -2314,7 +2403,6 @@ int pa_decode(const pa_decode_args *a, void *stream) {
     if (rc != PA_OK) return rc;
     rp.seq_lens = a->seq_lens;
     rp.max_tokens = k.max_tokens;
-    rp.max_seq_len = a->max_seq_len;
     if (flat) {
       rp.num_splits = a->flat_splits;
       rp.flat_cost = a->flat_seq_cost;
@@ -2331,8 +2419,9 @@ int pa_decode(const pa_decode_args *a, void *stream) {
       plan.mt.r = rp;
       e = launch_merge_table(plan.mt, a->head_dim, st);
     } else {
-      e = flat ? launch_reduce<kMergeFlat>(rp, a->batch, a->head_dim, st)
-               : launch_reduce<kMergeAuto>(rp, a->batch, a->head_dim, st);
+      const AutoMergeArgs ma = {rp, split_div(a->max_seq_len, a->num_splits), make_div(a->num_q_heads)};
+      e = flat ? launch_reduce<kMergeFlat>(rp, a->batch, a->num_q_heads, a->head_dim, st)
+               : launch_reduce<kMergeAuto>(ma, a->batch, a->num_q_heads, a->head_dim, st);
     }
     if (e != hipSuccess) return fail(PA_ERR_HIP, "reduce launch failed: %s", hipGetErrorString(e));
   }
@@ -2417,7 +2506,7 @@ int pa_flat_merge(const pa_decode_args *a, void *stream) {
     plan.mt.r = rp;
     e = launch_merge_table(plan.mt, a->head_dim, static_cast<hipStream_t>(stream));
   } else {
-    e = launch_reduce<kMergeFlat>(rp, a->batch, a->head_dim, static_cast<hipStream_t>(stream));
+    e = launch_reduce<kMergeFlat>(rp, a->batch, a->num_q_heads, a->head_dim, static_cast<hipStream_t>(stream));
   }
   if (e != hipSuccess) return fail(PA_ERR_HIP, "reduce launch failed: %s", hipGetErrorString(e));
   return ok();
@@ -2491,7 +2580,7 @@ int pa_split_reduce(const pa_reduce_args *r, void *stream) {
   int rc = check_reduce(r, &rp);
   if (rc != PA_OK) return rc;
   if (r->batch == 0) return ok();
-  hipError_t e = launch_reduce<kMergeAll>(rp, r->batch, r->head_dim, static_cast<hipStream_t>(stream));
+  hipError_t e = launch_reduce<kMergeAll>(rp, r->batch, r->num_heads, r->head_dim, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(PA_ERR_HIP, "reduce launch failed: %s", hipGetErrorString(e));
   return ok();
 }
