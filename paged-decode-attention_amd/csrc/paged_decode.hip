@@ -1699,17 +1699,96 @@ __device__ __forceinline__ void merge_into_out(const RParams &p, const float *ls
   write_merged<D>(p, acc, wsum, b, h, lane, active);
 }
 
-// ARGS: AutoMergeArgs for kMergeAuto, else RParams.
-template <int D, int KIND, typename ARGS>
-__global__ void __launch_bounds__(kMergeWaves * 64) split_reduce_kernel(const ARGS args) {
+// The same fold by a workgroup of kWideWaves waves, for rows cut into many
+// pieces (bound by round trips to the other XCDs' partials; the rule and both
+// sides' times are at wide_splits and wide_flat): wave w takes partials w, w + kWideWaves, ..., eight at a time with
+// their log2-sum-exps in the same round trip, and wave 0 folds the waves'
+// sums, in a fixed order.
+constexpr int kWideWaves = 4;
+constexpr int kWideHeld = 8;  // partials a wave holds at once
+
+template <int D>
+struct WideSums {
+  float m[kWideWaves], w[kWideWaves], acc[kWideWaves][D];
+};
+
+template <int D>
+__device__ __forceinline__ void merge_wide(const RParams &p, const float *lse, const float *part,
+                                           int64_t lse_step, int64_t part_step, int S, int b, int h,
+                                           int lane, int wave, WideSums<D> &sm) {
+  constexpr int kPer = D / 64 > 0 ? D / 64 : 1;
+  const bool active = lane * kPer < D;
+  float acc[kPer] = {}, wsum = 0.f, m = -INFINITY;
+  for (int s0 = wave; s0 < S; s0 += kWideWaves * kWideHeld) {
+    float ls[kWideHeld], v[kWideHeld][kPer];
+#pragma unroll
+    for (int i = 0; i < kWideHeld; ++i) {
+      const int s = s0 + kWideWaves * i;
+      ls[i] = -INFINITY;
+#pragma unroll
+      for (int j = 0; j < kPer; ++j) v[i][j] = 0.f;
+      if (s < S) {
+        ls[i] = lse[s * lse_step];
+        if (active) {
+#pragma unroll
+          for (int j = 0; j < kPer; ++j) v[i][j] = part[(int64_t)s * part_step + lane * kPer + j];
+        }
+      }
+    }
+    float mx = m;
+#pragma unroll
+    for (int i = 0; i < kWideHeld; ++i) mx = fmaxf(mx, ls[i]);
+    const float f = (m == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m - mx);
+    m = mx;
+    wsum *= f;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) acc[j] *= f;
+#pragma unroll
+    for (int i = 0; i < kWideHeld; ++i) {
+      const float w = (ls[i] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(ls[i] - m);
+      wsum += w;
+#pragma unroll
+      for (int j = 0; j < kPer; ++j) acc[j] += w * v[i][j];
+    }
+  }
+  if (lane == 0) {
+    sm.m[wave] = m;
+    sm.w[wave] = wsum;
+  }
+  if (active) {
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) sm.acc[wave][lane * kPer + j] = acc[j];
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  float M = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < kWideWaves; ++w) M = fmaxf(M, sm.m[w]);
+  wsum = 0.f;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) acc[j] = 0.f;
+#pragma unroll
+  for (int w = 0; w < kWideWaves; ++w) {
+    const float f = (sm.m[w] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(sm.m[w] - M);
+    wsum += f * sm.w[w];
+    if (active) {
+#pragma unroll
+      for (int j = 0; j < kPer; ++j) acc[j] += f * sm.acc[w][lane * kPer + j];
+    }
+  }
+  write_merged<D>(p, acc, active ? wsum : 0.f, b, h, lane, active);
+}
+
+// ARGS: AutoMergeArgs for kMergeAuto, else RParams. WIDE: one (b, h) per
+// workgroup of kWideWaves waves (merge_wide), else per wave.
+template <int D, int KIND, typename ARGS, bool WIDE>
+__global__ void __launch_bounds__((WIDE ? kWideWaves : kMergeWaves) * 64) split_reduce_kernel(const ARGS args) {
   const RParams &p = [&]() -> const RParams & {
     if constexpr (KIND == kMergeAuto) return args.r;
     else return args;
   }();
-  __shared__ float sw_all[kMergeWaves][kReduceChunk];
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  float *sw = sw_all[wave];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // XCD-contiguous order, as the split decode launches use: an XCD merges
   // a contiguous stretch of (sequence, head) pairs, whose partials that
   // XCD's ranges wrote (0.3-1.3 us per call at C2, C3 and C5)
@@ -1718,7 +1797,7 @@ __global__ void __launch_bounds__(kMergeWaves * 64) split_reduce_kernel(const AR
     const int n = gridDim.x, full = n - n % 8;
     if (wg < full) wg = (wg % 8) * (full / 8) + wg / 8;
   }
-  const int bh = wg * kMergeWaves + wave;
+  const int bh = WIDE ? wg : wg * kMergeWaves + wave;
   if (bh >= p.batch * p.num_heads) return;
   int b;
   if constexpr (KIND == kMergeAuto) b = div_by(bh, args.by_heads);
@@ -1771,7 +1850,13 @@ __global__ void __launch_bounds__(kMergeWaves * 64) split_reduce_kernel(const AR
     }
   }
 
-  merge_into_out<D>(p, lse, part, lse_step, part_step, S, b, h, lane, sw);
+  if constexpr (WIDE) {
+    __shared__ WideSums<D> sm;
+    merge_wide<D>(p, lse, part, lse_step, part_step, S, b, h, lane, wave, sm);
+  } else {
+    __shared__ float sw_all[kMergeWaves][kReduceChunk];
+    merge_into_out<D>(p, lse, part, lse_step, part_step, S, b, h, lane, sw_all[wave]);
+  }
 }
 
 // The flat split's merge when the host knows the lengths: a table of the
@@ -1793,22 +1878,27 @@ struct MergeTable {
 };
 static_assert(sizeof(MergeTable) <= 4096 && sizeof(FlatArgs) <= 4096, "kernel arguments over 4 KB");
 
-template <int D>
-__global__ void __launch_bounds__(kMergeWaves * 64) flat_merge_table_kernel(const MergeTable a) {
+template <int D, bool WIDE>
+__global__ void __launch_bounds__((WIDE ? kWideWaves : kMergeWaves) * 64) flat_merge_table_kernel(const MergeTable a) {
   const RParams &p = a.r;
-  __shared__ float sw_all[kMergeWaves][kReduceChunk];
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // workgroup h runs on XCD h % 8 (the hardware deals them round-robin)
-  const int x = blockIdx.x % 8, k = (blockIdx.x / 8) * kMergeWaves + wave;
+  const int x = blockIdx.x % 8, k = WIDE ? blockIdx.x / 8 : (blockIdx.x / 8) * kMergeWaves + wave;
   const int it = a.xstart[x] + k / p.num_heads;
   if (it >= a.xstart[x + 1]) return;
   const int h = k % p.num_heads;
   const int b = (int)a.seq[it], S = (int)a.nslot[it];
   const int64_t slot0 = a.slot[it];
-  merge_into_out<D>(p, p.part_lse + slot0 * p.slb + (int64_t)h * p.slh,
-                    p.part_out + slot0 * p.spb + (int64_t)h * p.sph, p.slb, p.spb, S, b, h, lane,
-                    sw_all[wave]);
+  const float *lse = p.part_lse + slot0 * p.slb + (int64_t)h * p.slh;
+  const float *part = p.part_out + slot0 * p.spb + (int64_t)h * p.sph;
+  if constexpr (WIDE) {
+    __shared__ WideSums<D> sm;
+    merge_wide<D>(p, lse, part, p.slb, p.spb, S, b, h, lane, wave, sm);
+  } else {
+    __shared__ float sw_all[kMergeWaves][kReduceChunk];
+    merge_into_out<D>(p, lse, part, p.slb, p.spb, S, b, h, lane, sw_all[wave]);
+  }
 }
 
 // ----------------------------------------------------------------------------
@@ -2139,32 +2229,55 @@ int check_reduce(const pa_reduce_args *r, RParams *rp) {
   return PA_OK;
 }
 
-template <int KIND, typename ARGS>
-hipError_t launch_reduce(const ARGS &args, int batch, int num_heads, int d, hipStream_t st) {
-  const int grid = (batch * num_heads + kMergeWaves - 1) / kMergeWaves;
-  const dim3 blk(kMergeWaves * 64);
+template <int KIND, typename ARGS, bool WIDE>
+hipError_t launch_reduce_w(const ARGS &args, int batch, int num_heads, int d, hipStream_t st) {
+  const int per = WIDE ? 1 : kMergeWaves;
+  const dim3 grid((batch * num_heads + per - 1) / per), blk((WIDE ? kWideWaves : kMergeWaves) * 64);
   switch (d) {
-    case 32: hipLaunchKernelGGL((split_reduce_kernel<32, KIND, ARGS>), dim3(grid), blk, 0, st, args); break;
-    case 64: hipLaunchKernelGGL((split_reduce_kernel<64, KIND, ARGS>), dim3(grid), blk, 0, st, args); break;
-    case 128: hipLaunchKernelGGL((split_reduce_kernel<128, KIND, ARGS>), dim3(grid), blk, 0, st, args); break;
-    default: hipLaunchKernelGGL((split_reduce_kernel<256, KIND, ARGS>), dim3(grid), blk, 0, st, args); break;
+    case 32: hipLaunchKernelGGL((split_reduce_kernel<32, KIND, ARGS, WIDE>), grid, blk, 0, st, args); break;
+    case 64: hipLaunchKernelGGL((split_reduce_kernel<64, KIND, ARGS, WIDE>), grid, blk, 0, st, args); break;
+    case 128: hipLaunchKernelGGL((split_reduce_kernel<128, KIND, ARGS, WIDE>), grid, blk, 0, st, args); break;
+    default: hipLaunchKernelGGL((split_reduce_kernel<256, KIND, ARGS, WIDE>), grid, blk, 0, st, args); break;
   }
   return hipGetLastError();
 }
 
-hipError_t launch_merge_table(const MergeTable &mt, int d, hipStream_t st) {
+template <int KIND, typename ARGS>
+hipError_t launch_reduce(const ARGS &args, int batch, int num_heads, int d, bool wide, hipStream_t st) {
+  return wide ? launch_reduce_w<KIND, ARGS, true>(args, batch, num_heads, d, st)
+                            : launch_reduce_w<KIND, ARGS, false>(args, batch, num_heads, d, st);
+}
+
+template <bool WIDE>
+hipError_t launch_merge_table_w(const MergeTable &mt, int d, hipStream_t st) {
   int most = 0;
   for (int x = 0; x < 8; ++x) most = std::max(most, mt.xstart[x + 1] - mt.xstart[x]);
-  const int grid = 8 * ((most * mt.r.num_heads + kMergeWaves - 1) / kMergeWaves);
-  const dim3 blk(kMergeWaves * 64);
+  const int per = WIDE ? 1 : kMergeWaves;
+  const dim3 grid(8 * ((most * mt.r.num_heads + per - 1) / per)), blk((WIDE ? kWideWaves : kMergeWaves) * 64);
   switch (d) {
-    case 32: hipLaunchKernelGGL((flat_merge_table_kernel<32>), dim3(grid), blk, 0, st, mt); break;
-    case 64: hipLaunchKernelGGL((flat_merge_table_kernel<64>), dim3(grid), blk, 0, st, mt); break;
-    case 128: hipLaunchKernelGGL((flat_merge_table_kernel<128>), dim3(grid), blk, 0, st, mt); break;
-    default: hipLaunchKernelGGL((flat_merge_table_kernel<256>), dim3(grid), blk, 0, st, mt); break;
+    case 32: hipLaunchKernelGGL((flat_merge_table_kernel<32, WIDE>), grid, blk, 0, st, mt); break;
+    case 64: hipLaunchKernelGGL((flat_merge_table_kernel<64, WIDE>), grid, blk, 0, st, mt); break;
+    case 128: hipLaunchKernelGGL((flat_merge_table_kernel<128, WIDE>), grid, blk, 0, st, mt); break;
+    default: hipLaunchKernelGGL((flat_merge_table_kernel<256, WIDE>), grid, blk, 0, st, mt); break;
   }
   return hipGetLastError();
 }
+
+hipError_t launch_merge_table(const MergeTable &mt, int d, bool wide, hipStream_t st) {
+  return wide ? launch_merge_table_w<true>(mt, d, st) : launch_merge_table_w<false>(mt, d, st);
+}
+
+// Whether a merge takes a workgroup of kWideWaves waves per row instead of one
+// wave: one wave holds 8 partials and folds more in a second and third round
+// trip, and the waves' fold costs 0.3 us where one would do. Whole calls,
+// graph-timed at the Llama-3-8B shape, one wave / kWideWaves, in us: classic
+// split B = 4, T = 1024 with 8 splits 8.9 / 9.3, B = 1, T = 2048 with 32 8.2 /
+// 7.9; flat F = 128, B = 64 (fp8, T <= 8192) 40.9 / 41.9, B = 32 (T <= 4095)
+// 46.7 / 45.8, B = 16 30.9 / 28.8, B = 8 (T <= 2500) 22.1 / 18.3. For the flat
+// split the rule knows only the ranges and the batch, the same with and without
+// host lengths, so that both merges fold alike.
+bool wide_splits(int num_splits) { return num_splits > 8; }
+bool wide_flat(const pa_decode_args *a) { return a->flat_splits >= 4 * (int64_t)a->batch; }
 
 // The flat split's ranges and merge list from host-side lengths, exactly as
 // the kernels derive them from seq_lens (flat_locate*, kMergeFlat): lengths
@@ -2417,11 +2530,11 @@ int pa_decode(const pa_decode_args *a, void *stream) {
   if (split && !(flat && !plan.needs_merge)) {
     if (flat && plan.merge_table) {
       plan.mt.r = rp;
-      e = launch_merge_table(plan.mt, a->head_dim, st);
+      e = launch_merge_table(plan.mt, a->head_dim, wide_flat(a), st);
     } else {
       const AutoMergeArgs ma = {rp, split_div(a->max_seq_len, a->num_splits), make_div(a->num_q_heads)};
-      e = flat ? launch_reduce<kMergeFlat>(rp, a->batch, a->num_q_heads, a->head_dim, st)
-               : launch_reduce<kMergeAuto>(ma, a->batch, a->num_q_heads, a->head_dim, st);
+      e = flat ? launch_reduce<kMergeFlat>(rp, a->batch, a->num_q_heads, a->head_dim, wide_flat(a), st)
+               : launch_reduce<kMergeAuto>(ma, a->batch, a->num_q_heads, a->head_dim, wide_splits(a->num_splits), st);
     }
     if (e != hipSuccess) return fail(PA_ERR_HIP, "reduce launch failed: %s", hipGetErrorString(e));
   }
@@ -2504,9 +2617,10 @@ int pa_flat_merge(const pa_decode_args *a, void *stream) {
   hipError_t e;
   if (plan.merge_table) {
     plan.mt.r = rp;
-    e = launch_merge_table(plan.mt, a->head_dim, static_cast<hipStream_t>(stream));
+    e = launch_merge_table(plan.mt, a->head_dim, wide_flat(a), static_cast<hipStream_t>(stream));
   } else {
-    e = launch_reduce<kMergeFlat>(rp, a->batch, a->num_q_heads, a->head_dim, static_cast<hipStream_t>(stream));
+    e = launch_reduce<kMergeFlat>(rp, a->batch, a->num_q_heads, a->head_dim, wide_flat(a),
+                                  static_cast<hipStream_t>(stream));
   }
   if (e != hipSuccess) return fail(PA_ERR_HIP, "reduce launch failed: %s", hipGetErrorString(e));
   return ok();
@@ -2580,7 +2694,8 @@ int pa_split_reduce(const pa_reduce_args *r, void *stream) {
   int rc = check_reduce(r, &rp);
   if (rc != PA_OK) return rc;
   if (r->batch == 0) return ok();
-  hipError_t e = launch_reduce<kMergeAll>(rp, r->batch, r->num_heads, r->head_dim, static_cast<hipStream_t>(stream));
+  hipError_t e = launch_reduce<kMergeAll>(rp, r->batch, r->num_heads, r->head_dim, wide_splits(r->num_splits),
+                                         static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(PA_ERR_HIP, "reduce launch failed: %s", hipGetErrorString(e));
   return ok();
 }

@@ -1,0 +1,51 @@
+"""The merge by four waves a row (more than 8 splits; a flat split with 4 ranges a sequence or more)
+at the edges of its passes and of its rule."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from helpers import max_abs, seeded_q
+from oracle import reference as oracle
+from pagedattn import LLAMA3_8B, allocate, split_reduce
+from pagedattn.hip_decode import paged_decode_hip
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("d", [32, 64, 128, 256])
+@pytest.mark.parametrize("splits", [8, 9, 31, 32, 33, 64, 65, 300])
+def test_split_reduce_edges(splits, d):
+    """8 a wave, 32 a pass; rows with some splits empty, one left, and none left (zeros)."""
+    g = torch.Generator().manual_seed(71)
+    part = torch.randn((2, 3, splits, d), generator=g)
+    lse = 20 * torch.randn((2, 3, splits), generator=g)
+    lse[0, 1, ::3] = float("-inf")
+    lse[1, 0, :] = float("-inf")
+    lse[1, 0, splits - 1] = -3.0
+    lse[1, 2, :] = float("-inf")
+    part[torch.isinf(lse)] = 0
+    got = split_reduce(part.cuda(), lse.cuda())
+    want = oracle.split_merge(part, lse)
+    want[1, 2] = 0
+    # fp32 sums of at most 300 terms, then fp16: half an ulp of a value up to 8 is 2^-9
+    assert max_abs(got, want) < 2.0 ** -9 + 1e-5
+
+
+@pytest.mark.parametrize("batch,flat", [(8, 31), (8, 32), (8, 33), (3, 40), (1, 200)])
+@pytest.mark.parametrize("kv_dtype", ["fp16", "int8"])
+def test_flat_rule_edges(batch, flat, kv_dtype):
+    """Either side of four ranges a sequence, host tables and the GPU scan alike, empty rows zero."""
+    lens = [(977 * i) % 3000 + 40 for i in range(batch)]
+    if batch > 2:
+        lens[1] = 0
+    c = allocate(LLAMA3_8B, batch, lens, kv_dtype=kv_dtype, seed=72, device="cuda")
+    q = seeded_q(batch, 32, 128, 73, device="cuda")
+    a = paged_decode_hip(q, c, flat_splits=flat, seq_lens_host=torch.tensor(lens, dtype=torch.int32))
+    b = paged_decode_hip(q, c, flat_splits=flat)
+    assert torch.equal(a, b)
+    want = oracle.reference_decode(q, c, out_dtype=torch.float32)
+    if batch > 2:
+        want[1] = 0
+    assert max_abs(a, want) < 2e-3
