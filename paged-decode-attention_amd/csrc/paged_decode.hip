@@ -2272,12 +2272,18 @@ hipError_t launch_merge_table(const MergeTable &mt, int d, bool wide, hipStream_
 // trip, and the waves' fold costs 0.3 us where one would do. Whole calls,
 // graph-timed at the Llama-3-8B shape, one wave / kWideWaves, in us: classic
 // split B = 4, T = 1024 with 8 splits 8.9 / 9.3, B = 1, T = 2048 with 32 8.2 /
-// 7.9; flat F = 128, B = 64 (fp8, T <= 8192) 40.9 / 41.9, B = 32 (T <= 4095)
-// 46.7 / 45.8, B = 16 30.9 / 28.8, B = 8 (T <= 2500) 22.1 / 18.3. For the flat
+// 7.9; flat F = 128, B = 64 (fp8, T <= 8192) 40.9 / 41.9, B = 32 T <= 4095
+// 46.7 / 45.8 but T <= 1622 24.3 / 25.6, B = 16 30.9 / 28.8, B = 8 (T <= 2500)
+// 22.1 / 18.3. For the flat
 // split the rule knows only the ranges and the batch, the same with and without
 // host lengths, so that both merges fold alike.
+// Above kWideMaxRows rows the launch of four times the waves costs more: int8, B =
+// 32, T = 16384, 64 heads, F = 256 177.3 / 179.1.
+constexpr int kWideMaxRows = 1024;
 bool wide_splits(int num_splits) { return num_splits > 8; }
-bool wide_flat(const pa_decode_args *a) { return a->flat_splits >= 4 * (int64_t)a->batch; }
+bool wide_flat(const pa_decode_args *a) {
+  return a->flat_splits >= 8 * (int64_t)a->batch && (int64_t)a->batch * a->num_q_heads <= kWideMaxRows;
+}
 
 // The flat split's ranges and merge list from host-side lengths, exactly as
 // the kernels derive them from seq_lens (flat_locate*, kMergeFlat): lengths

@@ -88,6 +88,36 @@ MIN_FLAT_TILES_PER_WAVE = 4
 # unbalance them.
 RAGGED_FLAT_SEQ_COST = 1
 RAGGED_FLAT_SEQ_COST_KV = {"fp8_e5m2": 2, "int8": 2}
+# A batch that gives the classic kernel at most one workgroup per CU unsplit is
+# cut into as many splits as keep it at one per CU (`few_splits`). It then runs
+# the classic kernel instead of the flat split while its longest chunk, in
+# tiles, is short enough: it skips the flat kernel's scan and wave-by-wave
+# segments (3 us for 2-byte KV, more for int8's two waves per SIMD), but streams
+# about CLASSIC_STREAM_LOSS slower and waits for its longest chunk. Lengths
+# known and ragged: chunk x (1 + CLASSIC_STREAM_LOSS) at most
+# CLASSIC_MARGIN_TILES over the batch's tiles per CU (UNSPLIT_MARGIN_TILES when
+# unsplit, with no merge either). Nearly uniform or unknown lengths: chunk at most
+# CLASSIC_MAX_CHUNK_TILES (UNSPLIT_MAX_CHUNK_TILES). Graph-timed whole calls, classic (its splits) / flat in
+# us, 256 CUs: Llama-3-8B shape fp16 B = 2, T = 16384 27.6 (16) / 28.1; B = 4, T
+# ~ U[512, 8192] 24.2 (8) / 25.2; B = 8, T ~ U[1000, 12000] 47.6 (4) / 36.6; B =
+# 16, T = 1024 17.0 (2) / 17.5, T ~ U[100, 2000] 20.9 (2) / 19.7, T ~ U[300, 6000]
+# 45.4 (2) / 34.8; B = 32, T ~ U[60, 1000] 18.9 (1) / 20.7, T ~ U[200, 3000] 44.5
+# (1) / 38.1; fp8 B = 2, T = 16384 18.4 (16) / 19.4; B = 4 16.8 (8) / 17.9; B = 16,
+# T ~ U[100, 2000] 15.3 (2) / 14.2; B = 32, T ~ U[60, 1000] 13.1 (1) / 14.8;
+# Llama-3-70B shape int8 B = 2, T = 16384 22.0 (16) / 26.6; B = 4, T ~ U[512, 8192]
+# 20.1 (8) / 26.1; B = 16, T ~ U[100, 2000] 19.1 (2) / 24.1, T ~ U[300, 6000] 39.9
+# (2) / 30.9; B = 32, T ~ U[60, 1000] 17.2 (1) / 26.2.
+CLASSIC_STREAM_LOSS = 0.08
+CLASSIC_MARGIN_TILES = {"fp16": 8, "bf16": 8, "fp8_e5m2": 10, "int8": 17}
+UNSPLIT_MARGIN_TILES = {"fp16": 14, "bf16": 14, "fp8_e5m2": 16, "int8": 17}
+CLASSIC_MAX_CHUNK_TILES = {"fp16": 24, "bf16": 24, "fp8_e5m2": 32, "int8": 40}
+UNSPLIT_MAX_CHUNK_TILES = {"fp16": 32, "bf16": 32, "fp8_e5m2": 32, "int8": 40}
+# few_splits: no more than this many while each holds less than
+# FEW_SPLIT_LONG_TILES (14 q / 2 kv heads, D = 64, fp16: B = 2, T = 4096 32 splits
+# 7.8, 64 8.8; T = 16384 10.0, 10.5; B = 1, T = 32768 64 splits 11.7, 32 12.6, 128
+# 13.0).
+FEW_SPLITS_MAX = 32
+FEW_SPLIT_LONG_TILES = 16
 # A single sequence up to this many tiles takes the classic split: cut into
 # one chunk per CU it merges 32 partials per head, the flat split 128 (graph-
 # timed whole calls, classic against flat: T = 16384 17.9 / 21.0 us, 32768
@@ -128,6 +158,10 @@ UNSPLIT_MAX_SHORT_ROW_BYTES_PER_CU = 192 << 10
 # over a factor of 64 (longest 4 times the mean) flat wins: B = 32 fp8 21.3 /
 # 27.4, B = 256 int8 31.8 / 44.1.
 PACKED_SPLIT_MAX_RAGGED = 2.25
+# A batch that runs unsplit without pairs is split in two for them from this many
+# tiles on: int8, T = 306, B = 164 10.1 us unsplit, 11.4 in two; T = 1024, B = 128
+# 16.2 and 14.6.
+PACKED_SPLIT_MIN_TILES = 24
 # Batches of short sequences that fill the CUs run unsplit, whatever their
 # size and merge or not: the flat split loses there, because its waves
 # switch sequences every few tiles. Per KV type, the longest sequence of a
@@ -309,6 +343,20 @@ def plan_num_splits(seq_lens, num_kv_heads: int, group: int, sm_count: int) -> t
     return int(splits), tmax
 
 
+def few_splits(batch: int, max_seq_len: int, num_kv_heads: int, group: int, sm_count: int) -> int:
+    """Splits of the classic kernel for a batch with at most one unsplit
+    workgroup per CU: as many as keep it at one per CU. One more would put two
+    on some CUs (an XCD holds the splits of neighbouring sequences): int8, B = 4,
+    T ~ U[512, 8192], 8 kv heads: 20.1 us with 8 splits, 25.1 with 10; B = 16,
+    T ~ U[300, 6000], 2 kv heads: 10.3 with 8, 13.0 with 9."""
+    tiles = _tiles(max_seq_len)
+    if tiles <= UNSPLIT_MAX_TILES:
+        return 1
+    splits = max(1, sm_count // max(1, batch * _units(num_kv_heads, group)))
+    splits = min(splits, max(FEW_SPLITS_MAX, tiles // FEW_SPLIT_LONG_TILES), tiles // MIN_SPLIT_TILES)
+    return max(1, min(splits, _abi.PA_MAX_SPLITS))
+
+
 def flat_splits_for(num_kv_heads: int, group: int, sm_count: int, waves_per_simd: int,
                     kv_dtype: str | None = None) -> int:
     """One round of waves over the (kv head, head tile) units: as many as
@@ -362,6 +410,9 @@ def plan_launch(batch: int, max_seq_len: int, num_kv_heads: int, group: int, sm_
     only `batch` and `max_seq_len` are known (a serving step's metadata,
     which holds the lengths on the device only), and the planner assumes
     a ragged batch whose every sequence may be that long. Rules, in order:
+      * with `kv_dtype` given and at most one unsplit workgroup per CU: the
+        classic kernel with `few_splits` splits, unless the flat split is the
+        better one (the rule at CLASSIC_STREAM_LOSS);
       * the flat split (one round of waves, `flat_splits_for`) when each of
         its waves gets at least MIN_FLAT_TILES_PER_WAVE tiles, the batch is
         at most FLAT_MAX_BATCH and is not a single sequence of up to
@@ -405,8 +456,8 @@ def packed_splits_for(seq_lens, plan: LaunchPlan, num_kv_heads: int, group: int,
     pairs, splits = batch * (num_kv_heads // 2), 1
     while splits * pairs < sm_count and _tiles(tmax) >= 2 * splits * MIN_SPLIT_TILES:
         splits *= 2
-    if plan.flat_splits == 0 and splits > 2:
-        return 0  # a small batch of the classic split: more splits cost more than pairs save
+    if plan.flat_splits == 0 and splits > 1 and (splits > 2 or _tiles(tmax) < PACKED_SPLIT_MIN_TILES):
+        return 0  # classic already: more splits, or a merge over short sequences, cost more than pairs save
     return min(splits, _abi.PA_MAX_SPLITS)
 
 
@@ -426,6 +477,18 @@ def _plan_launch(batch, max_seq_len, num_kv_heads, group, sm_count, waves_per_si
     flat = flat_splits_for(num_kv_heads, group, cus, waves_per_simd, kv_dtype)
     flat_ok = (batch <= FLAT_MAX_BATCH and tiles >= MIN_FLAT_TILES_PER_WAVE * flat
                and not (batch == 1 and _tiles(tmax) <= SINGLE_SEQ_SPLIT_MAX_TILES))
+    units = _units(num_kv_heads, group)
+    if 0 < batch * units <= cus and tmax > 0 and kv_dtype in CLASSIC_MARGIN_TILES:
+        splits = few_splits(batch, tmax, num_kv_heads, group, cus)
+        chunk = -(-_tiles(tmax) // splits)
+        if known and not _nearly_uniform(lens):
+            margin = (UNSPLIT_MARGIN_TILES if splits == 1 else CLASSIC_MARGIN_TILES)[kv_dtype]
+            classic = (1 + CLASSIC_STREAM_LOSS) * chunk <= tiles * units / cus + margin
+        else:
+            classic = chunk <= (UNSPLIT_MAX_CHUNK_TILES if splits == 1 else CLASSIC_MAX_CHUNK_TILES)[kv_dtype]
+        # (pairs of heads with known lengths: packed_splits_for chooses)
+        if not flat_ok or (classic and not (known and packs_heads(num_kv_heads, group, head_dim, kv_dtype))):
+            return LaunchPlan(splits, tmax, 0)
     if flat_ok:
         fills = known and _fills_unsplit(lens, num_kv_heads, group, cus)
         cost = RAGGED_FLAT_SEQ_COST_KV.get(kv_dtype, RAGGED_FLAT_SEQ_COST) \

@@ -1,4 +1,4 @@
-"""The merge by four waves a row (more than 8 splits; a flat split with 4 ranges a sequence or more)
+"""The merge by four waves a row (more than 8 splits; a flat split with 8 ranges a sequence or more)
 at the edges of its passes and of its rule."""
 
 from __future__ import annotations
@@ -33,10 +33,10 @@ def test_split_reduce_edges(splits, d):
     assert max_abs(got, want) < 2.0 ** -9 + 1e-5
 
 
-@pytest.mark.parametrize("batch,flat", [(8, 31), (8, 32), (8, 33), (3, 40), (1, 200)])
+@pytest.mark.parametrize("batch,flat", [(8, 63), (8, 64), (8, 65), (3, 40), (1, 200)])
 @pytest.mark.parametrize("kv_dtype", ["fp16", "int8"])
 def test_flat_rule_edges(batch, flat, kv_dtype):
-    """Either side of four ranges a sequence, host tables and the GPU scan alike, empty rows zero."""
+    """Either side of eight ranges a sequence, host tables and the GPU scan alike, empty rows zero."""
     lens = [(977 * i) % 3000 + 40 for i in range(batch)]
     if batch > 2:
         lens[1] = 0
