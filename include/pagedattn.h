@@ -309,6 +309,15 @@ int pa_decode_noalloc(const pa_decode_args *args, void *stream);
 int pa_flat_host_plan(const pa_decode_args *args, int32_t *ranges, int32_t *items, int32_t *n_items,
                       int32_t *in_kernel_args);
 
+/* For planners, on n host lengths (negative ones count as 0). stats[0 .. 2]: the
+ * longest, their sum, and their 32-token tiles in all. */
+int pa_lens_stats(const int32_t *lens, int n, int64_t *stats);
+
+/* *out = whether a flat decode of these host lengths (clamped to max_tokens) in
+ * flat_splits ranges with seq_cost tiles charged per sequence leaves work to its
+ * merge: a range boundary cuts a sequence, or one is empty. */
+int pa_flat_needs_merge(const int32_t *lens, int n, int max_tokens, int flat_splits, int seq_cost, int *out);
+
 /* Message for the last non-zero return on the calling thread ("" if none). */
 const char *pa_last_error(void);
 

@@ -328,8 +328,10 @@ extern "C" int pa_cache_write(const pa_cache_write_args *a, void *stream) {
   }
   const int64_t rows = (int64_t)a->num_tokens * a->num_kv_heads;
   const int64_t lanes = (int64_t)a->num_kv_heads * (a->head_dim / 8);  // of one token
-  const int64_t tpb = lanes <= 256 ? 256 / lanes : 1, parts = (lanes + 255) / 256;
-  const int64_t groups = (a->num_tokens + tpb - 1) / tpb * parts;
+  const bool whole = lanes <= 256;  // a group holds whole tokens
+  const uint32_t tpb = whole ? 256u / (uint32_t)lanes : 1u;
+  const int64_t parts = whole ? 1 : (lanes + 255) >> 8;
+  const int64_t groups = whole ? ((uint32_t)a->num_tokens + tpb - 1) / tpb : a->num_tokens * parts;
   if (lanes > 0xffffff00u || groups > 0x7fffffff)
     return pa_fail(PA_ERR_UNSUPPORTED, "too many rows (%lld)", (long long)rows);
   if (rows == 0) return pa_ok();
@@ -344,14 +346,12 @@ extern "C" int pa_cache_write(const pa_cache_write_args *a, void *stream) {
   p.slots = a->slot_mapping;
   p.tokens = (uint32_t)a->num_tokens;
   p.lanes = (uint32_t)lanes;
-  p.tpb = (uint32_t)tpb;
+  p.tpb = tpb;
   p.parts = (uint32_t)parts;
   p.groups = (uint32_t)groups;
-  p.inv_lanes = lanes <= 256 ? (65536u + (uint32_t)lanes - 1) / (uint32_t)lanes : 0;
+  p.inv_lanes = whole ? (65536u + (uint32_t)lanes - 1) / (uint32_t)lanes : 0;
   p.block_size = a->block_size;
-  p.log2_block = -1;
-  if ((a->block_size & (a->block_size - 1)) == 0)
-    for (p.log2_block = 0; (1 << p.log2_block) < a->block_size;) ++p.log2_block;
+  p.log2_block = (a->block_size & (a->block_size - 1)) == 0 ? __builtin_ctz(a->block_size) : -1;
   p.max_slot = (int64_t)a->num_blocks * a->block_size;
   p.skt = a->stride_kt * 2;
   p.skh = a->stride_kh * 2;

@@ -125,7 +125,7 @@ inline Div make_div(uint32_t d) {
   Div v = {d, 0, 0};
   if (d > 1) {
     const uint32_t l = 32 - __builtin_clz(d - 1);
-    v.mul = (uint32_t)((uint64_t(1) << (31 + l)) / d + 1);
+    v.mul = (d & (d - 1)) == 0 ? 0x80000001u : (uint32_t)((uint64_t(1) << (31 + l)) / d + 1);
     v.shift = l - 1;
   }
   return v;
@@ -1928,7 +1928,7 @@ int ilog2(int x) {
 }
 
 SplitDiv split_div(int max_seq_len, int num_splits) {
-  const int64_t tiles = ((int64_t)max_seq_len + kSplitAlign - 1) / kSplitAlign;
+  const uint32_t tiles = ((uint32_t)max_seq_len + kSplitAlign - 1) / kSplitAlign;
   SplitDiv s;
   s.max_seq_len = max_seq_len;
   s.chunk_tiles = (int)((tiles + num_splits - 1) / num_splits);
@@ -2156,7 +2156,8 @@ hipError_t launch_decode_t(const KParams &k, int grid, int mode, hipStream_t st,
     }
     return hipGetLastError();
   }
-  const ClassicArgs ca = {k, split_div(k.max_seq_len, k.num_splits), make_div(k.head_tiles), make_div(k.hkv)};
+  const ClassicArgs ca = {k, mode == kUnsplit ? SplitDiv{} : split_div(k.max_seq_len, k.num_splits),
+                          make_div(k.head_tiles), make_div(k.hkv)};
   if (mode == kAuto) {
     hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kAuto, PK>), g, blk, 0, st, ca);
   } else if (mode == kPartials) {
@@ -2538,9 +2539,11 @@ int pa_decode(const pa_decode_args *a, void *stream) {
       plan.mt.r = rp;
       e = launch_merge_table(plan.mt, a->head_dim, wide_flat(a), st);
     } else {
-      const AutoMergeArgs ma = {rp, split_div(a->max_seq_len, a->num_splits), make_div(a->num_q_heads)};
-      e = flat ? launch_reduce<kMergeFlat>(rp, a->batch, a->num_q_heads, a->head_dim, wide_flat(a), st)
-               : launch_reduce<kMergeAuto>(ma, a->batch, a->num_q_heads, a->head_dim, wide_splits(a->num_splits), st);
+      const int hq = a->num_q_heads, d = a->head_dim;
+      e = flat ? launch_reduce<kMergeFlat>(rp, a->batch, hq, d, wide_flat(a), st)
+               : launch_reduce<kMergeAuto>(
+                     AutoMergeArgs{rp, split_div(a->max_seq_len, a->num_splits), make_div(hq)}, a->batch, hq, d,
+                     wide_splits(a->num_splits), st);
     }
     if (e != hipSuccess) return fail(PA_ERR_HIP, "reduce launch failed: %s", hipGetErrorString(e));
   }
@@ -2647,6 +2650,48 @@ int pa_flat_host_plan(const pa_decode_args *a, int32_t *ranges, int32_t *items, 
   *n_items = all.n_items;
   if (in_kernel_args != nullptr)
     *in_kernel_args = (plan.ranges ? PA_HOST_PLAN_RANGES : 0) | (plan.merge_table ? PA_HOST_PLAN_MERGE : 0);
+  return ok();
+}
+
+int pa_lens_stats(const int32_t *lens, int n, int64_t *stats) {
+  if (n < 0 || (n > 0 && lens == nullptr) || stats == nullptr)
+    return fail(PA_ERR_INVALID, "lens and stats must be non-NULL, n %d >= 0", n);
+  int64_t longest = 0, sum = 0, tiles = 0;
+  for (int i = 0; i < n; ++i) {
+    const int64_t t = std::max(0, lens[i]);
+    longest = std::max(longest, t);
+    sum += t;
+    tiles += (t + kSplitAlign - 1) / kSplitAlign;
+  }
+  stats[0] = longest;
+  stats[1] = sum;
+  stats[2] = tiles;
+  return ok();
+}
+
+int pa_flat_needs_merge(const int32_t *lens, int n, int max_tokens, int flat_splits, int seq_cost, int *out) {
+  if (n < 0 || (n > 0 && lens == nullptr) || out == nullptr || seq_cost < 0)
+    return fail(PA_ERR_INVALID, "lens and out must be non-NULL, n %d and seq_cost %d >= 0", n, seq_cost);
+  *out = 1;
+  if (n == 0 || flat_splits <= 0) return ok();
+  auto tiles_of = [&](int i) {
+    return ((int64_t)std::max(0, std::min(lens[i], max_tokens)) + kSplitAlign - 1) / kSplitAlign;
+  };
+  int64_t total = 0;
+  for (int i = 0; i < n; ++i) {
+    const int64_t t = tiles_of(i);
+    if (t == 0) return ok();  // the merge writes an empty sequence's zeros
+    total += t + seq_cost;
+  }
+  const int64_t per = std::max<int64_t>(1, (total + flat_splits - 1) / flat_splits);
+  int64_t first = 0;
+  for (int i = 0; i < n; ++i) {
+    const int64_t t = tiles_of(i);
+    first += seq_cost;  // weight of the sequence's tile 0
+    if (first / per != (first + t - 1) / per) return ok();
+    first += t;
+  }
+  *out = 0;
   return ok();
 }
 

@@ -52,6 +52,8 @@ EXPORTED_SYMBOLS = (
     "pa_flat_merge",
     "pa_flat_waves_per_simd",
     "pa_flat_host_plan",
+    "pa_lens_stats",
+    "pa_flat_needs_merge",
     "pa_last_error",
     "pa_abi_version",
 )
@@ -202,6 +204,10 @@ def load() -> ctypes.CDLL:
         lib.pa_flat_waves_per_simd.restype = ctypes.c_int
         lib.pa_flat_host_plan.argtypes = [ctypes.POINTER(PaDecodeArgs), _vp, _vp, _vp, _vp]
         lib.pa_flat_host_plan.restype = ctypes.c_int
+        lib.pa_lens_stats.argtypes = [_vp, ctypes.c_int, _vp]
+        lib.pa_lens_stats.restype = ctypes.c_int
+        lib.pa_flat_needs_merge.argtypes = [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp]
+        lib.pa_flat_needs_merge.restype = ctypes.c_int
         lib.pa_last_error.argtypes = []
         lib.pa_last_error.restype = ctypes.c_char_p
         lib.pa_abi_version.argtypes = []
@@ -211,6 +217,14 @@ def load() -> ctypes.CDLL:
             raise HipLibraryMissing(f"{path} has ABI version {ver}, expected {PA_ABI_VERSION}")
         _LIB = lib
         return lib
+
+
+def load_if_built() -> ctypes.CDLL | None:
+    """The library, or None where it has not been built (for host-side helpers
+    that can do without it)."""
+    if _LIB is not None:
+        return _LIB
+    return load() if lib_path().exists() else None
 
 
 def check(rc: int, what: str) -> None:

@@ -257,17 +257,68 @@ def _lens_array(seq_lens) -> np.ndarray:
     return np.maximum(arr.astype(np.int64, copy=False).reshape(-1), 0)
 
 
+_STATS = ctypes.c_int64 * 3
+
+
+class _Lens:
+    """A batch's host lengths and what the planner asks of them: their number,
+    longest, sum and tiles, taken in one native pass where they are a contiguous
+    int32 CPU tensor (as the device lengths arrive), else with numpy (the 160
+    lengths of a ragged batch: 72 us of numpy calls per plan, 17 native)."""
+
+    __slots__ = ("size", "longest", "total", "tiles", "_native", "_array")
+
+    def __init__(self, seq_lens) -> None:
+        self._native = None
+        if (isinstance(seq_lens, torch.Tensor) and seq_lens.dtype == torch.int32 and seq_lens.dim() == 1
+                and not seq_lens.is_cuda and seq_lens.is_contiguous()):
+            lib = _abi.load_if_built()
+            if lib is not None:
+                stats = _STATS()
+                self.size = seq_lens.shape[0]
+                _abi.check(lib.pa_lens_stats(seq_lens.data_ptr(), self.size, stats), "pa_lens_stats")
+                self.longest, self.total, self.tiles = stats
+                self._native, self._array = seq_lens, None
+                return
+        self._array = arr = _lens_array(seq_lens)
+        self.size = int(arr.size)
+        self.longest = int(arr.max()) if self.size else 0
+        self.total, self.tiles = int(arr.sum()), int(_tiles_array(arr).sum())
+
+    @classmethod
+    def of(cls, seq_lens) -> _Lens:
+        return seq_lens if isinstance(seq_lens, _Lens) else cls(seq_lens)
+
+    def needs_merge(self, flat_splits: int, max_tokens: int | None, seq_cost: int) -> bool:
+        if self._native is not None:
+            got = ctypes.c_int(1)
+            most = 0x7fffffff if max_tokens is None else min(int(max_tokens), 0x7fffffff)
+            _abi.check(_abi.load().pa_flat_needs_merge(self._native.data_ptr(), self.size, most, int(flat_splits),
+                                                       int(seq_cost), ctypes.byref(got)), "pa_flat_needs_merge")
+            return bool(got.value)
+        lens = self._array
+        if max_tokens is not None:
+            lens = np.minimum(lens, max_tokens)
+        tiles = _tiles_array(lens)
+        weights = np.where(tiles > 0, tiles + seq_cost, 0)
+        total = int(weights.sum())
+        if total == 0 or flat_splits <= 0:
+            return True
+        if bool((tiles == 0).any()):
+            return True  # the merge writes an empty sequence's zeros
+        per = max(1, -(-total // flat_splits))
+        first = np.cumsum(weights) - weights + seq_cost  # weight of each sequence's tile 0
+        return bool(((first // per) != ((first + tiles - 1) // per)).any())
+
+
 def _tiles_array(lens: np.ndarray) -> np.ndarray:
     return (lens + (TILE_TOKENS - 1)) // TILE_TOKENS
 
 
 def _nearly_uniform(lens) -> bool:
     """Longest length at most 1.25 x the mean (a non-empty batch)."""
-    lens = _lens_array(lens)
-    if lens.size == 0:
-        return False
-    tmax = int(lens.max())
-    return tmax > 0 and tmax <= 1.25 * int(lens.sum()) / lens.size
+    lens = _Lens.of(lens)
+    return lens.longest > 0 and lens.longest <= 1.25 * lens.total / lens.size
 
 
 def packs_heads(num_kv_heads: int, group: int, head_dim: int | None, kv_dtype: str | None) -> bool:
@@ -278,7 +329,7 @@ def packs_heads(num_kv_heads: int, group: int, head_dim: int | None, kv_dtype: s
 
 def _fills_unsplit(lens, num_kv_heads: int, group: int, sm_count: int) -> bool:
     """A nearly uniform batch whose unsplit workgroups already give every CU one."""
-    lens = _lens_array(lens)
+    lens = _Lens.of(lens)
     return _nearly_uniform(lens) and lens.size * _units(num_kv_heads, group) >= max(1, sm_count)
 
 
@@ -320,14 +371,14 @@ def plan_num_splits(seq_lens, num_kv_heads: int, group: int, sm_count: int) -> t
         RAGGED_SPLIT_MIN_TILES tiles, else about four rounds of workgroups,
         chunk ~ sum(T) * heads / (4 CUs).
     """
-    lens = _lens_array(seq_lens)
-    if lens.size == 0 or int(lens.max()) == 0:
+    lens = _Lens.of(seq_lens)
+    if lens.longest == 0:
         return 1, 0
-    tmax = int(lens.max())
+    tmax = lens.longest
     units = _units(num_kv_heads, group)
     if _fills_unsplit(lens, num_kv_heads, group, sm_count) or _tiles(tmax) <= UNSPLIT_MAX_TILES:
         return 1, tmax
-    work, cus = int(lens.sum()) * units, max(1, sm_count)
+    work, cus = lens.total * units, max(1, sm_count)
     if lens.size * units >= cus:
         # every CU has a workgroup already (a ragged batch): split only long
         # sequences, into several rounds of workgroups
@@ -434,6 +485,8 @@ def plan_launch(batch: int, max_seq_len: int, num_kv_heads: int, group: int, sm_
     kernel would take pairs of heads, such a batch's plan also names the
     splits to launch it with instead (`packed_splits_for`).
     """
+    if seq_lens is not None:
+        seq_lens = _Lens.of(seq_lens)
     plan = _plan_launch(batch, max_seq_len, num_kv_heads, group, sm_count, waves_per_simd, kv_dtype,
                         head_dim, seq_lens)
     packed = packed_splits_for(seq_lens, plan, num_kv_heads, group, sm_count, kv_dtype, head_dim)
@@ -449,9 +502,9 @@ def packed_splits_for(seq_lens, plan: LaunchPlan, num_kv_heads: int, group: int,
     PACKED_SPLIT_MAX_RAGGED times the mean)."""
     if seq_lens is None or not packs_heads(num_kv_heads, group, head_dim, kv_dtype):
         return 0
-    lens = _lens_array(seq_lens)
-    batch, tmax = int(lens.size), plan.max_seq_len
-    if _tiles(tmax) <= UNSPLIT_MAX_TILES or tmax * batch > PACKED_SPLIT_MAX_RAGGED * int(lens.sum()):
+    lens = _Lens.of(seq_lens)
+    batch, tmax = lens.size, plan.max_seq_len
+    if _tiles(tmax) <= UNSPLIT_MAX_TILES or tmax * batch > PACKED_SPLIT_MAX_RAGGED * lens.total:
         return 0
     pairs, splits = batch * (num_kv_heads // 2), 1
     while splits * pairs < sm_count and _tiles(tmax) >= 2 * splits * MIN_SPLIT_TILES:
@@ -466,11 +519,9 @@ def _plan_launch(batch, max_seq_len, num_kv_heads, group, sm_count, waves_per_si
     """`plan_launch` without packed heads."""
     cus = max(1, sm_count)
     known = seq_lens is not None
-    lens = _lens_array(seq_lens) if known else None
+    lens = _Lens.of(seq_lens) if known else None
     if known:
-        batch = int(lens.size)
-        tmax = int(lens.max()) if batch else 0
-        tiles = int(_tiles_array(lens).sum())
+        batch, tmax, tiles = lens.size, lens.longest, lens.tiles
     else:
         tmax = max(0, int(max_seq_len))
         tiles = batch * _tiles(tmax)  # an upper bound
@@ -498,7 +549,7 @@ def _plan_launch(batch, max_seq_len, num_kv_heads, group, sm_count, waves_per_si
             if short_batch_runs_unsplit(batch, tmax, num_kv_heads, group, cus, kv_dtype,
                                         uniform=fills):
                 return LaunchPlan(1, tmax, 0)
-            kv_bytes = int(lens.sum()) * num_kv_heads * head_dim * _KV_ELEM_BYTES.get(kv_dtype, 2) * 2 \
+            kv_bytes = lens.total * num_kv_heads * head_dim * _KV_ELEM_BYTES.get(kv_dtype, 2) * 2 \
                 if known else 0
             limit = UNSPLIT_MAX_KV_BYTES_PER_CU.get(kv_dtype, 0)
             if head_dim * _KV_ELEM_BYTES.get(kv_dtype, 2) < UNSPLIT_MIN_ROW_BYTES:
@@ -519,8 +570,8 @@ def plan_decode(seq_lens, num_kv_heads: int, group: int, sm_count: int,
                 head_dim: int | None = None) -> tuple[int, int, int]:
     """(num_splits, max_seq_len, flat_splits) for a batch whose lengths the
     host knows: `plan_launch` with the lengths."""
-    lens = _lens_array(seq_lens)
-    p = plan_launch(int(lens.size), 0, num_kv_heads, group, sm_count, waves_per_simd, kv_dtype,
+    lens = _Lens.of(seq_lens)
+    p = plan_launch(lens.size, 0, num_kv_heads, group, sm_count, waves_per_simd, kv_dtype,
                     head_dim, seq_lens=lens)
     return p.num_splits, p.max_seq_len, p.flat_splits
 
@@ -538,19 +589,7 @@ def flat_needs_merge(seq_lens, flat_splits: int, max_tokens: int | None = None,
     launch's flat_seq_cost: a non-empty sequence weighs its tiles plus
     `seq_cost`, and the ranges take equal weight.
     """
-    lens = _lens_array(seq_lens)
-    if max_tokens is not None:
-        lens = np.minimum(lens, max_tokens)
-    tiles = _tiles_array(lens)
-    weights = np.where(tiles > 0, tiles + seq_cost, 0)
-    total = int(weights.sum())
-    if total == 0 or flat_splits <= 0:
-        return True
-    if bool((tiles == 0).any()):
-        return True  # the merge writes an empty sequence's zeros
-    per = max(1, -(-total // flat_splits))
-    first = np.cumsum(weights) - weights + seq_cost  # weight of each sequence's tile 0
-    return bool(((first // per) != ((first + tiles - 1) // per)).any())
+    return _Lens.of(seq_lens).needs_merge(flat_splits, max_tokens, seq_cost)
 
 
 class _Workspace:
@@ -588,6 +627,13 @@ class _Workspace:
         n_lse = b * hq * splits
         cur = self._ensure(n_out, n_lse, device)
         return cur[0][:n_out].view(b, hq, splits, d), cur[1][:n_lse].view(b, hq, splits)
+
+    def pointers(self, rows: int, d: int, device) -> tuple[int, int]:
+        """The workspace for `rows` partial rows of d floats and their
+        log2-sum-exps, as addresses: packed as `get` and `get_flat` view it,
+        without the views (four tensor objects a call)."""
+        out, lse = self._ensure(rows * d, rows, device)
+        return out.data_ptr(), lse.data_ptr()
 
     def get_flat(self, slots: int, hq: int, d: int, device) -> tuple[torch.Tensor, torch.Tensor]:
         """Flat-split slots: part_out [slots, hq, d], part_lse [slots, hq]."""
@@ -706,8 +752,10 @@ def _fill_args(
     flat_splits: int = 0,
     flat_seq_cost: int = 0,
     seq_lens_host: torch.Tensor | None = None,
+    workspace: tuple[int, int] | None = None,
 ) -> _abi.PaDecodeArgs:
-    """The pa_decode_args of one call: validated on the first call of its
+    """The pa_decode_args of one call (with the partials in part_out and
+    part_lse, or in `workspace` = `_Workspace.pointers`): validated on the first call of its
     geometry (`_pack_args`), afterwards a copy of that struct with this
     call's pointers (the C side validates every call again)."""
     k, v, bt, sl = cache.k_cache, cache.v_cache, cache.block_table, cache.seq_lens
@@ -718,7 +766,7 @@ def _fill_args(
            cache.kv_dtype, cache.block_size, shape.num_q_heads, shape.num_kv_heads, shape.head_dim,
            q.shape, q.stride(), q.dtype, q.get_device(), out.shape, out.stride(), out.dtype,
            out.get_device(), num_splits, sm_scale, max_seq_len, flat_splits, flat_seq_cost,
-           None if part_out is None else (part_out.shape, part_out.stride(), part_out.dtype,
+           workspace is not None if part_out is None else (part_out.shape, part_out.stride(), part_out.dtype,
                                           part_out.get_device(), part_lse.shape, part_lse.stride(),
                                           part_lse.dtype, part_lse.get_device()),
            seq_lens_host is None)
@@ -733,14 +781,16 @@ def _fill_args(
         a = _abi.PaDecodeArgs.from_buffer_copy(hit[1])
         a.q = q.data_ptr()
         a.out = out.data_ptr()
-        if part_out is not None:
+        if workspace is not None:
+            a.part_out, a.part_lse = workspace
+        elif part_out is not None:
             a.part_out = part_out.data_ptr()
             a.part_lse = part_lse.data_ptr()
         if seq_lens_host is not None and flat_splits > 0:
             a.seq_lens_host = seq_lens_host.data_ptr()
         return a
     tmpl = _pack_args(q, cache, out, num_splits, sm_scale, part_out, part_lse, max_seq_len,
-                      flat_splits, flat_seq_cost, seq_lens_host)
+                      flat_splits, flat_seq_cost, seq_lens_host, workspace)
     if len(_ARG_TEMPLATES) >= _ARG_TEMPLATES_MAX:
         _ARG_TEMPLATES.clear()
     refs = tuple(None if o is None else weakref.ref(o) for o in (k, v, bt, sl, ks, vs))
@@ -766,6 +816,7 @@ def _pack_args(
     flat_splits: int = 0,
     flat_seq_cost: int = 0,
     seq_lens_host: torch.Tensor | None = None,
+    workspace: tuple[int, int] | None = None,
 ) -> _abi.PaDecodeArgs:
     """Validate every tensor of a call and pack pa_decode_args."""
     b, hq, d = q.shape
@@ -827,7 +878,11 @@ def _pack_args(
     po = pl = None
     pst = (0, 0, 0)
     lst = (0, 0)
-    if part_out is not None:
+    if workspace is not None:  # packed [B + F, Hq, D] / [B + F, Hq] or [B, Hq, S, D] / [B, Hq, S]
+        po, pl = workspace
+        pst = (hq * d, d, 0) if flat_splits > 0 else (hq * num_splits * d, num_splits * d, d)
+        lst = (hq, 1) if flat_splits > 0 else (hq * num_splits, num_splits)
+    elif part_out is not None:
         po, pl = part_out.data_ptr(), part_lse.data_ptr()
         if flat_splits > 0:  # slots [B + F, Hq, D] / [B + F, Hq]
             if part_out.dim() != 3 or part_out.shape[0] < b + flat_splits or part_lse.shape[0] < b + flat_splits:
@@ -943,7 +998,6 @@ def paged_decode_hip(
         out = torch.empty((b, hq, d), dtype=q.dtype, device=q.device)
     if b == 0:
         return out
-    merge = True  # a flat decode runs its merge pass
     if flat_splits:
         num_splits = 1
         flat_seq_cost = int(flat_seq_cost or 0)
@@ -962,27 +1016,20 @@ def paged_decode_hip(
             flat_seq_cost = plan.flat_seq_cost
         if max_seq_len is None:
             max_seq_len = plan.max_seq_len
-        if flat_splits:
-            merge = flat_needs_merge(lens, flat_splits, cache.block_table.shape[1] * cache.block_size,
-                                     int(flat_seq_cost))
     num_splits = int(num_splits)
     scale = d ** -0.5 if sm_scale is None else float(sm_scale)  # shape.softmax_scale
 
-    part_out = part_lse = None
+    workspace = None
     flat = int(flat_splits or 0)
     if flat > 0:
         num_splits = 1
-        part_out, part_lse = _WS.get_flat(b + flat, hq, d, q.device)
+        workspace = _WS.pointers((b + flat) * hq, d, q.device)
     elif num_splits > 1:
-        part_out, part_lse = _WS.get(b, hq, num_splits, d, q.device)
-    args = _fill_args(q, cache, out, num_splits, scale, part_out, part_lse, max_seq_len or 0, flat,
-                      int(flat_seq_cost or 0) if flat else 0, seq_lens_host)
+        workspace = _WS.pointers(b * hq * num_splits, d, q.device)
+    args = _fill_args(q, cache, out, num_splits, scale, None, None, max_seq_len or 0, flat,
+                      int(flat_seq_cost or 0) if flat else 0, seq_lens_host, workspace)
     lib = _abi.load()
-    if flat > 0 and not merge:
-        # every sequence inside one range: the decode pass writes all of out
-        rc = _launch(q, lib.pa_decode_partials, args)
-        _abi.check(rc, "pa_decode_partials")
-        return out
+    # (with host lengths and every sequence inside one range, the library leaves the merge out)
     rc = _launch(q, lib.pa_decode, args)
     _abi.check(rc, "pa_decode")
     return out
