@@ -1172,20 +1172,31 @@ __device__ __forceinline__ int seq_tiles(const ro_i32 *seq_lens, int b, int max_
   return (t + kSplitAlign - 1) / kSplitAlign;
 }
 
-__device__ __forceinline__ int wave_sum(int x) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) x += __shfl_xor(x, o);
+// Wave-wide integer scan and sum by DPP adds inside rows of 16 lanes and
+// broadcasts of a row's last lane to the next rows (gfx9's row_bcast): six
+// dependent VALU adds, where shuffles through the LDS pipe take six round trips
+// of it, in front of a flat wave's first loads and in the merge that scans
+// seq_lens. Whole flat calls without host lengths, graph-timed, shuffles / DPP:
+// Llama-3-8B shape F = 128, B = 8 (T <= 2500) 18.6 / 17.6 us, B = 16 28.7 / 28.4,
+// B = 32 46.4 / 45.7, B = 64 fp8 41.1 / 40.5, B = 300 fp8 114.8 / 113.4; 14 q / 2 kv
+// heads F = 512, B = 200 43.8 / 42.4.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_add(int x) {
+  return x + __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false);
+}
+
+__device__ __forceinline__ int wave_incl_scan(int x) {
+  x = dpp_add<0x111, 0xf>(x);  // row_shr:1
+  x = dpp_add<0x112, 0xf>(x);  // row_shr:2
+  x = dpp_add<0x114, 0xf>(x);  // row_shr:4
+  x = dpp_add<0x118, 0xf>(x);  // row_shr:8
+  x = dpp_add<0x142, 0xa>(x);  // row_bcast:15 into rows 1 and 3
+  x = dpp_add<0x143, 0xc>(x);  // row_bcast:31 into rows 2 and 3
   return x;
 }
 
-__device__ __forceinline__ int wave_incl_scan(int x, int lane) {
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(x, o);
-    if (lane >= o) x += y;
-  }
-  return x;
-}
+// The sum over the wave, in every lane (all 64 lanes active).
+__device__ __forceinline__ int wave_sum(int x) { return __builtin_amdgcn_readlane(wave_incl_scan(x), 63); }
 
 // Total flat tiles of the batch (wave-uniform); `len0` receives this lane's
 // clamped length of sequence `lane` (0 past the batch).
@@ -1215,7 +1226,7 @@ __device__ __forceinline__ int flat_total(const ro_i32 *seq_lens, int batch, int
                                           int lane, int &len0) {
   if (batch <= 64) {  // one chunk
     len0 = lane < batch ? max(0, min(seq_lens[lane], max_tokens)) : 0;
-    return __builtin_amdgcn_readfirstlane(wave_sum(len_tiles(len0)));
+    return wave_sum(len_tiles(len0));
   }
   int total = 0;
   for (int base = 0; base < batch; base += 64 * kLenChunks) {
@@ -1244,12 +1255,12 @@ __device__ __forceinline__ SeqCursor flat_locate(const ro_i32 *seq_lens, int bat
   SeqCursor cur = {0, 0, 0, 0};
   if (len0 >= 0) {  // batch <= 64: one chunk, already loaded
     const int t = len_tiles(len0);
-    const int incl = wave_incl_scan(t, lane);
+    const int incl = wave_incl_scan(t);
     const uint64_t hit = __builtin_amdgcn_ballot_w64(incl > f);
     const int l = hit != 0 ? __builtin_ctzll(hit) : 0;
     cur.b = l;
-    cur.t = f - __shfl(incl - t, l);
-    cur.len = __shfl(len0, l);
+    cur.t = f - __builtin_amdgcn_readlane(incl - t, l);
+    cur.len = __builtin_amdgcn_readlane(len0, l);
   } else {
     int run = 0;  // tiles of the sequences before this pass
     for (int base = 0; base < batch; base += 64 * kLenChunks) {
@@ -1259,7 +1270,7 @@ __device__ __forceinline__ SeqCursor flat_locate(const ro_i32 *seq_lens, int bat
       int kk = -1;
 #pragma unroll
       for (int k = 0; k < kLenChunks; ++k) {
-        const int ck = __builtin_amdgcn_readfirstlane(wave_sum(len_tiles(len[k])));
+        const int ck = wave_sum(len_tiles(len[k]));
         if (kk < 0) {
           if (run + ck > f) kk = k;
           else run += ck;
@@ -1272,12 +1283,12 @@ __device__ __forceinline__ SeqCursor flat_locate(const ro_i32 *seq_lens, int bat
       for (int k = 0; k < kLenChunks; ++k)
         if (k == kk) lk = len[k];
       const int t = len_tiles(lk);
-      const int incl = wave_incl_scan(t, lane) + run;
+      const int incl = wave_incl_scan(t) + run;
       const uint64_t hit = __builtin_amdgcn_ballot_w64(incl > f);
       const int l = hit != 0 ? __builtin_ctzll(hit) : 0;
       cur.b = base + 64 * kk + l;
-      cur.t = f - __shfl(incl - t, l);
-      cur.len = __shfl(lk, l);
+      cur.t = f - __builtin_amdgcn_readlane(incl - t, l);
+      cur.len = __builtin_amdgcn_readlane(lk, l);
       break;
     }
   }
@@ -1305,7 +1316,7 @@ __device__ __forceinline__ SeqCursor flat_locate_weighted(const ro_i32 *seq_lens
     const int len = lane < batch ? max(0, min(seq_lens[lane], max_tokens)) : 0;
     const int t = len_tiles(len);
     const int w = seq_weight(t, cost);
-    const int incl = wave_incl_scan(w, lane);
+    const int incl = wave_incl_scan(w);
     const int W = __builtin_amdgcn_readlane(incl, 63);
     const int per = max(1, (W + F - 1) / F);
     const int r0 = j * per;
@@ -1349,7 +1360,7 @@ __device__ __forceinline__ SeqCursor flat_locate_weighted(const ro_i32 *seq_lens
     for (int k = 0; k < kLenChunks; ++k) {
       const int t = len_tiles(len[k]);
       const int w = seq_weight(t, cost);
-      const int incl = wave_incl_scan(w, lane) + run;
+      const int incl = wave_incl_scan(w) + run;
       const int first = incl - w + cost;
       const int a = min(max(r0 - first, 0), t), e = min(max(r1 - first, 0), t);
       start += wave_sum(a);
@@ -1508,8 +1519,10 @@ paged_decode_flat_kernel(const FlatArgs fa) {
       const float inv = (L > 0.f) ? 1.0f / L : 0.f;
       if (r16 < nh) {
         const int slot = cc.b + j;
-        store_acc<D, PK>(p, st.acc, inv, L, st.m, cc.b, qh0 + r16, c, seg_t0 == 0 && seq_end,
-                         (int64_t)slot * p.spb, (int64_t)slot * p.slb);
+        // (int8: its instances are short of scalar registers)
+        const KParams &e = KV == PA_KV_INT8 ? late_params() : p;
+        store_acc<D, PK>(e, st.acc, inv, L, st.m, cc.b, qh0 + r16, c, seg_t0 == 0 && seq_end,
+                         (int64_t)slot * e.spb, (int64_t)slot * e.slb);
       }
       if (i + 1 < n) {
         cursor_next(cc, ro(p.seq_lens), p.batch, p.max_tokens);
@@ -1820,8 +1833,9 @@ __global__ void __launch_bounds__((WIDE ? kWideWaves : kMergeWaves) * 64) split_
     int total = 0, cu = 0;  // all weight, weight before sequence b
     if (p.batch <= 64) {  // one chunk
       const int t = lane < p.batch ? seq_tiles(ro(p.seq_lens), lane, p.max_tokens) : 0;
-      total = wave_sum(seq_weight(t, cost));
-      cu = wave_sum(lane < b ? seq_weight(t, cost) : 0);
+      const int w = seq_weight(t, cost), incl = wave_incl_scan(w);
+      total = __builtin_amdgcn_readlane(incl, 63);
+      cu = __builtin_amdgcn_readlane(incl - w, b);
     }
     for (int base = 0; base < p.batch && p.batch > 64; base += 64 * kLenChunks) {
       int len[kLenChunks];
