@@ -156,8 +156,11 @@ typedef struct pa_decode_args {
    * (each start costs a wave about one tile of time) holds fewer tiles;
    * suits ragged batches. pa_flat_merge must be given the same value. */
   int32_t flat_seq_cost;
-  /* Flat split only (also an addition): the lengths in host memory, NULL
-   * when the caller has none. Given, they must equal seq_lens. The library
+  /* Also an addition: the lengths in host memory, NULL when the caller has
+   * none. Unsplit launches (num_splits 1, no flat split) of up to 1,024
+   * sequences and more than one round of workgroups start the longest sequences
+   * first (an order only: results do not depend on it, captured or not). Flat
+   * split: given, they must equal seq_lens. The library
    * then computes the ranges and the merge's list of cut and empty
    * sequences on the host and passes them in the kernel arguments, so no
    * wave reads seq_lens before its first K/V loads and the merge covers only

@@ -184,6 +184,20 @@ struct ClassicArgs {
   Div by_head_tiles, by_hkv;
 };
 
+// The unsplit kernel's arguments with an order of the batch: workgroups take
+// sequence order[0] first. Host lengths give the longest first: a ragged batch
+// of several rounds of workgroups otherwise ends with whatever long sequences
+// come last, alone on their CUs (eager unsplit calls, batch order / longest
+// first: fp16, 64 q / 8 kv heads, B = 160, T ~ U[32, 1023] 65.7 / 59.4 us; int8, B =
+// 200, T ~ U[100, 1000] 54.4 / 47.3; fp8, 32 / 8, B = 200 54.6 / 48.6). Selecting the
+// sequence of a rank inside each workgroup instead, for launches without host
+// lengths, cost 3-10 us a call.
+constexpr int kOrderMax = 1024;
+struct OrderedArgs : ClassicArgs {
+  uint16_t order[kOrderMax];
+};
+static_assert(sizeof(OrderedArgs) <= 4096, "kernel arguments over 4 KB");
+
 struct RParams {
   const float *part_out;
   const float *part_lse;
@@ -977,13 +991,15 @@ __device__ __forceinline__ SplitRange split_range(int seq_len, const SplitDiv &p
 //   kAuto      as kPartials for the splits that hold tokens; a sequence that
 //              fits in one split writes `out` directly, empty splits return at
 //              once (the merge kernel skips both)
-enum { kUnsplit = 0, kPartials = 1, kAuto = 2 };
+//   kOrdered   kUnsplit in the order of OrderedArgs
+enum { kUnsplit = 0, kPartials = 1, kAuto = 2, kOrdered = 4 };
 
 // Two workgroups (8 waves) per CU must fit in the register file: the
 // double-buffered tiles are sized for that budget.
-template <int KV, int SC, int D, int MODE, int PK>
+// ARGS: OrderedArgs for kOrdered, else ClassicArgs.
+template <int KV, int SC, int D, int MODE, int PK, typename ARGS>
 __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2)))
-paged_decode_kernel(const ClassicArgs ca) {
+paged_decode_kernel(const ARGS ca) {
   const KParams &p = ca.p;
   using G = Geo<KV, D>;
   constexpr int kRegs = 4 * G::kE;  // accumulator floats per lane
@@ -1009,17 +1025,20 @@ paged_decode_kernel(const ClassicArgs ca) {
   // 3-33% faster on split workloads (ragged most), 2% slower unsplit, so only
   // split launches remap. The tail past a multiple of 8 keeps its index.
   int wg = blockIdx.x;
-  if (MODE != kUnsplit) {
+  if (MODE != kUnsplit && MODE != kOrdered) {
     const int n = gridDim.x, full = n - n % 8;
     if (wg < full) wg = (wg % 8) * (full / 8) + wg / 8;
   }
   // wg = ((b * hkv + kvh) * head_tiles + ht) * num_splits + split
-  const int x1 = MODE == kUnsplit ? wg : div_by(wg, ca.s.by_splits);
-  const int split = MODE == kUnsplit ? 0 : wg - x1 * p.num_splits;
+  constexpr bool kWhole = MODE == kUnsplit || MODE == kOrdered;  // no splits
+  const int x1 = kWhole ? wg : div_by(wg, ca.s.by_splits);
+  const int split = kWhole ? 0 : wg - x1 * p.num_splits;
   const int x2 = div_by(x1, ca.by_head_tiles);
   const int ht = x1 - x2 * p.head_tiles;
-  const int b = div_by(x2, ca.by_hkv);
-  const int kvh = x2 - b * p.hkv;
+  const int rank = div_by(x2, ca.by_hkv);
+  const int kvh = x2 - rank * p.hkv;
+  int b = rank;
+  if constexpr (MODE == kOrdered) b = ca.order[rank];
 
   const int qh0 = kvh * p.group + ht * 16;
   const int nh = min(16, p.group - ht * 16);
@@ -1031,7 +1050,7 @@ paged_decode_kernel(const ClassicArgs ca) {
   // of the unsplit call at B = 24, T <= 192). The index is clamped to the row.
   const ro_i32 *bt_row = ro(p.bt) + (int64_t)b * p.sbtb;
   int guess_lo = 0;
-  if (MODE != kUnsplit) guess_lo = (int)min((uint32_t)split * (uint32_t)ca.s.chunk_tiles, kMaxTiles) << 5;
+  if (!kWhole) guess_lo = (int)min((uint32_t)split * (uint32_t)ca.s.chunk_tiles, kMaxTiles) << 5;
   const uint32_t guess = (uint32_t)guess_lo + wave * G::kTT;
   int early[2];
 #pragma unroll
@@ -1042,7 +1061,7 @@ paged_decode_kernel(const ClassicArgs ca) {
 
   int lo = 0, hi = seq_len;
   bool direct = true;  // write fp16 `out` (else a split partial)
-  if (MODE != kUnsplit) {
+  if (!kWhole) {
     const SplitRange r = split_range(seq_len, ca.s, split);
     if (MODE == kAuto && split >= r.n) return;  // an empty split: nothing to read or write
     lo = r.lo;
@@ -1062,7 +1081,7 @@ paged_decode_kernel(const ClassicArgs ca) {
   const int cnt = ntiles > wave ? (ntiles - wave + kWaves - 1) / kWaves : 0;
   auto n0_of = [&](int i) { return lo + (wave + kWaves * i) * G::kTT; };
   if (cnt > 0) {
-    if (MODE != kUnsplit && lo != guess_lo) {
+    if (!kWhole && lo != guess_lo) {
 #pragma unroll
       for (int u = 0; u < 2; ++u)
         early[u] = bt_row[min((uint32_t)(n0_of(0) + 16 * u) >> p.log2_page, (uint32_t)(p.max_blocks - 1))];
@@ -2147,12 +2166,33 @@ constexpr int kFlat = 3;
 // seq_lens_host): the flat ranges (FlatArgs) and the merge's sequences
 // (MergeTable), the same ranges the kernels would find by scanning seq_lens.
 struct HostPlan {
+  const int32_t *order_by = nullptr;  // unsplit: order the launch by these lengths
   bool ranges = false;       // fa holds the flat ranges
   bool merge_table = false;  // mt holds every sequence the merge must write
   bool needs_merge = true;   // some sequence is cut or empty
   FlatArgs fa;
   MergeTable mt;
 };
+
+// Sequence indices by length, longest first (equal ones by index).
+void longest_first(const int32_t *lens, int batch, uint16_t *order) {
+  uint64_t keys[kOrderMax];
+  for (int b = 0; b < batch; ++b)
+    keys[b] = (uint64_t)(0x7fffffff - std::max(0, lens[b])) << 16 | (uint64_t)b;
+  std::sort(keys, keys + batch);
+  for (int b = 0; b < batch; ++b) order[b] = (uint16_t)keys[b];
+}
+
+// Whether an unsplit launch is ordered by its host lengths: more workgroups than
+// the chip holds at once (the first kOrderMinWorkgroups all start together), and
+// not all of one length.
+constexpr int kOrderMinWorkgroups = 512;
+bool orders(const pa_decode_args *a, const KParams &k) {
+  if (a->seq_lens_host == nullptr || a->flat_splits > 0 || a->num_splits != 1 || a->batch > kOrderMax) return false;
+  if ((int64_t)a->batch * k.hkv * k.head_tiles <= kOrderMinWorkgroups) return false;
+  const auto mm = std::minmax_element(a->seq_lens_host, a->seq_lens_host + a->batch);
+  return *mm.second - (int64_t)*mm.first >= kSplitAlign;
+}
 
 template <int KV, int SC, int D, int PK>
 hipError_t launch_decode_t(const KParams &k, int grid, int mode, hipStream_t st, const HostPlan *hp) {
@@ -2172,12 +2212,17 @@ hipError_t launch_decode_t(const KParams &k, int grid, int mode, hipStream_t st,
   }
   const ClassicArgs ca = {k, mode == kUnsplit ? SplitDiv{} : split_div(k.max_seq_len, k.num_splits),
                           make_div(k.head_tiles), make_div(k.hkv)};
-  if (mode == kAuto) {
-    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kAuto, PK>), g, blk, 0, st, ca);
+  if (mode == kUnsplit && hp != nullptr && hp->order_by != nullptr) {
+    OrderedArgs oa;
+    static_cast<ClassicArgs &>(oa) = ca;
+    longest_first(hp->order_by, k.batch, oa.order);
+    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kOrdered, PK, OrderedArgs>), g, blk, 0, st, oa);
+  } else if (mode == kAuto) {
+    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kAuto, PK, ClassicArgs>), g, blk, 0, st, ca);
   } else if (mode == kPartials) {
-    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kPartials, PK>), g, blk, 0, st, ca);
+    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kPartials, PK, ClassicArgs>), g, blk, 0, st, ca);
   } else {
-    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kUnsplit, PK>), g, blk, 0, st, ca);
+    hipLaunchKernelGGL((paged_decode_kernel<KV, SC, D, kUnsplit, PK, ClassicArgs>), g, blk, 0, st, ca);
   }
   return hipGetLastError();
 }
@@ -2546,6 +2591,7 @@ int pa_decode(const pa_decode_args *a, void *stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
   HostPlan plan;
   if (flat) launch_host_plan(a, k, &plan, st);
+  if (orders(a, k)) plan.order_by = a->seq_lens_host;
   hipError_t e = launch_decode(k, a, flat ? kFlat : split ? kAuto : kUnsplit, st, &plan);
   if (e != hipSuccess) return fail(PA_ERR_HIP, "decode launch failed: %s", hipGetErrorString(e));
   if (split && !(flat && !plan.needs_merge)) {

@@ -205,6 +205,22 @@ WIDE_GROUP_MIN = 7
 # 469 / 439 (int8 at T = 1024 is the one case within 4% the other way).
 FLAT_MAX_BATCH = 1024
 
+# A ragged batch whose lengths the call itself reads (num_splits=None) runs
+# unsplit with its longest sequences first, instead of flat, from this much work
+# on: tiles per CU over the longest sequence's tiles (no CU then waits for one
+# sequence, and no wave switches sequences every few tiles).
+# ORDERED_MIN_ROUNDS_SHORT_ROWS: 2-byte KV at head_dim 64, whose flat split has
+# four times the ranges to merge. Eager whole calls, ordered / flat with host
+# tables in us, and the ratio: Llama-3-70B shape fp16 B = 160, T ~ U[32, 1023]
+# 59.4 / 64.8 (2.7), int8 B = 200, T ~ U[100, 1000] 47.3 / 51.0 (3.4), B = 96, T ~
+# U[64, 1500] 40.8 / 38.8 (1.6); Llama-3-8B shape fp16 B = 128, T ~ U[200, 3000]
+# 145.3 / 140.0 (2.3), bf16 B = 256, T log-uniform 16..1024 51.4 / 49.5 (2.0), fp8
+# B = 200, T ~ U[64, 1200] 48.6 / 46.4 (3.2); 14 q / 2 kv heads, D = 64, fp16 B =
+# 300, T ~ U[64, 1500] 24.1 / 28.2 (1.2), B = 512, T ~ U[32, 800] 21.9 / 32.0 (2.2).
+ORDERED_MIN_ROUNDS = {"fp16": 2.5, "bf16": 2.5, "int8": 3.0}
+ORDERED_MIN_ROUNDS_SHORT_ROWS = 1.0
+ORDERED_MAX_BATCH = 1024
+
 _KV_CODE = {"fp16": _abi.PA_KV_FP16, "fp8_e5m2": _abi.PA_KV_FP8_E5M2, "int8": _abi.PA_KV_INT8,
             "bf16": _abi.PA_KV_BF16}
 _STORE_DTYPE = {"fp16": torch.float16, "fp8_e5m2": torch.float8_e5m2, "int8": torch.int8,
@@ -489,8 +505,24 @@ def plan_launch(batch: int, max_seq_len: int, num_kv_heads: int, group: int, sm_
         seq_lens = _Lens.of(seq_lens)
     plan = _plan_launch(batch, max_seq_len, num_kv_heads, group, sm_count, waves_per_simd, kv_dtype,
                         head_dim, seq_lens)
-    packed = packed_splits_for(seq_lens, plan, num_kv_heads, group, sm_count, kv_dtype, head_dim)
-    return dataclasses.replace(plan, packed_splits=packed) if packed else plan
+    splits = packed_splits_for(seq_lens, plan, num_kv_heads, group, sm_count, kv_dtype, head_dim)
+    return dataclasses.replace(plan, packed_splits=splits) if splits else plan
+
+
+def ordered_batch_runs_unsplit(seq_lens, num_kv_heads: int, group: int, sm_count: int, kv_dtype: str | None,
+                               head_dim: int | None) -> bool:
+    """Whether a batch with known lengths runs faster unsplit, its longest
+    sequences first, than flat: ragged, more workgroups than two a CU, and
+    ORDERED_MIN_ROUNDS times the longest sequence's tiles of work for every CU."""
+    if seq_lens is None or head_dim is None or kv_dtype not in ORDERED_MIN_ROUNDS:
+        return False
+    lens = _Lens.of(seq_lens)
+    units = _units(num_kv_heads, group)
+    if lens.size > ORDERED_MAX_BATCH or lens.size * units <= 2 * sm_count or _nearly_uniform(lens):
+        return False
+    rounds = ORDERED_MIN_ROUNDS_SHORT_ROWS if head_dim * _KV_ELEM_BYTES[kv_dtype] <= UNSPLIT_MIN_ROW_BYTES \
+        and _KV_ELEM_BYTES[kv_dtype] == 2 else ORDERED_MIN_ROUNDS[kv_dtype]
+    return lens.tiles * units >= rounds * _tiles(lens.longest) * sm_count
 
 
 def packed_splits_for(seq_lens, plan: LaunchPlan, num_kv_heads: int, group: int, sm_count: int,
@@ -776,8 +808,7 @@ def _fill_args(
         hit = hit if (r[0]() is k and r[1]() is v and r[2]() is bt and r[3]() is sl
                       and (ks is None or r[4]() is ks) and (vs is None or r[5]() is vs)) else None
     if hit is not None:
-        if seq_lens_host is not None and flat_splits > 0:
-            _check_host_lens(seq_lens_host, q.shape[0])
+        host = _host_lens_pointer(seq_lens_host, q.shape[0], num_splits, flat_splits)
         a = _abi.PaDecodeArgs.from_buffer_copy(hit[1])
         a.q = q.data_ptr()
         a.out = out.data_ptr()
@@ -786,8 +817,8 @@ def _fill_args(
         elif part_out is not None:
             a.part_out = part_out.data_ptr()
             a.part_lse = part_lse.data_ptr()
-        if seq_lens_host is not None and flat_splits > 0:
-            a.seq_lens_host = seq_lens_host.data_ptr()
+        if host is not None:
+            a.seq_lens_host = host
         return a
     tmpl = _pack_args(q, cache, out, num_splits, sm_scale, part_out, part_lse, max_seq_len,
                       flat_splits, flat_seq_cost, seq_lens_host, workspace)
@@ -795,12 +826,30 @@ def _fill_args(
         _ARG_TEMPLATES.clear()
     refs = tuple(None if o is None else weakref.ref(o) for o in (k, v, bt, sl, ks, vs))
     _ARG_TEMPLATES[key] = (refs, tmpl)
-    return _abi.PaDecodeArgs.from_buffer_copy(tmpl)
+    args = _abi.PaDecodeArgs.from_buffer_copy(tmpl)
+    tmpl.seq_lens_host = None  # every call sets its own
+    return args
+
+
+def _host_lens_pointer(seq_lens_host, b: int, num_splits: int, flat_splits: int) -> int | None:
+    """The host lengths' address for launches that use them: flat ones, which
+    check them, and unsplit ones, which take them for an order where they are
+    what they should be and otherwise do without."""
+    if seq_lens_host is None or (flat_splits <= 0 and num_splits != 1):
+        return None
+    if flat_splits > 0:
+        _check_host_lens(seq_lens_host, b)
+    elif not (isinstance(seq_lens_host, torch.Tensor) and _is_host_lens(seq_lens_host, b)):
+        return None
+    return seq_lens_host.data_ptr()
+
+
+def _is_host_lens(t: torch.Tensor, b: int) -> bool:
+    return not t.is_cuda and t.dtype == torch.int32 and t.shape == (b,) and t.is_contiguous()
 
 
 def _check_host_lens(seq_lens_host: torch.Tensor, b: int) -> None:
-    if (seq_lens_host.device.type != "cpu" or seq_lens_host.dtype != torch.int32
-            or tuple(seq_lens_host.shape) != (b,) or not seq_lens_host.is_contiguous()):
+    if not _is_host_lens(seq_lens_host, b):
         raise ValueError(f"seq_lens_host must be a contiguous int32 CPU tensor of shape ({b},)")
 
 
@@ -892,10 +941,7 @@ def _pack_args(
             pst = part_out.stride()[:3]
         lst = part_lse.stride()[:2]
 
-    host_ptr = None
-    if seq_lens_host is not None and flat_splits > 0:
-        _check_host_lens(seq_lens_host, b)
-        host_ptr = seq_lens_host.data_ptr()
+    host_ptr = _host_lens_pointer(seq_lens_host, b, num_splits, flat_splits)
 
     # one constructor call, fields in declaration order (include/pagedattn.h)
     return _abi.PaDecodeArgs(
@@ -981,7 +1027,8 @@ def paged_decode_hip(
 
     `seq_lens_host` (an addition): the lengths as a contiguous int32 CPU
     tensor equal to `cache.seq_lens`, when the caller has them (a serving
-    step's metadata usually does). A flat launch then takes its ranges and
+    step's metadata usually does). A large unsplit launch starts the longest
+    sequences first (results do not depend on it). A flat launch then takes its ranges and
     its merge list from the host (no seq_lens scan on the GPU, no merge
     launch when no sequence is cut or empty). With `num_splits=None` the
     lengths come to the host anyway and are used so.
@@ -1012,6 +1059,9 @@ def paged_decode_hip(
         num_splits, flat_splits = plan.num_splits, plan.flat_splits
         if plan.packed_splits:
             num_splits, flat_splits = plan.packed_splits, 0
+        elif flat_splits and ordered_batch_runs_unsplit(lens, shape.num_kv_heads, shape.gqa_group,
+                                                        _cu_count(q.device), cache.kv_dtype, d):
+            flat_splits = 0  # (num_splits is 1)
         if flat_seq_cost is None:
             flat_seq_cost = plan.flat_seq_cost
         if max_seq_len is None:
