@@ -825,9 +825,9 @@ def _fill_args(
     if len(_ARG_TEMPLATES) >= _ARG_TEMPLATES_MAX:
         _ARG_TEMPLATES.clear()
     refs = tuple(None if o is None else weakref.ref(o) for o in (k, v, bt, sl, ks, vs))
-    _ARG_TEMPLATES[key] = (refs, tmpl)
     args = _abi.PaDecodeArgs.from_buffer_copy(tmpl)
-    tmpl.seq_lens_host = None  # every call sets its own
+    tmpl.seq_lens_host = None  # every call sets its own, also one of another thread from here on
+    _ARG_TEMPLATES[key] = (refs, tmpl)
     return args
 
 
