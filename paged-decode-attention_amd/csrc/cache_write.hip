@@ -57,7 +57,8 @@ struct WParams {
   uint32_t lanes;      // lanes of one token: num_kv_heads * head_dim / 8
   uint32_t tpb;        // tokens per group of 256 lanes (1 when a token takes several groups)
   uint32_t parts;      // groups per token (1 when a group holds whole tokens)
-  uint32_t groups;     // all groups; workgroup i takes groups i, i + gridDim.x, ...
+  uint32_t groups;     // all groups; workgroup i takes groups i, i + grid, ...
+  uint32_t grid;       // workgroups (gridDim.x would be read from the hidden arguments, cold)
   uint32_t inv_lanes;  // ceil(2^16 / lanes): x / lanes = x * inv_lanes >> 16 for x < 256, lanes <= 256
   int32_t block_size;
   int32_t log2_block;  // -1: block_size is not a power of two
@@ -206,7 +207,11 @@ template <int KV, int SC, int D, bool WIDE>
 __global__ void __launch_bounds__(256) cache_write_kernel(const WParams p) {
   constexpr int kLanesPerRow = D / 8;  // 8 fp16 (16 bytes) per lane
   const uint32_t tid = threadIdx.x;
-  for (uint32_t g = blockIdx.x; g < p.groups; g += gridDim.x) {
+  // The grid has at most p.groups workgroups, so the first pass needs no test:
+  // one would wait for its argument (cold on an eager launch) before the others
+  // are loaded.
+  uint32_t g = blockIdx.x;
+  do {
     uint32_t t, lane;  // token, lane in the token
     if (p.lanes <= 256) {
       const uint32_t tb = tid * p.inv_lanes >> 16;
@@ -262,7 +267,7 @@ __global__ void __launch_bounds__(256) cache_write_kernel(const WParams p) {
         }
       }
     }
-  }
+  } while ((g += p.grid) < p.groups);
 }
 
 template <int KV, int SC, int D>
@@ -362,7 +367,8 @@ extern "C" int pa_cache_write(const pa_cache_write_args *a, void *stream) {
   p.sch = a->stride_ch * elem;
   p.ssn = a->stride_sn * sb;
   p.sst = a->stride_st * sb;
-  const dim3 grid((uint32_t)(groups < kMaxGrid ? groups : kMaxGrid));
+  p.grid = (uint32_t)(groups < kMaxGrid ? groups : kMaxGrid);
+  const dim3 grid(p.grid);
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int d = a->head_dim;
   hipError_t e;
