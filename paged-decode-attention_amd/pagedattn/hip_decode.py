@@ -287,7 +287,7 @@ class _Lens:
     def __init__(self, seq_lens) -> None:
         self._native = None
         if (isinstance(seq_lens, torch.Tensor) and seq_lens.dtype == torch.int32 and seq_lens.dim() == 1
-                and not seq_lens.is_cuda and seq_lens.is_contiguous()):
+                and seq_lens.device.type == "cpu" and seq_lens.is_contiguous()):
             lib = _abi.load_if_built()
             if lib is not None:
                 stats = _STATS()
@@ -845,7 +845,7 @@ def _host_lens_pointer(seq_lens_host, b: int, num_splits: int, flat_splits: int)
 
 
 def _is_host_lens(t: torch.Tensor, b: int) -> bool:
-    return not t.is_cuda and t.dtype == torch.int32 and t.shape == (b,) and t.is_contiguous()
+    return t.device.type == "cpu" and t.dtype == torch.int32 and t.shape == (b,) and t.is_contiguous()
 
 
 def _check_host_lens(seq_lens_host: torch.Tensor, b: int) -> None:

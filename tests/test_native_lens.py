@@ -60,3 +60,20 @@ def test_argument_checks():
     assert lib.pa_flat_needs_merge(None, 2, 5, 1, 0, ctypes.byref(out)) == _abi.PA_ERR_INVALID
     assert lib.pa_flat_needs_merge(None, 0, 5, 1, -1, ctypes.byref(out)) == _abi.PA_ERR_INVALID
     assert lib.pa_flat_needs_merge(None, 0, 5, 1, 0, None) == _abi.PA_ERR_INVALID
+
+
+def test_host_lengths_are_cpu_tensors():
+    """A tensor without host memory (meta: its address reads as none given) is refused by flat
+    launches, left out of unsplit ones, and never handed to the native pass."""
+    from pagedattn.hip_decode import _check_host_lens, _host_lens_pointer
+
+    ok, meta = torch.tensor([5, 6, 7], dtype=torch.int32), torch.empty(3, dtype=torch.int32, device="meta")
+    _check_host_lens(ok, 3)
+    assert _host_lens_pointer(ok, 3, 1, 0) == _host_lens_pointer(ok, 3, 1, 8) == ok.data_ptr()
+    with pytest.raises(ValueError, match="contiguous int32 CPU tensor"):
+        _check_host_lens(meta, 3)
+    with pytest.raises(ValueError, match="contiguous int32 CPU tensor"):
+        _host_lens_pointer(meta, 3, 1, 8)
+    assert _host_lens_pointer(meta, 3, 1, 0) is None
+    with pytest.raises(NotImplementedError):  # torch's own refusal to read it, not the library's
+        _Lens(meta)
