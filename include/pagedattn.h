@@ -321,6 +321,12 @@ int pa_lens_stats(const int32_t *lens, int n, int64_t *stats);
  * merge: a range boundary cuts a sequence, or one is empty. */
 int pa_flat_needs_merge(const int32_t *lens, int n, int max_tokens, int flat_splits, int seq_cost, int *out);
 
+/* *out = whether the classic decode of these arguments (flat_splits 0) takes
+ * pairs of kv heads: by the heads' geometry and type, the strides and alignment
+ * of the cache and its scales, and the number of workgroups. Validates the
+ * arguments as pa_decode does and makes no HIP call. */
+int pa_decode_pairs(const pa_decode_args *args, int *out);
+
 /* Message for the last non-zero return on the calling thread ("" if none). */
 const char *pa_last_error(void);
 

@@ -2755,6 +2755,16 @@ int pa_flat_needs_merge(const int32_t *lens, int n, int max_tokens, int flat_spl
   return ok();
 }
 
+int pa_decode_pairs(const pa_decode_args *a, int *out) {
+  if (out == nullptr) return fail(PA_ERR_INVALID, "out is NULL");
+  *out = 0;
+  KParams k;
+  const int rc = build_params(a, a != nullptr && a->num_splits > 1, &k);
+  if (rc != PA_OK) return rc;
+  *out = k.pack == 2;
+  return ok();
+}
+
 int pa_flat_waves_per_simd(int kv_dtype, int scale_dtype, int head_dim, int *out) {
   if (out == nullptr) return fail(PA_ERR_INVALID, "out is NULL");
   *out = 0;

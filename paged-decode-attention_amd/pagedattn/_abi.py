@@ -54,6 +54,7 @@ EXPORTED_SYMBOLS = (
     "pa_flat_host_plan",
     "pa_lens_stats",
     "pa_flat_needs_merge",
+    "pa_decode_pairs",
     "pa_last_error",
     "pa_abi_version",
 )
@@ -208,6 +209,8 @@ def load() -> ctypes.CDLL:
         lib.pa_lens_stats.restype = ctypes.c_int
         lib.pa_flat_needs_merge.argtypes = [_vp, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _vp]
         lib.pa_flat_needs_merge.restype = ctypes.c_int
+        lib.pa_decode_pairs.argtypes = [ctypes.POINTER(PaDecodeArgs), _vp]
+        lib.pa_decode_pairs.restype = ctypes.c_int
         lib.pa_last_error.argtypes = []
         lib.pa_last_error.restype = ctypes.c_char_p
         lib.pa_abi_version.argtypes = []

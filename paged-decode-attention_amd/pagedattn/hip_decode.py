@@ -158,6 +158,10 @@ UNSPLIT_MAX_SHORT_ROW_BYTES_PER_CU = 192 << 10
 # over a factor of 64 (longest 4 times the mean) flat wins: B = 32 fp8 21.3 /
 # 27.4, B = 256 int8 31.8 / 44.1.
 PACKED_SPLIT_MAX_RAGGED = 2.25
+# The library takes pairs from this many workgroups of them on, whatever the
+# device (kPackMinWorkgroups in csrc/paged_decode.hip); with fewer, as a small
+# batch on a partition of few CUs has, a launch cut for pairs would run without.
+PACKED_MIN_WORKGROUPS = 192
 # A batch that runs unsplit without pairs is split in two for them from this many
 # tiles on: int8, T = 306, B = 164 10.1 us unsplit, 11.4 in two; T = 1024, B = 128
 # 16.2 and 14.6.
@@ -541,6 +545,8 @@ def packed_splits_for(seq_lens, plan: LaunchPlan, num_kv_heads: int, group: int,
     pairs, splits = batch * (num_kv_heads // 2), 1
     while splits * pairs < sm_count and _tiles(tmax) >= 2 * splits * MIN_SPLIT_TILES:
         splits *= 2
+    if pairs * splits < PACKED_MIN_WORKGROUPS:
+        return 0
     if plan.flat_splits == 0 and splits > 1 and (splits > 2 or _tiles(tmax) < PACKED_SPLIT_MIN_TILES):
         return 0  # classic already: more splits, or a merge over short sequences, cost more than pairs save
     return min(splits, _abi.PA_MAX_SPLITS)

@@ -1,0 +1,81 @@
+"""The planner's rules for pairs of kv heads, few-split classic launches and ordered batches, on both
+sides of each line, and its plans against the library's own rules. CPU only."""
+
+from __future__ import annotations
+
+import ctypes
+import random
+
+import pytest
+
+from pagedattn import _abi, plan_launch
+
+FAKE = 0x10000  # 16-byte aligned, never dereferenced
+
+
+def decode_args(batch, hq, hkv, kv, d=64, splits=1, **over):
+    """pa_decode_args of a contiguous cache, as the library's checks see them."""
+    a = _abi.PaDecodeArgs()
+    a.q = a.k_cache = a.v_cache = a.out = a.block_table = a.seq_lens = a.part_out = a.part_lse = FAKE
+    a.batch, a.num_q_heads, a.num_kv_heads, a.head_dim = batch, hq, hkv, d
+    a.block_size, a.num_blocks, a.max_blocks, a.num_splits = 16, 64, 8, splits
+    a.stride_qb, a.stride_qh = hq * d, d
+    a.stride_kn, a.stride_kt, a.stride_kh = 16 * hkv * d, hkv * d, d
+    a.stride_ob, a.stride_oh = hq * d, d
+    a.stride_btb = 8
+    a.kv_dtype = {"fp16": _abi.PA_KV_FP16, "bf16": _abi.PA_KV_BF16, "fp8_e5m2": _abi.PA_KV_FP8_E5M2,
+                  "int8": _abi.PA_KV_INT8}[kv]
+    a.scale_dtype = _abi.PA_SCALE_NONE
+    if kv == "int8":
+        a.k_scale = a.v_scale = FAKE
+        a.scale_dtype, a.stride_sn, a.stride_st = _abi.PA_SCALE_FP16, 16 * hkv, hkv
+    a.io_dtype = _abi.PA_IO_FP16
+    a.sm_scale = d ** -0.5
+    for k, v in over.items():
+        setattr(a, k, v)
+    return a
+
+
+def pairs(a) -> bool:
+    out = ctypes.c_int(-1)
+    _abi.check(_abi.load().pa_decode_pairs(ctypes.byref(a), ctypes.byref(out)), "pa_decode_pairs")
+    return bool(out.value)
+
+
+@pytest.mark.parametrize("cus", [32, 64, 128, 256, 304])
+def test_plans_for_pairs_get_pairs(cus):
+    """Whatever the device's size, a plan cut for pairs of heads is one that the library runs on pairs."""
+    r = random.Random(cus)
+    packed = 0
+    for _ in range(1500):
+        batch, hi = r.randint(1, 600), int(2 ** r.uniform(6, 16))
+        lens = [r.randint(max(1, hi // r.choice([1, 3])), hi) for _ in range(batch)]
+        kv, hkv, group = r.choice([("fp8_e5m2", 2, 7), ("int8", 2, 7), ("int8", 4, 4), ("fp8_e5m2", 8, 8)])
+        plan = plan_launch(batch, 0, hkv, group, cus, 2, kv_dtype=kv, head_dim=64, seq_lens=lens)
+        if plan.packed_splits:
+            packed += 1
+            assert pairs(decode_args(batch, hkv * group, hkv, kv, splits=plan.packed_splits)), (batch, hi, plan)
+    assert packed > 100
+
+
+def test_library_rule_for_pairs():
+    ok = decode_args(192, 14, 2, "int8")
+    assert pairs(ok)
+    # one workgroup of pairs fewer than the library's least, counted over the splits
+    assert not pairs(decode_args(191, 14, 2, "int8"))
+    assert pairs(decode_args(64, 14, 2, "int8", splits=3)) and not pairs(decode_args(64, 14, 2, "int8", splits=2))
+    # types, head dims, head counts and groups
+    assert pairs(decode_args(192, 14, 2, "fp8_e5m2")) and not pairs(decode_args(192, 14, 2, "fp16"))
+    assert not pairs(decode_args(192, 14, 2, "int8", d=128)) and not pairs(decode_args(192, 14, 2, "int8", d=32))
+    assert not pairs(decode_args(192, 6, 3, "int8")) and not pairs(decode_args(192, 18, 2, "int8"))
+    assert pairs(decode_args(192, 16, 2, "int8"))
+    # heads apart, a token stride under a pair, odd scales
+    assert not pairs(decode_args(192, 14, 2, "int8", stride_kh=128, stride_kt=256, stride_kn=4096))
+    assert not pairs(decode_args(192, 14, 2, "int8", stride_kt=64))
+    assert not pairs(decode_args(192, 14, 2, "int8", k_scale=FAKE + 2))
+    assert not pairs(decode_args(192, 14, 2, "int8", stride_st=3, stride_sn=48))
+    # a flat launch never does
+    assert not pairs(decode_args(192, 14, 2, "int8", flat_splits=512))
+    bad = ctypes.c_int(7)
+    assert _abi.load().pa_decode_pairs(None, ctypes.byref(bad)) == _abi.PA_ERR_INVALID and bad.value == 0
+    assert _abi.load().pa_decode_pairs(ctypes.byref(ok), None) == _abi.PA_ERR_INVALID
