@@ -324,7 +324,8 @@ int pa_flat_needs_merge(const int32_t *lens, int n, int max_tokens, int flat_spl
 /* *out = whether the classic decode of these arguments (flat_splits 0) takes
  * pairs of kv heads: by the heads' geometry and type, the strides and alignment
  * of the cache and its scales, and the number of workgroups. Validates the
- * arguments as pa_decode does and makes no HIP call. */
+ * arguments (the classic split's workspace aside, which may be NULL) as
+ * pa_decode does and makes no HIP call. */
 int pa_decode_pairs(const pa_decode_args *args, int *out);
 
 /* Message for the last non-zero return on the calling thread ("" if none). */

@@ -2759,7 +2759,7 @@ int pa_decode_pairs(const pa_decode_args *a, int *out) {
   if (out == nullptr) return fail(PA_ERR_INVALID, "out is NULL");
   *out = 0;
   KParams k;
-  const int rc = build_params(a, a != nullptr && a->num_splits > 1, &k);
+  const int rc = build_params(a, false, &k);
   if (rc != PA_OK) return rc;
   *out = k.pack == 2;
   return ok();

@@ -452,7 +452,8 @@ class LaunchPlan:
     tiles of weight the flat split charges each sequence (0 = equal tiles).
     `packed_splits` > 0: launch the classic kernel with that many splits
     instead, which takes pairs of heads and is faster; the other fields then
-    describe the launch without them.
+    describe the launch without them, for a cache whose layout does not pair
+    (`launch_kwargs` carries both: the plan does not see the cache).
     """
 
     num_splits: int
@@ -465,7 +466,10 @@ class LaunchPlan:
     def launch_kwargs(self) -> dict:
         """Keywords of `paged_decode_hip` that select this launch."""
         if self.packed_splits:
-            return {"num_splits": self.packed_splits, "max_seq_len": self.max_seq_len}
+            kw = {"num_splits": self.packed_splits, "max_seq_len": self.max_seq_len}
+            if (self.packed_splits, 0) != (self.num_splits, self.flat_splits):
+                kw["unpaired"] = (self.num_splits, self.flat_splits, self.flat_seq_cost)
+            return kw
         if self.flat_splits:
             return {"flat_splits": self.flat_splits, "flat_seq_cost": self.flat_seq_cost}
         return {"num_splits": self.num_splits, "max_seq_len": self.max_seq_len}
@@ -837,6 +841,13 @@ def _fill_args(
     return args
 
 
+def _takes_pairs(args: _abi.PaDecodeArgs) -> bool:
+    """Whether the library runs this classic launch on pairs of kv heads."""
+    got = ctypes.c_int(0)
+    _abi.check(_abi.load().pa_decode_pairs(ctypes.byref(args), ctypes.byref(got)), "pa_decode_pairs")
+    return bool(got.value)
+
+
 def _host_lens_pointer(seq_lens_host, b: int, num_splits: int, flat_splits: int) -> int | None:
     """The host lengths' address for launches that use them: flat ones, which
     check them, and unsplit ones, which take them for an order where they are
@@ -1003,6 +1014,7 @@ def paged_decode_hip(
     flat_splits: int | None = None,
     flat_seq_cost: int | None = None,
     seq_lens_host: torch.Tensor | None = None,
+    unpaired: tuple[int, int, int] | None = None,
 ) -> torch.Tensor:
     """Paged GQA decode attention. q: [B, Hq, D] fp16|bf16 -> [B, Hq, D] in q's dtype.
 
@@ -1038,6 +1050,11 @@ def paged_decode_hip(
     its merge list from the host (no seq_lens scan on the GPU, no merge
     launch when no sequence is cut or empty). With `num_splits=None` the
     lengths come to the host anyway and are used so.
+
+    `unpaired` (an addition, from `LaunchPlan.launch_kwargs`): `num_splits` was
+    planned for pairs of kv heads; where this cache's layout does not pair
+    (heads or scales apart), the launch (num_splits, flat_splits,
+    flat_seq_cost) is made instead.
     """
     del per_page_bt, num_warps, num_stages
     b, hq, d = q.shape
@@ -1064,6 +1081,7 @@ def paged_decode_hip(
                            kv_dtype=cache.kv_dtype, head_dim=d, seq_lens=lens)
         num_splits, flat_splits = plan.num_splits, plan.flat_splits
         if plan.packed_splits:
+            unpaired = plan.launch_kwargs().get("unpaired")
             num_splits, flat_splits = plan.packed_splits, 0
         elif flat_splits and ordered_batch_runs_unsplit(lens, shape.num_kv_heads, shape.gqa_group,
                                                         _cu_count(q.device), cache.kv_dtype, d):
@@ -1084,6 +1102,10 @@ def paged_decode_hip(
         workspace = _WS.pointers(b * hq * num_splits, d, q.device)
     args = _fill_args(q, cache, out, num_splits, scale, None, None, max_seq_len or 0, flat,
                       int(flat_seq_cost or 0) if flat else 0, seq_lens_host, workspace)
+    if unpaired is not None and not flat and not _takes_pairs(args):
+        splits, flat, cost = unpaired
+        return paged_decode_hip(q, cache, out, block_n, splits, sm_scale=sm_scale, max_seq_len=max_seq_len,
+                                flat_splits=flat, flat_seq_cost=cost, seq_lens_host=seq_lens_host)
     lib = _abi.load()
     # (with host lengths and every sequence inside one range, the library leaves the merge out)
     rc = _launch(q, lib.pa_decode, args)
@@ -1106,6 +1128,7 @@ def decode_noalloc(
     sm_scale: float | None = None,
     flat_seq_cost: int = 0,
     seq_lens_host: torch.Tensor | None = None,
+    unpaired: tuple[int, int, int] | None = None,
 ) -> torch.Tensor:
     """The decode through pa_decode_noalloc, which allocates nothing.
 
@@ -1117,6 +1140,7 @@ def decode_noalloc(
     (HIP graph capture, allocation-free serving loops). `out` must be given.
     Calls that overlap on one GPU share the scratch and race. A launch whose
     partials do not fit raises NotImplementedError before anything runs.
+    `unpaired` as for `paged_decode_hip`.
     """
     if out is None:
         raise ValueError("decode_noalloc writes into a caller-supplied out")
@@ -1124,6 +1148,9 @@ def decode_noalloc(
     flat = int(flat_splits or 0)
     args = _fill_args(q, cache, out, 1 if flat else int(num_splits), scale, None, None,
                       int(max_seq_len or 0), flat, int(flat_seq_cost or 0) if flat else 0, seq_lens_host)
+    if unpaired is not None and not flat and not _takes_pairs(args):
+        splits, flat, cost = unpaired
+        return decode_noalloc(q, cache, out, splits, max_seq_len, flat, sm_scale, cost, seq_lens_host)
     lib = _abi.load()
     rc = _launch(q, lib.pa_decode_noalloc, args)
     _abi.check(rc, "pa_decode_noalloc")

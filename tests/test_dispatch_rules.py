@@ -74,8 +74,23 @@ def test_library_rule_for_pairs():
     assert not pairs(decode_args(192, 14, 2, "int8", stride_kt=64))
     assert not pairs(decode_args(192, 14, 2, "int8", k_scale=FAKE + 2))
     assert not pairs(decode_args(192, 14, 2, "int8", stride_st=3, stride_sn=48))
+    # (the workspace has no say)
+    assert pairs(decode_args(64, 14, 2, "int8", splits=3, part_out=None, part_lse=None))
     # a flat launch never does
     assert not pairs(decode_args(192, 14, 2, "int8", flat_splits=512))
     bad = ctypes.c_int(7)
     assert _abi.load().pa_decode_pairs(None, ctypes.byref(bad)) == _abi.PA_ERR_INVALID and bad.value == 0
     assert _abi.load().pa_decode_pairs(ctypes.byref(ok), None) == _abi.PA_ERR_INVALID
+
+
+def test_plans_for_pairs_carry_the_launch_without_them():
+    """A plan does not see the cache: the keywords of a launch cut for pairs hold the other one, too."""
+    lens = [2048] * 256
+    kw = dict(kv_dtype="int8", head_dim=64, seq_lens=lens)
+    plan = plan_launch(256, 0, 2, 7, 256, 2, **kw)
+    assert plan.packed_splits == 1 and plan.flat_splits > 0
+    assert plan.launch_kwargs() == {"num_splits": 1, "max_seq_len": 2048,
+                                    "unpaired": (plan.num_splits, plan.flat_splits, plan.flat_seq_cost)}
+    # the same launch either way: nothing to carry
+    short = plan_launch(512, 0, 2, 7, 256, 2, kv_dtype="int8", head_dim=64, seq_lens=[320] * 512)
+    assert short.flat_splits == 0 and short.num_splits == 1 and "unpaired" not in short.launch_kwargs()

@@ -112,3 +112,47 @@ def test_forms_that_do_not_pair(form):
     q = seeded_q(len(lens), c.shape.num_q_heads, 64, 66, device="cuda")
     got = paged_decode_hip(q, c, num_splits=1)
     assert max_abs(got, oracle.reference_decode(q, c, out_dtype=torch.float32)) < 2e-3
+
+
+@pytest.mark.parametrize("form", ["contiguous", "head stride", "scale offset"])
+@pytest.mark.parametrize("entry", ["default", "planned", "noalloc"])
+def test_launch_of_a_cache_that_does_not_pair(monkeypatch, form, entry):
+    """A batch planned for pairs runs on them where the cache's layout pairs and otherwise takes the
+    launch without them: the flat split here."""
+    from pagedattn import hip_decode, plan_launch
+    from pagedattn.hip_decode import decode_noalloc
+
+    lens = [1500 + (i * 37) % 500 for i in range(256)]
+    c = _cache(14, 2, lens, "int8", torch.float16)
+    if form == "head stride":  # heads 128 bytes apart
+        wide = [torch.zeros((*t.shape[:3], 128), dtype=t.dtype, device="cuda") for t in (c.k_cache, c.v_cache)]
+        for w, t in zip(wide, (c.k_cache, c.v_cache)):
+            w[..., :64] = t
+        c = dataclasses.replace(c, k_cache=wide[0][..., :64], v_cache=wide[1][..., :64])
+    elif form == "scale offset":  # scales at odd half words
+        wide = [torch.zeros((*t.shape[:2], 3), dtype=t.dtype, device="cuda") for t in (c.k_scale, c.v_scale)]
+        for w, t in zip(wide, (c.k_scale, c.v_scale)):
+            w[..., 1:] = t
+        c = dataclasses.replace(c, k_scale=wide[0][..., 1:], v_scale=wide[1][..., 1:])
+    wps = hip_decode.flat_waves_per_simd("int8", 64, torch.float16)
+    plan = plan_launch(256, 0, 2, 7, hip_decode._cu_count(c.k_cache.device), wps, kv_dtype="int8", head_dim=64,
+                       seq_lens=lens)
+    assert plan.packed_splits and plan.flat_splits
+    launched = []
+    real = hip_decode._launch
+    monkeypatch.setattr(hip_decode, "_launch", lambda t, fn, a: launched.append(
+        (a.num_splits, a.flat_splits, a.flat_seq_cost)) or real(t, fn, a))
+    q = seeded_q(256, 14, 64, 67, device="cuda")
+    if entry == "default":
+        got = paged_decode_hip(q, c)
+    elif entry == "planned":
+        got = paged_decode_hip(q, c, **plan.launch_kwargs())
+    else:
+        got = decode_noalloc(q, c, torch.empty_like(q), **plan.launch_kwargs())
+    want = (plan.packed_splits, 0, 0) if form == "contiguous" else (1, plan.flat_splits, plan.flat_seq_cost)
+    assert launched == [want]
+    from helpers import subset_cache
+
+    rows = [0, 100, 255]
+    ref = oracle.reference_decode(q[rows].cpu(), subset_cache(c, rows), out_dtype=torch.float32)
+    assert max_abs(got[rows], ref) < 2e-3
