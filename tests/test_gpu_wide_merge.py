@@ -49,3 +49,15 @@ def test_flat_rule_edges(batch, flat, kv_dtype):
     if batch > 2:
         want[1] = 0
     assert max_abs(a, want) < 2e-3
+
+
+@pytest.mark.parametrize("splits", [9, 33, 70])
+def test_infinity_in_the_last_partial(splits):
+    """The places of a pass past the last partial repeat its loads and count for nothing: an infinity
+    there (an fp8 cache's overflow) stays one."""
+    g = torch.Generator().manual_seed(74)
+    part = torch.randn((1, 2, splits, 128), generator=g)
+    part[0, 1, splits - 1, 5] = float("inf")
+    lse = torch.randn((1, 2, splits), generator=g)
+    got = split_reduce(part.cuda(), lse.cuda()).cpu()
+    assert got[0, 1, 5] == float("inf") and int(torch.isfinite(got).sum()) == got.numel() - 1
