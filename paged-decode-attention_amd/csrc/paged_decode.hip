@@ -2315,7 +2315,7 @@ hipError_t launch_reduce_w(const ARGS &args, int batch, int num_heads, int d, hi
 template <int KIND, typename ARGS>
 hipError_t launch_reduce(const ARGS &args, int batch, int num_heads, int d, bool wide, hipStream_t st) {
   return wide ? launch_reduce_w<KIND, ARGS, true>(args, batch, num_heads, d, st)
-                            : launch_reduce_w<KIND, ARGS, false>(args, batch, num_heads, d, st);
+              : launch_reduce_w<KIND, ARGS, false>(args, batch, num_heads, d, st);
 }
 
 template <bool WIDE>
@@ -2338,21 +2338,39 @@ hipError_t launch_merge_table(const MergeTable &mt, int d, bool wide, hipStream_
 }
 
 // Whether a merge takes a workgroup of kWideWaves waves per row instead of one
-// wave: one wave holds 8 partials and folds more in a second and third round
-// trip, and the waves' fold costs 0.3 us where one would do. Whole calls,
-// graph-timed at the Llama-3-8B shape, one wave / kWideWaves, in us: classic
-// split B = 4, T = 1024 with 8 splits 8.9 / 9.3, B = 1, T = 2048 with 32 8.2 /
-// 7.9; flat F = 128, B = 64 (fp8, T <= 8192) 40.9 / 41.9, B = 32 T <= 4095
-// 46.7 / 45.8 but T <= 1622 24.3 / 25.6, B = 16 30.9 / 28.8, B = 8 (T <= 2500)
-// 22.1 / 18.3. For the flat
-// split the rule knows only the ranges and the batch, the same with and without
-// host lengths, so that both merges fold alike.
-// Above kWideMaxRows rows the launch of four times the waves costs more: int8, B =
-// 32, T = 16384, 64 heads, F = 256 177.3 / 179.1.
-constexpr int kWideMaxRows = 1024;
-bool wide_splits(int num_splits) { return num_splits > 8; }
+// wave: one wave holds 8 partials and folds more in further round trips, and the
+// waves' fold costs 0.3 us where one would do; with many rows, the launch of four
+// times the waves costs more than the round trips. The most rows for the merge of
+// a flat split, of a classic one and for pa_split_reduce, whose partials are as
+// often in the caches (a launch under 2^32 threads, as well: one wave a row takes
+// four times the rows). Graph-timed, one wave / kWideWaves in us:
+//   pa_split_reduce, head_dim 128: 256 rows of 9 splits 4.01 / 3.12, of 16 3.22 /
+//     3.11, of 64 3.88 / 3.55; 512 of 16 3.36 / 3.48; 1,024 of 16 3.63 / 4.17;
+//     4,096 of 9 5.19 / 8.03; head_dim 64, 1,024 of 64 4.27 / 5.19;
+//   whole calls with a classic split: Llama-3-8B shape B = 1, T = 2048, 16 splits
+//     7.91 / 7.71, B = 16, T ~ U[256, 4096], 12 splits (512 rows) 39.3 / 39.0, B =
+//     70, T = 1024, 9 splits (2,240) 62.0 / 63.9; 14 q / 2 kv heads, D = 64, B = 4,
+//     T ~ U[256, 4096], 16 splits 8.59 / 7.39, B = 70, 9 splits (980) 12.3 / 12.8;
+//     9 splits of which 8 hold tokens (B = 1, T = 2048) 8.44 / 8.74;
+//   flat, Llama-3-8B shape F = 128: B = 8, T ~ U[312, 2500] 19.6 / 15.5, B = 16, T ~
+//     U[750, 6000] 45.4 / 44.2; Llama-3-70B shape B = 16 (1,024 rows), int8, F = 256,
+//     T ~ U[750, 6000] 34.5 / 33.9; int8, B = 32, T = 16384 (2,048 rows) 177.3 / 179.1.
+// For the flat split the rule knows only the ranges and the batch, the same with
+// and without host lengths, so that both merges fold alike.
+constexpr int kWideMaxRowsFlat = 1024, kWideMaxRowsSplit = 512, kWideMaxRowsAlone = 256;
+
+bool wide_reduce(const pa_reduce_args *r) {
+  return r->num_splits > kWideHeld && (int64_t)r->batch * r->num_heads <= kWideMaxRowsAlone;
+}
+
+bool wide_auto(const pa_decode_args *a, const SplitDiv &s) {
+  int pieces = a->num_splits;  // of the longest sequence
+  if (s.chunk_tiles > 0) pieces = std::min(pieces, (a->max_seq_len - 1) / (s.chunk_tiles * kSplitAlign) + 1);
+  return pieces > kWideHeld && (int64_t)a->batch * a->num_q_heads <= kWideMaxRowsSplit;
+}
+
 bool wide_flat(const pa_decode_args *a) {
-  return a->flat_splits >= 8 * (int64_t)a->batch && (int64_t)a->batch * a->num_q_heads <= kWideMaxRows;
+  return a->flat_splits >= 8 * (int64_t)a->batch && (int64_t)a->batch * a->num_q_heads <= kWideMaxRowsFlat;
 }
 
 // The flat split's ranges and merge list from host-side lengths, exactly as
@@ -2610,10 +2628,12 @@ int pa_decode(const pa_decode_args *a, void *stream) {
       e = launch_merge_table(plan.mt, a->head_dim, wide_flat(a), st);
     } else {
       const int hq = a->num_q_heads, d = a->head_dim;
-      e = flat ? launch_reduce<kMergeFlat>(rp, a->batch, hq, d, wide_flat(a), st)
-               : launch_reduce<kMergeAuto>(
-                     AutoMergeArgs{rp, split_div(a->max_seq_len, a->num_splits), make_div(hq)}, a->batch, hq, d,
-                     wide_splits(a->num_splits), st);
+      if (flat) {
+        e = launch_reduce<kMergeFlat>(rp, a->batch, hq, d, wide_flat(a), st);
+      } else {
+        const AutoMergeArgs m = {rp, split_div(a->max_seq_len, a->num_splits), make_div(hq)};
+        e = launch_reduce<kMergeAuto>(m, a->batch, hq, d, wide_auto(a, m.s), st);
+      }
     }
     if (e != hipSuccess) return fail(PA_ERR_HIP, "reduce launch failed: %s", hipGetErrorString(e));
   }
@@ -2825,7 +2845,7 @@ int pa_split_reduce(const pa_reduce_args *r, void *stream) {
   int rc = check_reduce(r, &rp);
   if (rc != PA_OK) return rc;
   if (r->batch == 0) return ok();
-  hipError_t e = launch_reduce<kMergeAll>(rp, r->batch, r->num_heads, r->head_dim, wide_splits(r->num_splits),
+  hipError_t e = launch_reduce<kMergeAll>(rp, r->batch, r->num_heads, r->head_dim, wide_reduce(r),
                                          static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(PA_ERR_HIP, "reduce launch failed: %s", hipGetErrorString(e));
   return ok();

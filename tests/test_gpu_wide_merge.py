@@ -61,3 +61,16 @@ def test_infinity_in_the_last_partial(splits):
     lse = torch.randn((1, 2, splits), generator=g)
     got = split_reduce(part.cuda(), lse.cuda()).cpu()
     assert got[0, 1, 5] == float("inf") and int(torch.isfinite(got).sum()) == got.numel() - 1
+
+
+@pytest.mark.parametrize("batch,heads", [(8, 32), (257, 1), (1 << 19, 32)])
+def test_split_reduce_rows(batch, heads):
+    """The most rows that four waves take, one more, and more rows than a launch of four waves each
+    could hold (2^32 threads): all of them the same row here, its partials by stride 0."""
+    g = torch.Generator().manual_seed(75)
+    part, lse = torch.randn((1, 1, 9, 32), generator=g).cuda(), torch.randn((1, 1, 9), generator=g).cuda()
+    got = split_reduce(part.expand(batch, heads, 9, 32), lse.expand(batch, heads, 9))
+    want = oracle.split_merge(part.cpu(), lse.cpu())
+    # fp32 sums of 9 terms, then fp16: half an ulp of a value up to 4 is 2^-10
+    assert max_abs(got[:1, :1], want) < 2.0 ** -10 + 1e-5
+    assert bool((got == got[0, 0]).all())
