@@ -1806,6 +1806,9 @@ __device__ __forceinline__ void merge_wide(const RParams &p, const float *lse, c
   float M = -INFINITY;
 #pragma unroll
   for (int w = 0; w < kWideWaves; ++w) M = fmaxf(M, sm.m[w]);
+  // (a row of empty partials is zeros, whatever they hold: the one-wave merge
+  // does not read them either, above the kWideHeld that it reads at once)
+  const bool empty = S > kWideHeld && M == -INFINITY;
   wsum = 0.f;
 #pragma unroll
   for (int j = 0; j < kPer; ++j) acc[j] = 0.f;
@@ -1813,7 +1816,7 @@ __device__ __forceinline__ void merge_wide(const RParams &p, const float *lse, c
   for (int w = 0; w < kWideWaves; ++w) {
     const float f = (sm.m[w] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(sm.m[w] - M);
     wsum += f * sm.w[w];
-    if (active) {
+    if (active && !empty) {
 #pragma unroll
       for (int j = 0; j < kPer; ++j) acc[j] += f * sm.acc[w][lane * kPer + j];
     }

@@ -74,3 +74,15 @@ def test_split_reduce_rows(batch, heads):
     # fp32 sums of 9 terms, then fp16: half an ulp of a value up to 4 is 2^-10
     assert max_abs(got[:1, :1], want) < 2.0 ** -10 + 1e-5
     assert bool((got == got[0, 0]).all())
+
+
+@pytest.mark.parametrize("d", [32, 128])
+@pytest.mark.parametrize("splits", [9, 33])
+def test_rows_of_empty_partials_are_zeros(splits, d):
+    """Whatever the unused partials hold (uninitialised memory: NaN here)."""
+    part, lse = torch.full((2, 3, splits, d), float("nan")), torch.full((2, 3, splits), float("-inf"))
+    part[1, 2], lse[1, 2] = 1.5, 0.0
+    got = split_reduce(part.cuda(), lse.cuda())
+    assert bool((got[1, 2] == 1.5).all())
+    got[1, 2] = 0
+    assert bool((got == 0).all())
