@@ -35,6 +35,7 @@ _SCALE_CODE = {torch.float16: _abi.PA_SCALE_FP16, torch.float32: _abi.PA_SCALE_F
 # first step each call copies a struct and sets three pointers.
 _WRITE_TEMPLATES: dict[tuple, tuple] = {}
 _WRITE_TEMPLATES_MAX = 512
+_copy_args = _abi.PaCacheWriteArgs.from_buffer_copy
 
 
 def reshape_and_cache(
@@ -48,19 +49,23 @@ def reshape_and_cache(
     scales are written too. Asynchronous on the current stream.
     """
     k, v, ks, vs = cache.k_cache, cache.v_cache, cache.k_scale, cache.v_scale
-    tkey = (id(k), k.data_ptr(), id(v), v.data_ptr(), id(ks), 0 if ks is None else ks.data_ptr(), id(vs),
-            0 if vs is None else vs.data_ptr(), cache.kv_dtype, cache.block_size, cache.shape.num_kv_heads,
-            cache.shape.head_dim, key.shape, key.stride(), key.dtype, key.get_device(), value.shape,
-            value.stride(), value.dtype, value.get_device(), slot_mapping.shape, slot_mapping.stride(),
-            slot_mapping.dtype, slot_mapping.get_device())
+    shape = cache.shape
+    # (is_contiguous stands for the slots' stride: one dimension)
+    tkey = (id(k), k.data_ptr(), id(v), v.data_ptr(), None if ks is None else (id(ks), ks.data_ptr()),
+            None if vs is None else (id(vs), vs.data_ptr()), cache.kv_dtype, cache.block_size, shape.num_kv_heads,
+            shape.head_dim, key.shape, key.stride(), key.dtype, key.get_device(), value.shape, value.stride(),
+            value.dtype, value.get_device(), slot_mapping.shape, slot_mapping.is_contiguous(), slot_mapping.dtype,
+            slot_mapping.get_device())
     hit = _WRITE_TEMPLATES.get(tkey)
     if hit is not None:
-        r = hit[0]
+        r, tmpl = hit
         if (r[0]() is k and r[1]() is v and (ks is None or r[2]() is ks)
                 and (vs is None or r[3]() is vs)):
-            a = _abi.PaCacheWriteArgs.from_buffer_copy(hit[1])
+            a = _copy_args(tmpl)
             a.key, a.value, a.slot_mapping = key.data_ptr(), value.data_ptr(), slot_mapping.data_ptr()
-            _abi.check(_launch(key, _abi.load().pa_cache_write, a), "pa_cache_write")
+            rc = _launch(key, _abi.load().pa_cache_write, a)
+            if rc:
+                _abi.check(rc, "pa_cache_write")
             return
     a = _pack_write_args(key, value, cache, slot_mapping)
     if len(_WRITE_TEMPLATES) >= _WRITE_TEMPLATES_MAX:

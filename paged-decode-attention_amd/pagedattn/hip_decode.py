@@ -780,6 +780,7 @@ def _ptr(t: torch.Tensor | None) -> int | None:
 # (resize_, set_) is not noticed.
 _ARG_TEMPLATES: dict[tuple, tuple] = {}
 _ARG_TEMPLATES_MAX = 512
+_copy_args = _abi.PaDecodeArgs.from_buffer_copy
 
 
 def _fill_args(
@@ -803,8 +804,8 @@ def _fill_args(
     k, v, bt, sl = cache.k_cache, cache.v_cache, cache.block_table, cache.seq_lens
     ks, vs = cache.k_scale, cache.v_scale
     shape = cache.shape
-    key = (id(k), k.data_ptr(), id(v), v.data_ptr(), id(bt), bt.data_ptr(), id(sl),
-           sl.data_ptr(), id(ks), 0 if ks is None else ks.data_ptr(), id(vs), 0 if vs is None else vs.data_ptr(),
+    key = (id(k), k.data_ptr(), id(v), v.data_ptr(), id(bt), bt.data_ptr(), id(sl), sl.data_ptr(),
+           None if ks is None else (id(ks), ks.data_ptr()), None if vs is None else (id(vs), vs.data_ptr()),
            cache.kv_dtype, cache.block_size, shape.num_q_heads, shape.num_kv_heads, shape.head_dim,
            q.shape, q.stride(), q.dtype, q.get_device(), out.shape, out.stride(), out.dtype,
            out.get_device(), num_splits, sm_scale, max_seq_len, flat_splits, flat_seq_cost,
@@ -818,8 +819,9 @@ def _fill_args(
         hit = hit if (r[0]() is k and r[1]() is v and r[2]() is bt and r[3]() is sl
                       and (ks is None or r[4]() is ks) and (vs is None or r[5]() is vs)) else None
     if hit is not None:
-        host = _host_lens_pointer(seq_lens_host, q.shape[0], num_splits, flat_splits)
-        a = _abi.PaDecodeArgs.from_buffer_copy(hit[1])
+        host = None if seq_lens_host is None else _host_lens_pointer(seq_lens_host, q.shape[0], num_splits,
+                                                                     flat_splits)
+        a = _copy_args(hit[1])
         a.q = q.data_ptr()
         a.out = out.data_ptr()
         if workspace is not None:
@@ -1106,10 +1108,10 @@ def paged_decode_hip(
         splits, flat, cost = unpaired
         return paged_decode_hip(q, cache, out, block_n, splits, sm_scale=sm_scale, max_seq_len=max_seq_len,
                                 flat_splits=flat, flat_seq_cost=cost, seq_lens_host=seq_lens_host)
-    lib = _abi.load()
     # (with host lengths and every sequence inside one range, the library leaves the merge out)
-    rc = _launch(q, lib.pa_decode, args)
-    _abi.check(rc, "pa_decode")
+    rc = _launch(q, _abi.load().pa_decode, args)
+    if rc:
+        _abi.check(rc, "pa_decode")
     return out
 
 

@@ -249,3 +249,17 @@ def test_int8_rows_with_nan_and_infinity(scale_dtype):
     assert torch.equal(c.k_cache[0, [0, 2]].cpu(), want[[0, 2]])
     assert torch.equal(c.k_scale[0, [0, 2]].cpu(), scale[[0, 2]])
     assert bool((c.k_cache[0, 1] == 0).all()) and bool(torch.isinf(c.k_scale[0, 1]).all())
+
+
+def test_argument_cache_tells_strided_slots():
+    """Slots of one shape and another stride are validated again, after a write that was taken."""
+    c = allocate(ModelShape(2, 2, 64, "s"), 1, [64], seed=55, device="cuda", shuffle=False)
+    rows = torch.randn((4, 2, 64), device="cuda").half()
+    wide = torch.arange(8, device="cuda")
+    for _ in range(2):
+        reshape_and_cache(rows, rows, c, wide[:4])
+    with pytest.raises(ValueError, match="contiguous"):
+        reshape_and_cache(rows, rows, c, wide[::2])
+    one = rows[:1]
+    reshape_and_cache(one, one, c, wide[::8])  # one slot: any stride
+    assert torch.equal(c.k_cache.view(-1, 2, 64)[0], rows[0])
