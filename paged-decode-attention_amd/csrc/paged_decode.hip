@@ -1997,7 +1997,14 @@ SplitDiv split_div(int max_seq_len, int num_splits) {
 //   int8, B = 16, T = 32768: 16 splits (256 workgroups) 35.1 / 32.3, 8 splits
 //     (128) 46.3 / 51.6; fp8, B = 8, T = 65536: 32 splits 45.2 / 26.8, 16 (128)
 //     30.0 / 31.3; B = 192 unsplit (192 workgroups) 30.0 / 26.9.
+// Short chunks lose: with at most kPackMinTokens a workgroup (two tiles a wave)
+// the fewer workgroups cost more than the shared instructions save. Unsplit, B =
+// 256, one head / two, in us: T = 16 fp8 0.90 of the time, int8 0.86; T = 100 1.01 /
+// 0.98; T ~ U[10, 160] 1.01 / 0.94; T = 256 1.19 / 1.12 (that many times faster with
+// two). 256 workgroups of chunks of 64 tokens fp8 0.94, int8 0.94; of 128 0.95 /
+// 0.94; of 256 0.99 / 0.97; of 384 1.04 / 0.99; of 512 1.09 / 1.02.
 constexpr int kPackMinWorkgroups = 192;
+constexpr int kPackMinTokens = 256;
 
 bool packs_heads(const pa_decode_args *a, const KParams &k) {
   const bool one_byte = a->kv_dtype == PA_KV_FP8_E5M2 || a->kv_dtype == PA_KV_INT8;
@@ -2012,7 +2019,10 @@ bool packs_heads(const pa_decode_args *a, const KParams &k) {
     if (!aligned(a->k_scale, 4) || !aligned(a->v_scale, 4) || k.sst % 4 != 0 || k.ssn % 4 != 0 || k.sst < pair)
       return false;
   }
-  return (int64_t)a->batch * (k.hkv / 2) * a->num_splits >= kPackMinWorkgroups;
+  // (the longest sequence, as far as the launch knows it)
+  const int longest = a->max_seq_len > 0 ? std::min(a->max_seq_len, k.max_tokens) : k.max_tokens;
+  return longest > (int64_t)kPackMinTokens * a->num_splits &&
+         (int64_t)a->batch * (k.hkv / 2) * a->num_splits >= kPackMinWorkgroups;
 }
 
 // Validates and fills the kernel parameter block. `need_partials` is true when

@@ -159,9 +159,11 @@ UNSPLIT_MAX_SHORT_ROW_BYTES_PER_CU = 192 << 10
 # 27.4, B = 256 int8 31.8 / 44.1.
 PACKED_SPLIT_MAX_RAGGED = 2.25
 # The library takes pairs from this many workgroups of them on, whatever the
-# device (kPackMinWorkgroups in csrc/paged_decode.hip); with fewer, as a small
-# batch on a partition of few CUs has, a launch cut for pairs would run without.
+# device, and for chunks of more tokens than this (kPackMinWorkgroups and
+# kPackMinTokens in csrc/paged_decode.hip); otherwise, as for a small batch on a
+# partition of few CUs, a launch cut for pairs would run without.
 PACKED_MIN_WORKGROUPS = 192
+PACKED_MIN_TOKENS = 256
 # A batch that runs unsplit without pairs is split in two for them from this many
 # tiles on: int8, T = 306, B = 164 10.1 us unsplit, 11.4 in two; T = 1024, B = 128
 # 16.2 and 14.6.
@@ -537,17 +539,17 @@ def packed_splits_for(seq_lens, plan: LaunchPlan, num_kv_heads: int, group: int,
                       kv_dtype: str | None, head_dim: int | None) -> int:
     """Splits of the classic kernel where it takes pairs of heads (`packs_heads`)
     and beats `plan`: the fewest, as a power of two, that give every CU a
-    workgroup, chunks of at least MIN_SPLIT_TILES tiles. 0: `plan` stands (other
+    workgroup, chunks of more than PACKED_MIN_TOKENS tokens. 0: `plan` stands (other
     geometries, unknown lengths, short sequences, a batch with a sequence over
     PACKED_SPLIT_MAX_RAGGED times the mean)."""
     if seq_lens is None or not packs_heads(num_kv_heads, group, head_dim, kv_dtype):
         return 0
     lens = _Lens.of(seq_lens)
     batch, tmax = lens.size, plan.max_seq_len
-    if _tiles(tmax) <= UNSPLIT_MAX_TILES or tmax * batch > PACKED_SPLIT_MAX_RAGGED * lens.total:
+    if tmax <= PACKED_MIN_TOKENS or tmax * batch > PACKED_SPLIT_MAX_RAGGED * lens.total:
         return 0
     pairs, splits = batch * (num_kv_heads // 2), 1
-    while splits * pairs < sm_count and _tiles(tmax) >= 2 * splits * MIN_SPLIT_TILES:
+    while splits * pairs < sm_count and tmax > 2 * splits * PACKED_MIN_TOKENS:
         splits *= 2
     if pairs * splits < PACKED_MIN_WORKGROUPS:
         return 0

@@ -18,11 +18,11 @@ def decode_args(batch, hq, hkv, kv, d=64, splits=1, **over):
     a = _abi.PaDecodeArgs()
     a.q = a.k_cache = a.v_cache = a.out = a.block_table = a.seq_lens = a.part_out = a.part_lse = FAKE
     a.batch, a.num_q_heads, a.num_kv_heads, a.head_dim = batch, hq, hkv, d
-    a.block_size, a.num_blocks, a.max_blocks, a.num_splits = 16, 64, 8, splits
+    a.block_size, a.num_blocks, a.max_blocks, a.num_splits = 16, 64, 64, splits
     a.stride_qb, a.stride_qh = hq * d, d
     a.stride_kn, a.stride_kt, a.stride_kh = 16 * hkv * d, hkv * d, d
     a.stride_ob, a.stride_oh = hq * d, d
-    a.stride_btb = 8
+    a.stride_btb = 64
     a.kv_dtype = {"fp16": _abi.PA_KV_FP16, "bf16": _abi.PA_KV_BF16, "fp8_e5m2": _abi.PA_KV_FP8_E5M2,
                   "int8": _abi.PA_KV_INT8}[kv]
     a.scale_dtype = _abi.PA_SCALE_NONE
@@ -54,7 +54,9 @@ def test_plans_for_pairs_get_pairs(cus):
         plan = plan_launch(batch, 0, hkv, group, cus, 2, kv_dtype=kv, head_dim=64, seq_lens=lens)
         if plan.packed_splits:
             packed += 1
-            assert pairs(decode_args(batch, hkv * group, hkv, kv, splits=plan.packed_splits)), (batch, hi, plan)
+            a = decode_args(batch, hkv * group, hkv, kv, splits=plan.packed_splits, max_seq_len=plan.max_seq_len,
+                            max_blocks=-(-max(lens) // 16))
+            assert pairs(a), (batch, hi, plan)
     assert packed > 100
 
 
@@ -64,6 +66,12 @@ def test_library_rule_for_pairs():
     # one workgroup of pairs fewer than the library's least, counted over the splits
     assert not pairs(decode_args(191, 14, 2, "int8"))
     assert pairs(decode_args(64, 14, 2, "int8", splits=3)) and not pairs(decode_args(64, 14, 2, "int8", splits=2))
+    # chunks of more than 256 tokens, of the longest sequence or of the block table's room for one
+    assert pairs(decode_args(192, 14, 2, "int8", max_seq_len=257)) and not pairs(decode_args(192, 14, 2, "int8", max_seq_len=256))
+    assert pairs(decode_args(64, 14, 2, "int8", splits=3, max_seq_len=769))
+    assert not pairs(decode_args(64, 14, 2, "int8", splits=3, max_seq_len=768))
+    assert pairs(decode_args(192, 14, 2, "int8", max_blocks=17)) and not pairs(decode_args(192, 14, 2, "int8", max_blocks=16))
+    assert not pairs(decode_args(192, 14, 2, "int8", max_blocks=16, max_seq_len=9999))
     # types, head dims, head counts and groups
     assert pairs(decode_args(192, 14, 2, "fp8_e5m2")) and not pairs(decode_args(192, 14, 2, "fp16"))
     assert not pairs(decode_args(192, 14, 2, "int8", d=128)) and not pairs(decode_args(192, 14, 2, "int8", d=32))

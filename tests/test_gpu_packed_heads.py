@@ -156,3 +156,79 @@ def test_launch_of_a_cache_that_does_not_pair(monkeypatch, form, entry):
     rows = [0, 100, 255]
     ref = oracle.reference_decode(q[rows].cpu(), subset_cache(c, rows), out_dtype=torch.float32)
     assert max_abs(got[rows], ref) < 2e-3
+
+
+def _wide_table(c, tokens=512):
+    """The same sequences under a block table for `tokens` tokens: room for lengths that pair."""
+    bt = torch.zeros((c.block_table.shape[0], tokens // c.block_size), dtype=torch.int32, device="cuda")
+    bt[:, :c.block_table.shape[1]] = c.block_table
+    return dataclasses.replace(c, block_table=bt)
+
+
+def _launch_pairs(monkeypatch):
+    """Whether each launch from here on took pairs."""
+    from pagedattn import hip_decode
+
+    took, real = [], hip_decode._launch
+    monkeypatch.setattr(hip_decode, "_launch", lambda t, fn, a: took.append(hip_decode._takes_pairs(a)) or real(t, fn, a))
+    return took
+
+
+@pytest.mark.parametrize("q_dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kv_dtype,scale_dtype", KV)
+@pytest.mark.parametrize("hq,hkv,splits,page", [
+    (14, 2, 1, 16),
+    (14, 2, 3, 32),
+    (16, 2, 2, 16),
+    (4, 4, 1, 64),
+    (24, 4, 9, 16),   # folded by four waves a row
+])
+def test_pairs_of_long_chunks(monkeypatch, kv_dtype, scale_dtype, q_dtype, hq, hkv, splits, page):
+    """At the smallest batch and chunk that pair, with sequences longer than max_seq_len among them
+    (split by their own lengths), against the oracle and against single heads."""
+    took = _launch_pairs(monkeypatch)
+    batch, told = -(-192 // (hkv // 2 * splits)), 256 * splits + 1
+    g = torch.Generator().manual_seed(68)
+    lens = torch.randint(1, told + 1, (batch,), generator=g).tolist()
+    lens[:6] = [1, 33, 0, told, told + 300, 2 * told]
+    c = _cache(hq, hkv, lens, kv_dtype, scale_dtype, page)
+    q = seeded_q(batch, hq, 64, 69, device="cuda").to(q_dtype)
+    q[:, ::3] *= 3
+    kw = {"num_splits": splits, "max_seq_len": told}
+    got = paged_decode_hip(q, c, **kw)
+    one = paged_decode_hip(q, c, **dict(kw, max_seq_len=told - 1))  # a token less: every head by itself
+    assert took == [True, False]
+    want = oracle.reference_decode(q, c, out_dtype=torch.float32)
+    want[2] = 0
+    # 2e-3 in fp16; a bf16 result is rounded to 8 bits, half an ulp of a value up to 8 is 2^-6
+    tol = 2e-3 if q_dtype == torch.float16 else 2.0 ** -6 + 2e-3
+    assert max_abs(got, want) < tol and max_abs(got, one) < 2 * tol
+    assert torch.equal(paged_decode_hip(q, c, **kw), got)
+
+
+@pytest.mark.parametrize("kv_dtype,scale_dtype", KV)
+def test_paired_one_token_rows_are_the_dequantised_v_rows(monkeypatch, kv_dtype, scale_dtype):
+    from pagedattn import dequantize_kv
+
+    took = _launch_pairs(monkeypatch)
+    c = _wide_table(_cache(14, 2, [1] * 200, kv_dtype, scale_dtype))
+    out = paged_decode_hip(seeded_q(200, 14, 64, 64, device="cuda"), c, num_splits=1)
+    first = c.block_table[:, 0].long()
+    rows = c.v_cache.view(torch.uint8)[first, 0].view(c.v_cache.dtype)
+    v = dequantize_kv(rows, None if c.v_scale is None else c.v_scale[first, 0], kv_dtype)
+    assert took == [True] and torch.equal(out, v.repeat_interleave(7, dim=1))
+
+
+@pytest.mark.parametrize("what", ["k", "v"])
+def test_infinities_of_one_paired_head_stay_in_it(monkeypatch, what):
+    took = _launch_pairs(monkeypatch)
+    c = _wide_table(_cache(14, 2, [50] * 192, "fp8_e5m2", None))
+    q = seeded_q(192, 14, 64, 65, device="cuda")
+    clean = paged_decode_hip(q, c, num_splits=1)
+    store = (c.k_cache if what == "k" else c.v_cache).view(torch.uint8)
+    store[c.block_table[3, 1].long(), 2, 0, 5] = 0x7C  # +inf, head 0, sequence 3
+    got = paged_decode_hip(q, c, num_splits=1)
+    assert took == [True, True]
+    assert torch.equal(got[:, 7:], clean[:, 7:])
+    assert torch.equal(got[:3], clean[:3]) and torch.equal(got[4:], clean[4:])
+    assert not bool(torch.isfinite(got[3, :7]).all())
