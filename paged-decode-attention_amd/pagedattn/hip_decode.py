@@ -146,17 +146,30 @@ UNSPLIT_MAX_KV_BYTES_PER_CU = {"fp16": 2 << 20, "bf16": 2 << 20, "fp8_e5m2": 768
 UNSPLIT_MIN_ROW_BYTES = 128
 UNSPLIT_MAX_SHORT_ROW_BYTES_PER_CU = 192 << 10
 # The classic kernel takes two 64-element kv heads of a 1-byte cache as one row
-# of 128 (`packs_heads`), and then streams such rows faster than the flat split,
-# unsplit or cut into the splits that give every CU a workgroup (rounded up to a
-# power of two), unless one sequence is far longer than the others: up to
-# PACKED_SPLIT_MAX_RAGGED times the mean. Graph-timed at the Qwen2.5-0.5B shape
-# (256 CUs), flat (the better of F = 512 and 1024) / this rule in us: T ~ U[128,
-# 2047] B = 256 fp8 27.1 / 17.6, int8 33.2 / 27.2; T ~ U[200, 3000] B = 96 fp8
-# 22.0 / 16.3, int8 28.7 / 20.4 (4 splits); T ~ U[1000, 16000] B = 32 fp8 23.9 /
-# 18.8 (8 splits), int8 27.8 / 29.0; T = 4096 B = 256 fp8 56.4 / 45.6, int8 71.7
-# / 54.9; T ~ U[64, 1024] B = 1024 int8 69.4 / 37.8. With lengths log-uniform
-# over a factor of 64 (longest 4 times the mean) flat wins: B = 32 fp8 21.3 /
+# of 128 (`packs_heads`) and then streams such rows faster than the flat split,
+# but waits for the CU with the most to do: unsplit, or cut into the splits that
+# give every CU a workgroup (rounded up to a power of two), it is taken where
+#   * the workgroups are many (PACKED_MANY_WORKGROUPS a CU; more where a token's
+#     row is wide, which the flat split streams better), or the longest chunk's
+#     tiles are at most a times the tiles of pairs that a CU gets, and c
+#     (PACKED_SHARE = a, c; PACKED_SHARE_ONE_EACH with no more workgroups than CUs),
+#     less PACKED_MERGE_TILES for the merge of a split launch, and
+#   * no sequence is longer than PACKED_SPLIT_MAX_RAGGED times the mean.
+# Eager whole calls on 4,900 random batches that ran flat without pairs (1 to 700
+# sequences of up to 100,000 tokens, 256 CUs): where the rule takes pairs they are
+# 1.23 times as fast for int8, 1.16 for fp8 (geometric means; the worst 0.91 and
+# 0.92), elsewhere 0.86 and 0.89. Flat / pairs at 14 q / 2 kv heads in us: taken, int8
+# B = 192, T = 2047 (2 splits) 30.8 / 26.3, B = 256, T ~ U[128, 2047] 27.5 / 24.5; left,
+# int8 B = 192, T ~ U[128, 8000] (2 splits) 56.8 / 65.1, B = 160, T ~ U[128, 2047] 22.1 /
+# 22.9, fp8 B = 129, T ~ U[2100, 33660] (2 splits) 105.7 / 175.9. With lengths log-
+# uniform over a factor of 64 (longest 4 times the mean) flat wins: B = 32 fp8 21.3 /
 # 27.4, B = 256 int8 31.8 / 44.1.
+PACKED_MANY_WORKGROUPS = 2.0
+PACKED_MANY_WORKGROUPS_WIDE = 2.75
+PACKED_WIDE_ROW_BYTES = {"fp8_e5m2": 512}
+PACKED_SHARE = {"fp8_e5m2": (0.6, 21), "int8": (0.9, 24)}
+PACKED_SHARE_ONE_EACH = {"fp8_e5m2": (1.1, 30), "int8": (1.1, 39)}
+PACKED_MERGE_TILES = {"fp8_e5m2": 18, "int8": 27}
 PACKED_SPLIT_MAX_RAGGED = 2.25
 # The library takes pairs from this many workgroups of them on, whatever the
 # device, and for chunks of more tokens than this (kPackMinWorkgroups and
@@ -164,10 +177,11 @@ PACKED_SPLIT_MAX_RAGGED = 2.25
 # partition of few CUs, a launch cut for pairs would run without.
 PACKED_MIN_WORKGROUPS = 192
 PACKED_MIN_TOKENS = 256
-# A batch that runs unsplit without pairs is split in two for them from this many
-# tiles on: int8, T = 306, B = 164 10.1 us unsplit, 11.4 in two; T = 1024, B = 128
-# 16.2 and 14.6.
-PACKED_SPLIT_MIN_TILES = 24
+# A batch that runs unsplit and has too few workgroups for pairs is cut in two for
+# them from this many tiles on, unsplit / in two: int8 B = 170, T <= 852 0.95 of the
+# time, B = 172, T <= 955 1.16; 30 batches from here on 1.15 (the worst 0.97), 30
+# below it (from 24 tiles) 1.01 (0.80).
+PACKED_SPLIT_MIN_TILES = 30
 # Batches of short sequences that fill the CUs run unsplit, whatever their
 # size and merge or not: the flat split loses there, because its waves
 # switch sequences every few tiles. Per KV type, the longest sequence of a
@@ -538,24 +552,32 @@ def ordered_batch_runs_unsplit(seq_lens, num_kv_heads: int, group: int, sm_count
 def packed_splits_for(seq_lens, plan: LaunchPlan, num_kv_heads: int, group: int, sm_count: int,
                       kv_dtype: str | None, head_dim: int | None) -> int:
     """Splits of the classic kernel where it takes pairs of heads (`packs_heads`)
-    and beats `plan`: the fewest, as a power of two, that give every CU a
-    workgroup, chunks of more than PACKED_MIN_TOKENS tokens. 0: `plan` stands (other
-    geometries, unknown lengths, short sequences, a batch with a sequence over
-    PACKED_SPLIT_MAX_RAGGED times the mean)."""
+    and beats `plan`. Instead of a flat split: the fewest, as a power of two, that
+    give every CU a workgroup, chunks of more than PACKED_MIN_TOKENS tokens, where
+    the rule at PACKED_SHARE says so. Instead of an unsplit launch with too few
+    workgroups for pairs: two. 0: `plan` stands (also for other geometries and
+    unknown lengths)."""
     if seq_lens is None or not packs_heads(num_kv_heads, group, head_dim, kv_dtype):
         return 0
-    lens = _Lens.of(seq_lens)
-    batch, tmax = lens.size, plan.max_seq_len
-    if tmax <= PACKED_MIN_TOKENS or tmax * batch > PACKED_SPLIT_MAX_RAGGED * lens.total:
+    lens, cus, tmax = _Lens.of(seq_lens), max(1, sm_count), plan.max_seq_len
+    pairs, splits = lens.size * (num_kv_heads // 2), 1
+    if tmax <= PACKED_MIN_TOKENS or tmax * lens.size > PACKED_SPLIT_MAX_RAGGED * lens.total:
         return 0
-    pairs, splits = batch * (num_kv_heads // 2), 1
-    while splits * pairs < sm_count and tmax > 2 * splits * PACKED_MIN_TOKENS:
+    if plan.flat_splits == 0:
+        if plan.num_splits > 1 or pairs >= PACKED_MIN_WORKGROUPS or 2 * pairs < max(cus, PACKED_MIN_WORKGROUPS):
+            return 0
+        return 2 if _tiles(tmax) >= PACKED_SPLIT_MIN_TILES else 0
+    while splits * pairs < cus and tmax > 2 * splits * PACKED_MIN_TOKENS:
         splits *= 2
-    if pairs * splits < PACKED_MIN_WORKGROUPS:
+    if splits * pairs < PACKED_MIN_WORKGROUPS or splits > _abi.PA_MAX_SPLITS:
         return 0
-    if plan.flat_splits == 0 and splits > 1 and (splits > 2 or _tiles(tmax) < PACKED_SPLIT_MIN_TILES):
-        return 0  # classic already: more splits, or a merge over short sequences, cost more than pairs save
-    return min(splits, _abi.PA_MAX_SPLITS)
+    wide = num_kv_heads * head_dim >= PACKED_WIDE_ROW_BYTES.get(kv_dtype, 1 << 30)
+    if splits * pairs <= (PACKED_MANY_WORKGROUPS_WIDE if wide else PACKED_MANY_WORKGROUPS) * cus:
+        share, more = (PACKED_SHARE_ONE_EACH if splits * pairs <= cus else PACKED_SHARE)[kv_dtype]
+        most = share * lens.tiles * (num_kv_heads // 2) / cus + more
+        if -(-_tiles(tmax) // splits) > most - (PACKED_MERGE_TILES[kv_dtype] if splits > 1 else 0):
+            return 0
+    return splits
 
 
 def _plan_launch(batch, max_seq_len, num_kv_heads, group, sm_count, waves_per_simd, kv_dtype, head_dim,

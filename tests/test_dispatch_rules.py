@@ -9,6 +9,13 @@ import random
 import pytest
 
 from pagedattn import _abi, plan_launch
+from pagedattn.hip_decode import (
+    PACKED_MERGE_TILES,
+    PACKED_SHARE,
+    PACKED_SHARE_ONE_EACH,
+    PACKED_SPLIT_MAX_RAGGED,
+    PACKED_SPLIT_MIN_TILES,
+)
 
 FAKE = 0x10000  # 16-byte aligned, never dereferenced
 
@@ -102,3 +109,47 @@ def test_plans_for_pairs_carry_the_launch_without_them():
     # the same launch either way: nothing to carry
     short = plan_launch(512, 0, 2, 7, 256, 2, kv_dtype="int8", head_dim=64, seq_lens=[320] * 512)
     assert short.flat_splits == 0 and short.num_splits == 1 and "unpaired" not in short.launch_kwargs()
+
+
+def packed(lens, kv="int8", hkv=2, cus=256):
+    return plan_launch(len(lens), 0, hkv, 7, cus, 2, kv_dtype=kv, head_dim=64, seq_lens=lens).packed_splits
+
+
+@pytest.mark.parametrize("kv,batch,splits,others", [
+    ("int8", 274, 1, 100), ("int8", 180, 2, 120), ("int8", 128, 2, 200), ("int8", 256, 1, 200),
+    ("fp8_e5m2", 274, 1, 30), ("fp8_e5m2", 240, 2, 80), ("fp8_e5m2", 64, 4, 400), ("fp8_e5m2", 256, 1, 100)])
+def test_pairs_instead_of_flat(kv, batch, splits, others):
+    """Few workgroups: taken while the longest chunk is within its share, on both sides of the line."""
+    share, more = (PACKED_SHARE_ONE_EACH if batch * splits <= 256 else PACKED_SHARE)[kv]
+    seen = set()
+    for longest in range(others, 2 * others + 1):
+        lens = [32 * longest] + [32 * others] * (batch - 1)
+        most = share * (longest + (batch - 1) * others) / 256 + more - (PACKED_MERGE_TILES[kv] if splits > 1 else 0)
+        fits = -(-longest // splits) <= most
+        assert packed(lens, kv) == (splits if fits else 0), longest
+        seen.add(fits)
+    assert seen == {True, False}
+
+
+def test_pairs_limits():
+    # many workgroups are taken up to PACKED_SPLIT_MAX_RAGGED times the mean, whatever the share
+    n = 1000
+    lens = [32 * 225] + [32 * 100] * (n - 1)
+    for i in range(1, 126):
+        lens[i] -= 32  # mean 100 tiles
+    assert PACKED_SPLIT_MAX_RAGGED == 2.25 and max(lens) * n == 2.25 * sum(lens)
+    assert packed(lens) == packed(lens, "fp8_e5m2") == 1
+    lens[1] -= 1
+    assert packed(lens) == packed(lens, "fp8_e5m2") == 0
+    assert packed([32 * 220] + [32 * 100] * 512) == 1
+    assert packed([32 * 220] + [32 * 100] * 511) == 0  # one fewer: the share's rule
+    # more of them where a token's row is wide in fp8 (700 and 712 workgroups of 8 heads)
+    assert packed([32 * 200] + [32 * 100] * 174, "fp8_e5m2", 8) == 0
+    assert packed([32 * 200] + [32 * 100] * 177, "fp8_e5m2", 8) == 1
+    assert packed([32 * 200] + [32 * 100] * 174, "int8", 8) == 1
+    # 1-byte types only; the fewest splits, as a power of two, that give every CU a workgroup of pairs
+    assert packed([8192] * 256, "fp16") == packed([8192] * 256, "bf16") == 0
+    assert [packed([8192] * b) for b in (256, 250, 128, 120, 64, 60)] == [1, 2, 2, 4, 4, 8]
+    # an unsplit launch with too few workgroups for pairs is cut in two from PACKED_SPLIT_MIN_TILES on
+    t = 32 * PACKED_SPLIT_MIN_TILES
+    assert packed([t] * 132) == 2 and packed([t - 32] * 132) == 0 and packed([t] * 127) == 0 and packed([t] * 192) == 0
