@@ -112,6 +112,16 @@ CLASSIC_MARGIN_TILES = {"fp16": 8, "bf16": 8, "fp8_e5m2": 10, "int8": 17}
 UNSPLIT_MARGIN_TILES = {"fp16": 14, "bf16": 14, "fp8_e5m2": 16, "int8": 17}
 CLASSIC_MAX_CHUNK_TILES = {"fp16": 24, "bf16": 24, "fp8_e5m2": 32, "int8": 40}
 UNSPLIT_MAX_CHUNK_TILES = {"fp16": 32, "bf16": 32, "fp8_e5m2": 32, "int8": 40}
+# A batch with too little work for the flat split takes few_splits unless it is known
+# to be so ragged that the longest chunk is over FEW_SPLIT_SHARE times the tiles of
+# a CU, and FEW_SPLIT_SHARE_TILES: then more splits, as plan_num_splits cuts it,
+# spread its long sequences. Eager whole calls, plan_num_splits / few_splits in us:
+# int8, 8 q / 8 kv heads, B = 19, T log-uniform to 4320 34.0 (4) / 48.2 (1); Llama-3-8B
+# shape fp16 B = 20, T log-uniform to 2176 22.7 (3) / 27.7 (1), int8 B = 9, to 14816
+# 41.0 (8) / 56.2 (3). On 3,589 such random batches, few_splits always: 1.052 times as
+# fast (geometric mean; 122 lose over 5%, the worst half); by this rule 1.045 (11; 0.92).
+FEW_SPLIT_SHARE = 2.5
+FEW_SPLIT_SHARE_TILES = 2
 # few_splits: no more than this many while each holds less than
 # FEW_SPLIT_LONG_TILES (14 q / 2 kv heads, D = 64, fp16: B = 2, T = 4096 32 splits
 # 7.8, 64 8.8; T = 16384 10.0, 10.5; B = 1, T = 32768 64 splits 11.7, 32 12.6, 128
@@ -502,8 +512,9 @@ def plan_launch(batch: int, max_seq_len: int, num_kv_heads: int, group: int, sm_
     which holds the lengths on the device only), and the planner assumes
     a ragged batch whose every sequence may be that long. Rules, in order:
       * with `kv_dtype` given and at most one unsplit workgroup per CU: the
-        classic kernel with `few_splits` splits, unless the flat split is the
-        better one (the rule at CLASSIC_STREAM_LOSS);
+        classic kernel with `few_splits` splits, unless the flat split or more
+        splits are the better choice (the rules at CLASSIC_STREAM_LOSS and
+        FEW_SPLIT_SHARE);
       * the flat split (one round of waves, `flat_splits_for`) when each of
         its waves gets at least MIN_FLAT_TILES_PER_WAVE tiles, the batch is
         at most FLAT_MAX_BATCH and is not a single sequence of up to
@@ -603,8 +614,12 @@ def _plan_launch(batch, max_seq_len, num_kv_heads, group, sm_count, waves_per_si
             classic = (1 + CLASSIC_STREAM_LOSS) * chunk <= tiles * units / cus + margin
         else:
             classic = chunk <= (UNSPLIT_MAX_CHUNK_TILES if splits == 1 else CLASSIC_MAX_CHUNK_TILES)[kv_dtype]
-        # (pairs of heads with known lengths: packed_splits_for chooses)
-        if not flat_ok or (classic and not (known and packs_heads(num_kv_heads, group, head_dim, kv_dtype))):
+        if not flat_ok:  # the other choice is plan_num_splits, below
+            classic = (not known or _nearly_uniform(lens)
+                       or chunk <= FEW_SPLIT_SHARE * tiles * units / cus + FEW_SPLIT_SHARE_TILES)
+        elif known and packs_heads(num_kv_heads, group, head_dim, kv_dtype):
+            classic = False  # packed_splits_for chooses between the flat split and pairs
+        if classic:
             return LaunchPlan(splits, tmax, 0)
     if flat_ok:
         fills = known and _fills_unsplit(lens, num_kv_heads, group, cus)

@@ -10,11 +10,24 @@ import pytest
 
 from pagedattn import _abi, plan_launch
 from pagedattn.hip_decode import (
+    CLASSIC_MARGIN_TILES,
+    CLASSIC_MAX_CHUNK_TILES,
+    CLASSIC_STREAM_LOSS,
+    FEW_SPLIT_LONG_TILES,
+    FEW_SPLIT_SHARE,
+    FEW_SPLIT_SHARE_TILES,
+    FEW_SPLITS_MAX,
+    MIN_SPLIT_TILES,
     PACKED_MERGE_TILES,
     PACKED_SHARE,
     PACKED_SHARE_ONE_EACH,
     PACKED_SPLIT_MAX_RAGGED,
     PACKED_SPLIT_MIN_TILES,
+    UNSPLIT_MARGIN_TILES,
+    UNSPLIT_MAX_CHUNK_TILES,
+    UNSPLIT_MAX_TILES,
+    few_splits,
+    plan_num_splits,
 )
 
 FAKE = 0x10000  # 16-byte aligned, never dereferenced
@@ -153,3 +166,74 @@ def test_pairs_limits():
     # an unsplit launch with too few workgroups for pairs is cut in two from PACKED_SPLIT_MIN_TILES on
     t = 32 * PACKED_SPLIT_MIN_TILES
     assert packed([t] * 132) == 2 and packed([t - 32] * 132) == 0 and packed([t] * 127) == 0 and packed([t] * 192) == 0
+
+
+def classic(lens, kv, hkv, group, head_dim, known=True, cus=256):
+    """Splits of the classic kernel in the batch's plan, 0 where it is flat."""
+    p = plan_launch(len(lens), max(lens), hkv, group, cus, 2, kv_dtype=kv, head_dim=head_dim,
+                    seq_lens=lens if known else None)
+    return 0 if p.flat_splits else p.num_splits
+
+
+def test_few_splits_keep_one_workgroup_a_cu():
+    for batch, want in ((1, 32), (2, 16), (3, 10), (4, 8), (5, 6), (31, 1), (32, 1)):
+        assert few_splits(batch, 16384, 8, 4, 256) == want
+    # 16 heads a group are one tile, 17 are two
+    assert few_splits(4, 16384, 8, 16, 256) == 8 and few_splits(4, 16384, 8, 17, 256) == 4
+    # short sequences stay whole; from there chunks of MIN_SPLIT_TILES tiles at least
+    whole = 32 * UNSPLIT_MAX_TILES
+    assert few_splits(1, whole, 2, 7, 256) == 1
+    assert few_splits(1, whole + 1, 2, 7, 256) == (UNSPLIT_MAX_TILES + 1) // MIN_SPLIT_TILES
+    # FEW_SPLITS_MAX until each holds FEW_SPLIT_LONG_TILES tiles
+    long = 32 * FEW_SPLITS_MAX * FEW_SPLIT_LONG_TILES
+    assert few_splits(1, long, 2, 7, 256) == FEW_SPLITS_MAX
+    assert few_splits(1, long + 32 * FEW_SPLIT_LONG_TILES, 2, 7, 256) == FEW_SPLITS_MAX + 1
+    assert few_splits(1, 1 << 30, 1, 1, 1 << 20) == _abi.PA_MAX_SPLITS
+    # more workgroups than CUs already
+    assert few_splits(300, 16384, 8, 4, 256) == 1
+
+
+@pytest.mark.parametrize("kv,hkv,group", [("fp16", 8, 4), ("bf16", 8, 4), ("fp8_e5m2", 8, 4), ("int8", 8, 8)])
+def test_few_split_batches_without_lengths(kv, hkv, group):
+    """Uniform or unknown lengths: classic while the longest chunk is within its limit."""
+    for batch, splits, most in ((8, 4, CLASSIC_MAX_CHUNK_TILES[kv]), (32, 1, UNSPLIT_MAX_CHUNK_TILES[kv])):
+        fits = 32 * splits * most
+        for known in (False, True):
+            assert classic([fits] * batch, kv, hkv, group, 128, known) == splits
+            if splits > 1 or not known:  # (above it, known uniform lengths have rules of their own)
+                assert classic([fits + 1] * batch, kv, hkv, group, 128, known) == 0
+    # one workgroup more than CUs: the rule does not apply
+    assert classic([32 * UNSPLIT_MAX_CHUNK_TILES[kv]] * 33, kv, hkv, group, 128, False) == 0
+
+
+@pytest.mark.parametrize("kv,hkv,group", [("fp16", 8, 4), ("bf16", 8, 4), ("fp8_e5m2", 8, 4), ("int8", 8, 8)])
+def test_few_split_ragged_batches(kv, hkv, group):
+    """Known ragged lengths: classic while the longest chunk, CLASSIC_STREAM_LOSS slower, is within the
+    margin over the tiles that the flat split gives a CU."""
+    seen = set()
+    rest = (140, 33) if kv == "int8" else (80, 20)  # tiles of the others: enough work for the flat split
+    for batch, splits, margin, tiles in ((8, 4, CLASSIC_MARGIN_TILES[kv], rest[0]),
+                                         (32, 1, UNSPLIT_MARGIN_TILES[kv], rest[1])):
+        for longest in range(tiles, 3 * tiles):
+            lens = [32 * longest] + [32 * tiles] * (batch - 1)
+            if max(lens) <= 1.25 * sum(lens) / batch:
+                continue  # nearly uniform
+            a_cu = (longest + (batch - 1) * tiles) * 8 / 256
+            want = splits if (1 + CLASSIC_STREAM_LOSS) * -(-longest // splits) <= a_cu + margin else 0
+            assert classic(lens, kv, hkv, group, 128) == want, longest
+            seen.add((splits, want))
+    assert seen == {(4, 4), (4, 0), (1, 1), (1, 0)}
+
+
+def test_batches_with_little_work():
+    """Too little for the flat split: few_splits, or the splits of plan_num_splits where the longest chunk
+    is known to be far over a CU's share; without lengths few_splits."""
+    seen = set()
+    for longest in range(9, 200):
+        lens = [32 * longest] + [32 * 5] * 19  # 160 workgroups unsplit, under 512 tiles
+        fits = longest <= FEW_SPLIT_SHARE * (longest + 95) * 8 / 256 + FEW_SPLIT_SHARE_TILES
+        want = few_splits(20, max(lens), 8, 4, 256) if fits else plan_num_splits(lens, 8, 4, 256)[0]
+        assert classic(lens, "fp16", 8, 4, 128) == want, longest
+        seen.add((fits, want))
+    assert seen >= {(True, 1), (False, 2), (False, 3)}
+    assert classic([32 * 25] * 20, "fp16", 8, 4, 128, False) == few_splits(20, 800, 8, 4, 256) == 1
