@@ -236,19 +236,29 @@ WIDE_GROUP_MIN = 7
 FLAT_MAX_BATCH = 1024
 
 # A ragged batch whose lengths the call itself reads (num_splits=None) runs
-# unsplit with its longest sequences first, instead of flat, from this much work
-# on: tiles per CU over the longest sequence's tiles (no CU then waits for one
-# sequence, and no wave switches sequences every few tiles).
-# ORDERED_MIN_ROUNDS_SHORT_ROWS: 2-byte KV at head_dim 64, whose flat split has
-# four times the ranges to merge. Eager whole calls, ordered / flat with host
-# tables in us, and the ratio: Llama-3-70B shape fp16 B = 160, T ~ U[32, 1023]
-# 59.4 / 64.8 (2.7), int8 B = 200, T ~ U[100, 1000] 47.3 / 51.0 (3.4), B = 96, T ~
-# U[64, 1500] 40.8 / 38.8 (1.6); Llama-3-8B shape fp16 B = 128, T ~ U[200, 3000]
-# 145.3 / 140.0 (2.3), bf16 B = 256, T log-uniform 16..1024 51.4 / 49.5 (2.0), fp8
-# B = 200, T ~ U[64, 1200] 48.6 / 46.4 (3.2); 14 q / 2 kv heads, D = 64, fp16 B =
-# 300, T ~ U[64, 1500] 24.1 / 28.2 (1.2), B = 512, T ~ U[32, 800] 21.9 / 32.0 (2.2).
-ORDERED_MIN_ROUNDS = {"fp16": 2.5, "bf16": 2.5, "int8": 3.0}
+# unsplit with its longest sequences first, instead of flat, where no CU then waits
+# for one sequence and no wave switches sequences every few tiles: 2-byte KV only,
+# from ORDERED_MIN_ROUNDS times the longest sequence's tiles a CU on, with
+# ORDERED_MIN_GROUP q heads a kv head or more and ORDERED_KV_BYTES_PER_CU of K/V.
+# Rows of 128 bytes (head_dim 64), whose flat split has four times the ranges to
+# merge: from ORDERED_MIN_ROUNDS_SHORT_ROWS on up to ORDERED_SHORT_ROWS_BYTES_PER_CU,
+# beyond that from ORDERED_MIN_ROUNDS_SHORT_ROWS_LARGE.
+# Eager calls of 2,091 random batches with host lengths (256 CUs), flat / ordered: the
+# rule's batches at head_dim 128 and 256 1.05 times as fast, the worst 0.93;
+# outside it 8 q heads a kv head under 250 KB a CU 0.96, 4 under 500 KB 0.95 and over 2
+# MB 0.99, 1 head 0.95; int8 0.85 (the worst 0.44), at any length; head_dim 64 1.15 to
+# 2.0, over 1.5 MB and under 2 rounds 0.97. In us: Llama-3-70B shape fp16 B = 160, T ~
+# U[32, 1023] 64.8 / 59.4; 14 q / 2 kv heads, D = 64, fp16 B = 300, T ~ U[64, 1500]
+# 28.2 / 24.1, B = 512, T ~ U[32, 800] 32.0 / 21.9.
+ORDERED_MIN_ROUNDS = 2.5
+ORDERED_MIN_GROUP = 4
+ORDERED_KV_BYTES_PER_CU = (512 << 10, 2 << 20)
 ORDERED_MIN_ROUNDS_SHORT_ROWS = 1.0
+ORDERED_MIN_ROUNDS_SHORT_ROWS_LARGE = 2.0
+ORDERED_SHORT_ROWS_BYTES_PER_CU = 1536 << 10
+# The library orders launches of more workgroups than this, whatever the device
+# (kOrderMinWorkgroups in csrc/paged_decode.hip), and batches up to this.
+ORDERED_MIN_WORKGROUPS = 512
 ORDERED_MAX_BATCH = 1024
 
 _KV_CODE = {"fp16": _abi.PA_KV_FP16, "fp8_e5m2": _abi.PA_KV_FP8_E5M2, "int8": _abi.PA_KV_INT8,
@@ -547,17 +557,22 @@ def plan_launch(batch: int, max_seq_len: int, num_kv_heads: int, group: int, sm_
 def ordered_batch_runs_unsplit(seq_lens, num_kv_heads: int, group: int, sm_count: int, kv_dtype: str | None,
                                head_dim: int | None) -> bool:
     """Whether a batch with known lengths runs faster unsplit, its longest
-    sequences first, than flat: ragged, more workgroups than two a CU, and
-    ORDERED_MIN_ROUNDS times the longest sequence's tiles of work for every CU."""
-    if seq_lens is None or head_dim is None or kv_dtype not in ORDERED_MIN_ROUNDS:
+    sequences first, than flat (the rule at ORDERED_MIN_ROUNDS): ragged, 2-byte KV,
+    and more workgroups than two a CU and than the library leaves in batch order."""
+    if seq_lens is None or head_dim is None or kv_dtype not in ("fp16", "bf16"):
         return False
-    lens = _Lens.of(seq_lens)
+    lens, cus = _Lens.of(seq_lens), max(1, sm_count)
     units = _units(num_kv_heads, group)
-    if lens.size > ORDERED_MAX_BATCH or lens.size * units <= 2 * sm_count or _nearly_uniform(lens):
+    if (lens.size > ORDERED_MAX_BATCH or lens.size * units <= max(2 * cus, ORDERED_MIN_WORKGROUPS)
+            or _nearly_uniform(lens)):
         return False
-    rounds = ORDERED_MIN_ROUNDS_SHORT_ROWS if head_dim * _KV_ELEM_BYTES[kv_dtype] <= UNSPLIT_MIN_ROW_BYTES \
-        and _KV_ELEM_BYTES[kv_dtype] == 2 else ORDERED_MIN_ROUNDS[kv_dtype]
-    return lens.tiles * units >= rounds * _tiles(lens.longest) * sm_count
+    kv_bytes = lens.total * num_kv_heads * head_dim * 4 / cus
+    rounds = lens.tiles * units / (_tiles(lens.longest) * cus)
+    if head_dim * 2 <= UNSPLIT_MIN_ROW_BYTES:
+        return rounds >= (ORDERED_MIN_ROUNDS_SHORT_ROWS if kv_bytes <= ORDERED_SHORT_ROWS_BYTES_PER_CU
+                          else ORDERED_MIN_ROUNDS_SHORT_ROWS_LARGE)
+    least, most = ORDERED_KV_BYTES_PER_CU
+    return group >= ORDERED_MIN_GROUP and rounds >= ORDERED_MIN_ROUNDS and least <= kv_bytes <= most
 
 
 def packed_splits_for(seq_lens, plan: LaunchPlan, num_kv_heads: int, group: int, sm_count: int,

@@ -18,6 +18,7 @@ from pagedattn.hip_decode import (
     FEW_SPLIT_SHARE_TILES,
     FEW_SPLITS_MAX,
     MIN_SPLIT_TILES,
+    ORDERED_MAX_BATCH,
     PACKED_MERGE_TILES,
     PACKED_SHARE,
     PACKED_SHARE_ONE_EACH,
@@ -27,6 +28,7 @@ from pagedattn.hip_decode import (
     UNSPLIT_MAX_CHUNK_TILES,
     UNSPLIT_MAX_TILES,
     few_splits,
+    ordered_batch_runs_unsplit,
     plan_num_splits,
 )
 
@@ -237,3 +239,59 @@ def test_batches_with_little_work():
         seen.add((fits, want))
     assert seen >= {(True, 1), (False, 2), (False, 3)}
     assert classic([32 * 25] * 20, "fp16", 8, 4, 128, False) == few_splits(20, 800, 8, 4, 256) == 1
+
+
+def ordered_lens(tiles, longest, others):
+    """A batch of `tiles` tiles in all: one sequence of `longest`, the others of about `others`."""
+    lens = [32 * longest] + [32 * others] * ((tiles - longest) // others)
+    lens[-1] += 32 * (tiles - sum(n // 32 for n in lens))
+    return lens
+
+
+@pytest.mark.parametrize("kv,head_dim,hkv,group,rounds,longest,others", [
+    ("fp16", 128, 8, 8, 2.5, 30, 14), ("bf16", 128, 8, 4, 2.5, 40, 12), ("fp16", 64, 8, 7, 1.0, 100, 20),
+    ("fp16", 64, 8, 7, 2.0, 200, 60)])
+def test_ordered_batches_by_rounds(kv, head_dim, hkv, group, rounds, longest, others):
+    """Unsplit with the longest first: from `rounds` times the longest sequence's tiles of work a CU."""
+    def ordered(lens, kv=kv, cus=256, hkv=hkv, group=group, head_dim=head_dim):
+        return ordered_batch_runs_unsplit(lens, hkv, group, cus, kv, head_dim)
+
+    lens = ordered_lens(int(rounds * longest * 256) // hkv, longest, others)
+    assert len(lens) * hkv > 512 and ordered(lens)
+    lens[-1] -= 32
+    assert not ordered(lens)
+    lens[-1] += 32
+    # 1-byte types, unknown heads or lengths, a uniform batch
+    assert not ordered(lens, kv="int8") and not ordered(lens, kv="fp8_e5m2") and not ordered(lens, kv=None)
+    assert not ordered(lens, head_dim=None) and not ordered(None)
+    assert not ordered([32 * longest] * len(lens))
+
+
+def test_ordered_batches_by_size():
+    def ordered(lens, hkv=8, group=8, cus=256, head_dim=128):
+        return ordered_batch_runs_unsplit(lens, hkv, group, cus, "fp16", head_dim)
+
+    # K/V a CU between the limits (8 heads of 256 bytes, K and V: 16 bytes a token and CU)
+    lens = [600] + [200] * 400
+    assert ordered(lens)
+    small = [90] + [40] * 817
+    small[1] += 32768 - sum(small)
+    assert 16 * sum(small) == 512 << 10 and ordered(small)
+    small[2] -= 1
+    assert not ordered(small)
+    large = [600] + [250] * 520
+    large[1] += 131072 - sum(large)
+    assert 16 * sum(large) == 2 << 20 and ordered(large)
+    large[2] += 1
+    assert not ordered(large)
+    # few q heads a kv head
+    assert ordered(lens, group=4) and not ordered(lens, group=3)
+    # two workgroups a CU or fewer, and no fewer than the library orders on a smaller device
+    few = [300] + [130] * 99
+    assert not ordered(few[:64], cus=64) and ordered(few[:65], cus=64)
+    # rows of 128 bytes: up to 1.5 MB a CU from one round on (above: two)
+    rows = ordered_lens(100 * 256 // 8, 100, 20)
+    assert ordered(rows, group=7, head_dim=64)
+    # batches beyond the order's size
+    many = [64] + [33] * (ORDERED_MAX_BATCH - 1)
+    assert ordered(many) and not ordered(many + [33])
