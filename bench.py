@@ -626,6 +626,13 @@ def _loop_us(step, n: int, repeats: int) -> list[float]:
     return [evs[2 * r].elapsed_time(evs[2 * r + 1]) * 1e3 / n for r in range(repeats)]
 
 
+def planned_launch(plan) -> tuple[int, int]:
+    """(num_splits, flat_splits) that a call with this plan's keywords launches
+    on a contiguous cache, as the workloads' caches are."""
+    kw = plan.launch_kwargs()
+    return kw.get("num_splits", 1), kw.get("flat_splits", 0)
+
+
 def measure(cfg: str, args, dev, cpu: bool) -> dict:
     """Time one BASELINE config on the GPU and check it. Returns the numbers
     and, under "_keep", the inputs (for the headline's CPU baseline)."""
@@ -665,7 +672,7 @@ def measure(cfg: str, args, dev, cpu: bool) -> dict:
     wps = flat_waves_per_simd(wl.kv_dtype, shape.head_dim, sdt)
     plan = plan_launch(wl.batch, 0, shape.num_kv_heads, shape.gqa_group, cus, wps,
                        kv_dtype=wl.kv_dtype, head_dim=shape.head_dim, seq_lens=wl.lens)
-    splits, flat, cost = plan.num_splits, plan.flat_splits, plan.flat_seq_cost
+    (splits, flat), cost = planned_launch(plan), plan.flat_seq_cost
     if args.flat is not None or args.splits:
         flat = int(args.flat or 0)
         splits = 1 if flat else (args.splits or

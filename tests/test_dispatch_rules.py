@@ -126,6 +126,22 @@ def test_plans_for_pairs_carry_the_launch_without_them():
     assert short.flat_splits == 0 and short.num_splits == 1 and "unpaired" not in short.launch_kwargs()
 
 
+def test_the_bench_times_the_planned_launch():
+    """Splits and flat ranges as the plan's keywords give them, cut for pairs of heads or not."""
+    import pathlib
+    import sys
+
+    sys.path.insert(0, str(pathlib.Path(__file__).resolve().parent.parent))
+    import bench
+
+    plan = plan_launch(256, 0, 2, 7, 256, 2, kv_dtype="int8", head_dim=64, seq_lens=[2048] * 256)
+    assert plan.packed_splits == 1 and plan.flat_splits > 0 and bench.planned_launch(plan) == (1, 0)
+    plan = plan_launch(64, 0, 8, 4, 256, 2, kv_dtype="fp16", head_dim=128, seq_lens=[4096] * 64)
+    assert bench.planned_launch(plan) == (1, plan.flat_splits) and plan.flat_splits > 0
+    plan = plan_launch(1, 0, 8, 4, 256, 2, kv_dtype="fp16", head_dim=128, seq_lens=[2048])
+    assert bench.planned_launch(plan) == (plan.num_splits, 0) and plan.num_splits > 1
+
+
 def packed(lens, kv="int8", hkv=2, cus=256):
     return plan_launch(len(lens), 0, hkv, 7, cus, 2, kv_dtype=kv, head_dim=64, seq_lens=lens).packed_splits
 
