@@ -311,6 +311,52 @@ def test_boundary_plans_as_the_wrapper_with_host_lengths(monkeypatch, shape, kv)
             (len(lens), max(lens))
 
 
+def _wrapper_launch(monkeypatch, lens, kv, shape):
+    """What `paged_decode_hip(q, cache)` itself launches for the batch, in `launch_kwargs` form."""
+    from pagedattn import ModelShape, PagedKVCache, hip_decode
+
+    hq, hkv, d = shape
+    seen = []
+    monkeypatch.setattr(hip_decode, "_cu_count", lambda dev: 256)
+    monkeypatch.setattr(hip_decode, "flat_waves_per_simd", lambda *a: 1)
+    monkeypatch.setattr(hip_decode._WS, "pointers", lambda *a: (256, 256))
+    monkeypatch.setattr(hip_decode, "_fill_args", lambda q, cache, out, splits, scale, part_out, part_lse, msl, flat,
+                        cost, host, workspace: seen.append((splits, msl, flat, cost, host)))
+    monkeypatch.setattr(hip_decode, "_launch", lambda *a: 0)
+    t = torch.tensor(lens, dtype=torch.int32)
+    cache = PagedKVCache(shape=ModelShape(hq, hkv, d, "w"), block_size=16, kv_dtype=kv, k_cache=None, v_cache=None,
+                         k_scale=None, v_scale=None, block_table=None, seq_lens=t)
+    hip_decode.paged_decode_hip(torch.zeros(len(lens), hq, d, dtype=torch.float16), cache)
+    (splits, msl, flat, cost, host), = seen
+    assert host.tolist() == t.tolist()
+    return {"flat_splits": flat, "flat_seq_cost": cost} if flat else {"num_splits": splits, "max_seq_len": msl}
+
+
+@pytest.mark.parametrize("shape", [(32, 8, 128), (64, 8, 128), (14, 2, 64)], ids=["8b", "70b", "qwen"])
+@pytest.mark.parametrize("kv", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
+def test_boundary_launches_as_the_default_call(monkeypatch, shape, kv):
+    """With the step's lengths on the host, the boundary launches what a call with q and the cache alone
+    launches, except the ragged batches that such a call runs unsplit, longest first: the boundary
+    keeps the flat split there, as `plan_launch` gives it."""
+    from pagedattn.hip_decode import ordered_batch_runs_unsplit
+
+    hq, hkv, d = shape
+    name = "bf16" if kv == torch.bfloat16 else "fp16"
+    g = torch.Generator().manual_seed(2)
+    batches = [[t] * b for b, t in UNIFORM if b * t <= 2_000_000]
+    batches += [torch.randint(lo, hi, (b,), generator=g).tolist() for b in (3, 17, 64, 160, 300, 512, 1000)
+                for lo, hi in ((1, 300), (32, 1023), (200, 3000), (1000, 16000)) if b * hi <= 4_000_000]
+    ordered = 0
+    for lens in batches:
+        want, got = _wrapper_launch(monkeypatch, lens, name, shape), _boundary_plan(monkeypatch, lens, kv=kv, shape=shape)
+        if "flat_splits" in got and ordered_batch_runs_unsplit(lens, hkv, hq // hkv, 256, name, d):
+            ordered += 1
+            assert want == {"num_splits": 1, "max_seq_len": max(lens)}, (len(lens), max(lens))
+        else:
+            assert got == want, (len(lens), max(lens))
+    assert ordered > 0
+
+
 @pytest.mark.parametrize("shape", [(32, 8, 128), (64, 8, 128), (14, 2, 64)], ids=["8b", "70b", "qwen"])
 def test_boundary_without_host_lengths_on_uniform_batches(monkeypatch, shape):
     """Metadata with device-only lengths: the boundary plans from the batch
