@@ -68,6 +68,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "launch_math.h"
 #include "pagedattn.h"
 #include "pa_errors.h"
 
@@ -89,7 +90,6 @@ constexpr int kFlatWaves = 4;      // flat kernel: one wave per SIMD of a CU (2-
 constexpr int kFlatWavesInt8 = 8;
 template <int KV> constexpr int flat_waves() { return KV == PA_KV_INT8 ? kFlatWavesInt8 : kFlatWaves; }
 inline int flat_waves_of(int kv) { return kv == PA_KV_INT8 ? kFlatWavesInt8 : kFlatWaves; }
-constexpr int kSplitAlign = 32;    // split ranges are multiples of this many tokens
 constexpr float kRescaleLog2 = 8.0f;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr uint32_t kInt8Sign = 0x80808080u;      // int8 x -> x + 128 in every byte
@@ -108,32 +108,6 @@ constexpr int kDeepTiles = 16;
 // on the GPU instead.
 constexpr int kHostTab = PA_HOST_TABLE_MAX;
 constexpr uint32_t kMaxTiles = (1u << 26) - 1;  // 32-token tiles of the longest sequence (2^31 tokens)
-
-// Division of an n < 2^31 by a d that the host knows: floor(n / d) = n * mul >>
-// (32 + shift), mul = floor(2^(31 + l) / d) + 1, l = ceil(log2 d), shift = l -
-// 1 (Granlund and Montgomery's division by an invariant). A general 32-bit
-// division is ~25 dependent instructions in front of a kernel's first loads
-// and a 64-bit one ~150; with these the classic split's two kernels start
-// their loads 0.4 us earlier: whole calls at the Llama-3-8B shape, graph-timed,
-// B = 1, T = 2048 8.7 -> 8.3 us, B = 8, T <= 2500 17.0 -> 16.5, unsplit B = 24,
-// T <= 192 (Qwen2.5-0.5B shape) 4.66 -> 4.49.
-struct Div {
-  uint32_t d, mul, shift;
-};
-
-inline Div make_div(uint32_t d) {
-  Div v = {d, 0, 0};
-  if (d > 1) {
-    const uint32_t l = 32 - __builtin_clz(d - 1);
-    v.mul = (d & (d - 1)) == 0 ? 0x80000001u : (uint32_t)((uint64_t(1) << (31 + l)) / d + 1);
-    v.shift = l - 1;
-  }
-  return v;
-}
-
-__device__ __forceinline__ uint32_t div_by(uint32_t n, const Div &v) {
-  return v.d == 1 ? n : __umulhi(n, v.mul) >> v.shift;
-}
 
 struct KParams {
   const uint8_t *q;
@@ -167,13 +141,6 @@ struct KParams {
   // Neighbouring kv heads that one wave takes as one of pack times the head
   // dim: then hkv counts packs, and group and skh are a pack's.
   int32_t pack;
-};
-
-// The classic split's division of a sequence: tiles of a split of max_seq_len
-// tokens (0: not given), and the divisors.
-struct SplitDiv {
-  int32_t max_seq_len, chunk_tiles;
-  Div by_splits, by_chunk;
 };
 
 // The classic kernel's arguments. (The flat kernel keeps the smaller ones: its
@@ -951,36 +918,6 @@ __device__ __forceinline__ void regroup(float *y, const float *o, float scale) {
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int sl = 0; sl < kE; ++sl) y[kE * i + sl] = o[4 * sl + i] * scale;
-}
-
-// Token range [lo, hi) of one split, and how many of the sequence's splits
-// hold tokens. chunk = ceil(ceil(T / 32) / S) * 32 tokens, T = the sequence's
-// length (the reference's per-sequence rule, triton_decode.py:78-85), or the
-// chunk of a max_seq_len-token sequence when max_seq_len > 0 and that is
-// larger (ragged batches: long sequences take all S splits, short ones few;
-// never below the sequence's own chunk, so no token is dropped).
-struct SplitRange {
-  int lo, hi, n;
-};
-
-__device__ __forceinline__ SplitRange split_range(int seq_len, const SplitDiv &p, int split) {
-  static_assert(kSplitAlign == 32, "lengths are counted in 32-token tiles");
-  const uint32_t tiles = ((uint32_t)seq_len + 31) >> 5;  // < 2^27
-  uint32_t chunk = (uint32_t)p.chunk_tiles;
-  uint32_t n;
-  if (chunk != 0 && seq_len <= p.max_seq_len) {
-    n = div_by(tiles + chunk - 1, p.by_chunk);
-  } else {
-    // T = 0 still has one split
-    chunk = max(max(div_by(tiles + p.by_splits.d - 1, p.by_splits), chunk), 1u);
-    n = (tiles + chunk - 1) / chunk;
-  }
-  const uint32_t lo = min((uint32_t)split * chunk, tiles);
-  SplitRange r;
-  r.lo = (int)min(lo << 5, (uint32_t)seq_len);
-  r.hi = (int)min(min(lo + chunk, tiles) << 5, (uint32_t)seq_len);
-  r.n = max(1, (int)n);
-  return r;
 }
 
 // What a workgroup does with its result:
@@ -1971,16 +1908,6 @@ int ilog2(int x) {
   int r = 0;
   while ((1 << r) < x) ++r;
   return r;
-}
-
-SplitDiv split_div(int max_seq_len, int num_splits) {
-  const uint32_t tiles = ((uint32_t)max_seq_len + kSplitAlign - 1) / kSplitAlign;
-  SplitDiv s;
-  s.max_seq_len = max_seq_len;
-  s.chunk_tiles = (int)((tiles + num_splits - 1) / num_splits);
-  s.by_splits = make_div(num_splits);
-  s.by_chunk = make_div(std::max(1, s.chunk_tiles));
-  return s;
 }
 
 // Whether the classic kernel takes two kv heads as one of twice the head dim
