@@ -665,7 +665,8 @@ def plan_decode(seq_lens, num_kv_heads: int, group: int, sm_count: int,
                 waves_per_simd: int = 1, kv_dtype: str | None = None,
                 head_dim: int | None = None) -> tuple[int, int, int]:
     """(num_splits, max_seq_len, flat_splits) for a batch whose lengths the
-    host knows: `plan_launch` with the lengths."""
+    host knows: `plan_launch` with the lengths, without pairs of heads (its
+    `launch_kwargs` has the launch with them)."""
     lens = _Lens.of(seq_lens)
     p = plan_launch(lens.size, 0, num_kv_heads, group, sm_count, waves_per_simd, kv_dtype,
                     head_dim, seq_lens=lens)
@@ -1039,7 +1040,9 @@ def _stream(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
-_get_device = getattr(torch._C, "_cuda_getDevice", None)
+_get_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+_current_stream = _raw_stream or (lambda idx: torch.cuda.current_stream(idx).cuda_stream)
+_byref = ctypes.byref
 
 
 def _launch(t: torch.Tensor, fn, args) -> int:
@@ -1048,12 +1051,10 @@ def _launch(t: torch.Tensor, fn, args) -> int:
     every wrapper: a device index and the raw stream handle, no device or
     stream objects."""
     idx = t.get_device()
-    cur = _get_device() if _get_device is not None else torch.cuda.current_device()
-    if idx == cur:
-        return fn(ctypes.byref(args), _raw_stream(idx) if _raw_stream is not None
-                  else torch.cuda.current_stream(idx).cuda_stream)
+    if idx == _get_device():
+        return fn(_byref(args), _current_stream(idx))
     with torch.cuda.device(idx):
-        return fn(ctypes.byref(args), _stream(torch.device("cuda", idx)))
+        return fn(_byref(args), _stream(torch.device("cuda", idx)))
 
 
 def paged_decode_hip(
@@ -1102,9 +1103,9 @@ def paged_decode_hip(
     `seq_lens_host` (an addition): the lengths as a contiguous int32 CPU
     tensor equal to `cache.seq_lens`, when the caller has them (a serving
     step's metadata usually does). A large unsplit launch starts the longest
-    sequences first (results do not depend on it). A flat launch then takes its ranges and
-    its merge list from the host (no seq_lens scan on the GPU, no merge
-    launch when no sequence is cut or empty). With `num_splits=None` the
+    sequences first (results do not depend on it). A flat launch then takes
+    its ranges and its merge list from the host (no seq_lens scan on the GPU,
+    no merge launch when no sequence is cut or empty). With `num_splits=None` the
     lengths come to the host anyway and are used so.
 
     `unpaired` (an addition, from `LaunchPlan.launch_kwargs`): `num_splits` was

@@ -263,3 +263,26 @@ def test_argument_cache_tells_strided_slots():
     one = rows[:1]
     reshape_and_cache(one, one, c, wide[::8])  # one slot: any stride
     assert torch.equal(c.k_cache.view(-1, 2, 64)[0], rows[0])
+
+
+@pytest.mark.parametrize("scale_dtype", [torch.float16, torch.float32])
+def test_int8_rows_of_every_maximum(scale_dtype):
+    """A row for every finite fp16 magnitude as its maximum, the elements spread over the row or next to
+    half-integer quotients: scales and bytes equal the oracle's."""
+    top = torch.arange(1, 0x7C00, dtype=torch.int16).view(torch.float16)
+    n, d = top.numel(), 64
+    g = torch.Generator().manual_seed(56)
+    a = top.float()[:, None]
+    x = (torch.rand((n, d), generator=g) * 2 - 1) * a
+    half = (torch.randint(-127, 127, (n, d // 2), generator=g) + 0.5) * (a / 127)  # quotients near k + 1/2
+    x[:, : d // 2] = half
+    x = x.half().clamp(-top[:, None], top[:, None])
+    x[:, 7] = top
+    c = allocate(ModelShape(1, 1, d, "m"), 1, [-(-n // 16) * 16], kv_dtype="int8", scale_dtype=scale_dtype, seed=57,
+                 device="cuda", fill_device="cuda")
+    ref = _cpu_copy(c)
+    rows, slots = x[:, None], torch.arange(n)
+    reshape_and_cache(rows.cuda(), -rows.cuda(), c, slots.cuda())
+    oracle.write_kv(rows, -rows, ref, slots)
+    assert torch.equal(c.k_scale.cpu(), ref.k_scale) and torch.equal(c.v_scale.cpu(), ref.v_scale)
+    assert torch.equal(c.k_cache.cpu(), ref.k_cache) and torch.equal(c.v_cache.cpu(), ref.v_cache)
