@@ -11,8 +11,10 @@
 //             stays NaN, as torch's cast does
 //   int8      amax over head_dim (clamped to 1e-6), scale = amax / 127 rounded
 //             to the scale type, q = round_half_even(x / scale) clamped to
-//             +-127; fp32 IEEE division throughout, so the bytes equal
-//             torch's
+//             +-127. Bytes and scales are those of fp32 IEEE division, as
+//             torch's: amax / 127 is a product corrected by its remainder,
+//             x / scale a product with the reciprocal, and the division itself
+//             in lanes where the two could round to different integers
 //
 // One (token, kv_head) row per D/8 lanes, 16 bytes (8 fp16) per lane; the
 // int8 row maximum is a DPP reduction inside those lanes. A workgroup holds
