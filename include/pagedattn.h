@@ -157,18 +157,18 @@ typedef struct pa_decode_args {
    * suits ragged batches. pa_flat_merge must be given the same value. */
   int32_t flat_seq_cost;
   /* Also an addition: the lengths in host memory, NULL when the caller has
-   * none. Unsplit launches (num_splits 1, no flat split) of up to 1,024
-   * sequences and more than one round of workgroups start the longest sequences
-   * first (an order only: results do not depend on it, captured or not). Flat
-   * split: given, they must equal seq_lens. The library
-   * then computes the ranges and the merge's list of cut and empty
-   * sequences on the host and passes them in the kernel arguments, so no
+   * none: `batch` of them, whatever the launch. Unsplit launches (num_splits 1,
+   * no flat split) of up to 1,024 sequences and more than 512 workgroups start
+   * the longest sequences first where those are long (an order only: no result
+   * depends on it, and a captured launch keeps it). Flat split: given, they must
+   * equal seq_lens. The library then computes the ranges and the merge's list of
+   * cut and empty sequences on the host and passes them in the kernel arguments, so no
    * wave reads seq_lens before its first K/V loads and the merge covers only
    * the sequences that need it (and is not launched when none do). Launches
    * beyond PA_HOST_TABLE_MAX ranges or merge entries, a batch above 4096 or
    * sequences of 2^25 tokens and more use the GPU scan as without them.
-   * Read during the call only. Ignored while the stream is being captured
-   * into a HIP graph: tables in a graph's kernel arguments would be replayed
+   * Read during the call only. Flat launches ignore them while the stream is
+   * being captured into a HIP graph: tables in a graph's kernel arguments would be replayed
    * with whatever lengths seq_lens then holds, so captured launches scan. */
   const int32_t *seq_lens_host;
 } pa_decode_args;

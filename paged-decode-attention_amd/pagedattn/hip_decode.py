@@ -114,14 +114,18 @@ CLASSIC_MAX_CHUNK_TILES = {"fp16": 24, "bf16": 24, "fp8_e5m2": 32, "int8": 40}
 UNSPLIT_MAX_CHUNK_TILES = {"fp16": 32, "bf16": 32, "fp8_e5m2": 32, "int8": 40}
 # A batch with too little work for the flat split takes few_splits unless it is known
 # to be so ragged that the longest chunk is over FEW_SPLIT_SHARE times the tiles of
-# a CU, and FEW_SPLIT_SHARE_TILES: then more splits, as plan_num_splits cuts it,
-# spread its long sequences. Eager whole calls, plan_num_splits / few_splits in us:
-# int8, 8 q / 8 kv heads, B = 19, T log-uniform to 4320 34.0 (4) / 48.2 (1); Llama-3-8B
-# shape fp16 B = 20, T log-uniform to 2176 22.7 (3) / 27.7 (1), int8 B = 9, to 14816
-# 41.0 (8) / 56.2 (3). On 3,589 such random batches, few_splits always: 1.052 times as
-# fast (geometric mean; 122 lose over 5%, the worst half); by this rule 1.045 (11; 0.92).
+# a CU, and FEW_SPLIT_SHARE_TILES (FEW_UNSPLIT_SHARE_TILES unsplit, without a merge):
+# then more splits, as plan_num_splits cuts it, spread its long sequences. Eager whole
+# calls, plan_num_splits / few_splits in us: int8, 8 q / 8 kv heads, B = 19, T log-uniform
+# to 4320 34.0 (4) / 48.2 (1); Llama-3-8B shape fp16 B = 20, T log-uniform to 2176 22.7
+# (3) / 27.7 (1), int8 B = 9, to 14816 41.0 (8) / 56.2 (3); but 14 q / 2 kv heads fp16 B =
+# 76, T log-uniform to 380 7.3 (4) / 5.1 (1). On the 1,992 ragged ones of 4,708 random
+# batches for which the two choose different splits, against plan_num_splits
+# everywhere: this rule 1.067 times as fast (geometric mean; 18 lose over 5%, the worst
+# 0.86), few_splits everywhere 1.056 (155; 0.50).
 FEW_SPLIT_SHARE = 2.5
-FEW_SPLIT_SHARE_TILES = 2
+FEW_SPLIT_SHARE_TILES = 5
+FEW_UNSPLIT_SHARE_TILES = 18
 # few_splits: no more than this many while each holds less than
 # FEW_SPLIT_LONG_TILES (14 q / 2 kv heads, D = 64, fp16: B = 2, T = 4096 32 splits
 # 7.8, 64 8.8; T = 16384 10.0, 10.5; B = 1, T = 32768 64 splits 11.7, 32 12.6, 128
@@ -157,29 +161,33 @@ UNSPLIT_MIN_ROW_BYTES = 128
 UNSPLIT_MAX_SHORT_ROW_BYTES_PER_CU = 192 << 10
 # The classic kernel takes two 64-element kv heads of a 1-byte cache as one row
 # of 128 (`packs_heads`) and then streams such rows faster than the flat split,
-# but waits for the CU with the most to do: unsplit, or cut into the splits that
-# give every CU a workgroup (rounded up to a power of two), it is taken where
+# but waits for the CU with the most to do: unsplit, or cut into the fewest splits (a
+# power of two) up to those that give every CU a workgroup, it is taken where
 #   * the workgroups are many (PACKED_MANY_WORKGROUPS a CU; more where a token's
 #     row is wide, which the flat split streams better), or the longest chunk's
 #     tiles are at most a times the tiles of pairs that a CU gets, and c
 #     (PACKED_SHARE = a, c; PACKED_SHARE_ONE_EACH with no more workgroups than CUs),
-#     less PACKED_MERGE_TILES for the merge of a split launch, and
+#     less PACKED_MERGE_TILES for the merge of a split launch, or, lengths nearly
+#     uniform and rows not wide, at most PACKED_SHORT_CHUNK_TILES (fp8, B = 77, T =
+#     1469 13.6 / 10.9; 55 such batches 1.03 times as fast, the worst 0.94), and
 #   * no sequence is longer than PACKED_SPLIT_MAX_RAGGED times the mean.
-# Eager whole calls on 4,900 random batches that ran flat without pairs (1 to 700
-# sequences of up to 100,000 tokens, 256 CUs): where the rule takes pairs they are
-# 1.23 times as fast for int8, 1.16 for fp8 (geometric means; the worst 0.91 and
-# 0.92), elsewhere 0.86 and 0.89. Flat / pairs at 14 q / 2 kv heads in us: taken, int8
-# B = 192, T = 2047 (2 splits) 30.8 / 26.3, B = 256, T ~ U[128, 2047] 27.5 / 24.5; left,
-# int8 B = 192, T ~ U[128, 8000] (2 splits) 56.8 / 65.1, B = 160, T ~ U[128, 2047] 22.1 /
-# 22.9, fp8 B = 129, T ~ U[2100, 33660] (2 splits) 105.7 / 175.9. With lengths log-
-# uniform over a factor of 64 (longest 4 times the mean) flat wins: B = 32 fp8 21.3 /
-# 27.4, B = 256 int8 31.8 / 44.1.
+# Eager whole calls on 4,961 random batches that ran flat without pairs (1 to 700
+# sequences of up to 100,000 tokens, 256 CUs): by this rule 1.107 times as fast for
+# int8, 1.068 for fp8 (geometric means; taken in half of them, the worst 0.91 and 0.92;
+# the best of every launch timed 1.118 and 1.080; pairs everywhere 1.01). Flat / pairs
+# at 14 q / 2 kv heads in us: taken, int8 B = 192, T = 2047 (2 splits) 30.8 / 26.3, B =
+# 256, T ~ U[128, 2047] 27.5 / 24.5, fp8 B = 213, T ~ U[40, 651] 14.1 / 8.4 unsplit, 12.9
+# in two; left, int8 B = 192, T ~ U[128, 8000] (2 splits) 56.8 / 65.1, B = 160, T ~ U[128,
+# 2047] 22.1 / 22.9, fp8 B = 129, T ~ U[2100, 33660] (2 splits) 105.7 / 175.9. With
+# lengths log-uniform over a factor of 64 (longest 4 times the mean) flat wins: B = 32
+# fp8 21.3 / 27.4, B = 256 int8 31.8 / 44.1.
 PACKED_MANY_WORKGROUPS = 2.0
 PACKED_MANY_WORKGROUPS_WIDE = 2.75
 PACKED_WIDE_ROW_BYTES = {"fp8_e5m2": 512}
 PACKED_SHARE = {"fp8_e5m2": (0.6, 21), "int8": (0.9, 24)}
 PACKED_SHARE_ONE_EACH = {"fp8_e5m2": (1.1, 30), "int8": (1.1, 39)}
 PACKED_MERGE_TILES = {"fp8_e5m2": 18, "int8": 27}
+PACKED_SHORT_CHUNK_TILES = 16
 PACKED_SPLIT_MAX_RAGGED = 2.25
 # The library takes pairs from this many workgroups of them on, whatever the
 # device, and for chunks of more tokens than this (kPackMinWorkgroups and
@@ -238,21 +246,21 @@ FLAT_MAX_BATCH = 1024
 # A ragged batch whose lengths the call itself reads (num_splits=None) runs
 # unsplit with its longest sequences first, instead of flat, where no CU then waits
 # for one sequence and no wave switches sequences every few tiles: 2-byte KV only,
-# from ORDERED_MIN_ROUNDS times the longest sequence's tiles a CU on, with
-# ORDERED_MIN_GROUP q heads a kv head or more and ORDERED_KV_BYTES_PER_CU of K/V.
+# from ORDERED_MIN_ROUNDS times the longest sequence's tiles a CU on, with the K/V a
+# CU that ORDERED_KV_BYTES_PER_CU gives for a number of q heads a kv head and more.
 # Rows of 128 bytes (head_dim 64), whose flat split has four times the ranges to
 # merge: from ORDERED_MIN_ROUNDS_SHORT_ROWS on up to ORDERED_SHORT_ROWS_BYTES_PER_CU,
 # beyond that from ORDERED_MIN_ROUNDS_SHORT_ROWS_LARGE.
 # Eager calls of 2,091 random batches with host lengths (256 CUs), flat / ordered: the
-# rule's batches at head_dim 128 and 256 1.05 times as fast, the worst 0.93;
-# outside it 8 q heads a kv head under 250 KB a CU 0.96, 4 under 500 KB 0.95 and over 2
-# MB 0.99, 1 head 0.95; int8 0.85 (the worst 0.44), at any length; head_dim 64 1.15 to
-# 2.0, over 1.5 MB and under 2 rounds 0.97. In us: Llama-3-70B shape fp16 B = 160, T ~
-# U[32, 1023] 64.8 / 59.4; 14 q / 2 kv heads, D = 64, fp16 B = 300, T ~ U[64, 1500]
-# 28.2 / 24.1, B = 512, T ~ U[32, 800] 32.0 / 21.9.
+# rule's batches at head_dim 128 and 256 1.06 times as fast with 8 q heads a kv head
+# (the worst 1.00), 1.03 with 4 (0.93); outside it 8 q heads under 250 KB a CU 0.94, 4
+# under 500 KB 0.95 and over 2 MB 0.99, 1 head 0.95; int8 0.85 (the worst 0.44), at any
+# length; head_dim 64 1.15 to 2.0, over 1.5 MB and under 2 rounds 0.97. In us:
+# Llama-3-70B shape fp16 B = 160, T ~ U[32, 1023] 64.8 / 59.4, B = 243, T ~ U[133, 2135]
+# 217 / 204; 14 q / 2 kv heads, D = 64, fp16 B = 300, T ~ U[64, 1500] 28.2 / 24.1, B =
+# 512, T ~ U[32, 800] 32.0 / 21.9.
 ORDERED_MIN_ROUNDS = 2.5
-ORDERED_MIN_GROUP = 4
-ORDERED_KV_BYTES_PER_CU = (512 << 10, 2 << 20)
+ORDERED_KV_BYTES_PER_CU = {8: (256 << 10, 6 << 20), 4: (512 << 10, 2 << 20)}
 ORDERED_MIN_ROUNDS_SHORT_ROWS = 1.0
 ORDERED_MIN_ROUNDS_SHORT_ROWS_LARGE = 2.0
 ORDERED_SHORT_ROWS_BYTES_PER_CU = 1536 << 10
@@ -571,18 +579,20 @@ def ordered_batch_runs_unsplit(seq_lens, num_kv_heads: int, group: int, sm_count
     if head_dim * 2 <= UNSPLIT_MIN_ROW_BYTES:
         return rounds >= (ORDERED_MIN_ROUNDS_SHORT_ROWS if kv_bytes <= ORDERED_SHORT_ROWS_BYTES_PER_CU
                           else ORDERED_MIN_ROUNDS_SHORT_ROWS_LARGE)
-    least, most = ORDERED_KV_BYTES_PER_CU
-    return group >= ORDERED_MIN_GROUP and rounds >= ORDERED_MIN_ROUNDS and least <= kv_bytes <= most
+    for heads, (least, most) in ORDERED_KV_BYTES_PER_CU.items():
+        if group >= heads:
+            return rounds >= ORDERED_MIN_ROUNDS and least <= kv_bytes <= most
+    return False
 
 
 def packed_splits_for(seq_lens, plan: LaunchPlan, num_kv_heads: int, group: int, sm_count: int,
                       kv_dtype: str | None, head_dim: int | None) -> int:
     """Splits of the classic kernel where it takes pairs of heads (`packs_heads`)
     and beats `plan`. Instead of a flat split: the fewest, as a power of two, that
-    give every CU a workgroup, chunks of more than PACKED_MIN_TOKENS tokens, where
-    the rule at PACKED_SHARE says so. Instead of an unsplit launch with too few
-    workgroups for pairs: two. 0: `plan` stands (also for other geometries and
-    unknown lengths)."""
+    the rule at PACKED_SHARE accepts, up to the fewest that give every CU a
+    workgroup, chunks of more than PACKED_MIN_TOKENS tokens. Instead of an unsplit
+    launch with too few workgroups for pairs: two. 0: `plan` stands (also for other
+    geometries and unknown lengths)."""
     if seq_lens is None or not packs_heads(num_kv_heads, group, head_dim, kv_dtype):
         return 0
     lens, cus, tmax = _Lens.of(seq_lens), max(1, sm_count), plan.max_seq_len
@@ -593,17 +603,22 @@ def packed_splits_for(seq_lens, plan: LaunchPlan, num_kv_heads: int, group: int,
         if plan.num_splits > 1 or pairs >= PACKED_MIN_WORKGROUPS or 2 * pairs < max(cus, PACKED_MIN_WORKGROUPS):
             return 0
         return 2 if _tiles(tmax) >= PACKED_SPLIT_MIN_TILES else 0
-    while splits * pairs < cus and tmax > 2 * splits * PACKED_MIN_TOKENS:
-        splits *= 2
-    if splits * pairs < PACKED_MIN_WORKGROUPS or splits > _abi.PA_MAX_SPLITS:
-        return 0
     wide = num_kv_heads * head_dim >= PACKED_WIDE_ROW_BYTES.get(kv_dtype, 1 << 30)
-    if splits * pairs <= (PACKED_MANY_WORKGROUPS_WIDE if wide else PACKED_MANY_WORKGROUPS) * cus:
-        share, more = (PACKED_SHARE_ONE_EACH if splits * pairs <= cus else PACKED_SHARE)[kv_dtype]
-        most = share * lens.tiles * (num_kv_heads // 2) / cus + more
-        if -(-_tiles(tmax) // splits) > most - (PACKED_MERGE_TILES[kv_dtype] if splits > 1 else 0):
-            return 0
-    return splits
+    many = (PACKED_MANY_WORKGROUPS_WIDE if wide else PACKED_MANY_WORKGROUPS) * cus
+    a_cu, uniform = lens.tiles * (num_kv_heads // 2) / cus, _nearly_uniform(lens)
+    while tmax > splits * PACKED_MIN_TOKENS and splits <= _abi.PA_MAX_SPLITS:
+        workgroups = splits * pairs
+        if workgroups >= PACKED_MIN_WORKGROUPS:
+            share, more = (PACKED_SHARE_ONE_EACH if workgroups <= cus else PACKED_SHARE)[kv_dtype]
+            most = share * a_cu + more - (PACKED_MERGE_TILES[kv_dtype] if splits > 1 else 0)
+            if uniform and not wide:
+                most = max(most, PACKED_SHORT_CHUNK_TILES)
+            if workgroups > many or -(-_tiles(tmax) // splits) <= most:
+                return splits
+            if workgroups >= cus:
+                return 0
+        splits *= 2
+    return 0
 
 
 def _plan_launch(batch, max_seq_len, num_kv_heads, group, sm_count, waves_per_simd, kv_dtype, head_dim,
@@ -630,8 +645,8 @@ def _plan_launch(batch, max_seq_len, num_kv_heads, group, sm_count, waves_per_si
         else:
             classic = chunk <= (UNSPLIT_MAX_CHUNK_TILES if splits == 1 else CLASSIC_MAX_CHUNK_TILES)[kv_dtype]
         if not flat_ok:  # the other choice is plan_num_splits, below
-            classic = (not known or _nearly_uniform(lens)
-                       or chunk <= FEW_SPLIT_SHARE * tiles * units / cus + FEW_SPLIT_SHARE_TILES)
+            more = FEW_UNSPLIT_SHARE_TILES if splits == 1 else FEW_SPLIT_SHARE_TILES
+            classic = not known or _nearly_uniform(lens) or chunk <= FEW_SPLIT_SHARE * tiles * units / cus + more
         elif known and packs_heads(num_kv_heads, group, head_dim, kv_dtype):
             classic = False  # packed_splits_for chooses between the flat split and pairs
         if classic:

@@ -17,11 +17,13 @@ from pagedattn.hip_decode import (
     FEW_SPLIT_SHARE,
     FEW_SPLIT_SHARE_TILES,
     FEW_SPLITS_MAX,
+    FEW_UNSPLIT_SHARE_TILES,
     MIN_SPLIT_TILES,
     ORDERED_MAX_BATCH,
     PACKED_MERGE_TILES,
     PACKED_SHARE,
     PACKED_SHARE_ONE_EACH,
+    PACKED_SHORT_CHUNK_TILES,
     PACKED_SPLIT_MAX_RAGGED,
     PACKED_SPLIT_MIN_TILES,
     UNSPLIT_MARGIN_TILES,
@@ -146,20 +148,26 @@ def packed(lens, kv="int8", hkv=2, cus=256):
     return plan_launch(len(lens), 0, hkv, 7, cus, 2, kv_dtype=kv, head_dim=64, seq_lens=lens).packed_splits
 
 
-@pytest.mark.parametrize("kv,batch,splits,others", [
-    ("int8", 274, 1, 100), ("int8", 180, 2, 120), ("int8", 128, 2, 200), ("int8", 256, 1, 200),
-    ("fp8_e5m2", 274, 1, 30), ("fp8_e5m2", 240, 2, 80), ("fp8_e5m2", 64, 4, 400), ("fp8_e5m2", 256, 1, 100)])
-def test_pairs_instead_of_flat(kv, batch, splits, others):
-    """Few workgroups: taken while the longest chunk is within its share, on both sides of the line."""
-    share, more = (PACKED_SHARE_ONE_EACH if batch * splits <= 256 else PACKED_SHARE)[kv]
-    seen = set()
-    for longest in range(others, 2 * others + 1):
-        lens = [32 * longest] + [32 * others] * (batch - 1)
+@pytest.mark.parametrize("kv,batch,others,seen", [
+    ("int8", 274, 100, {1, 0}), ("int8", 180, 120, {2, 0}), ("int8", 128, 200, {2, 0}), ("int8", 256, 200, {1, 0}),
+    ("int8", 230, 100, {1, 2, 0}), ("fp8_e5m2", 274, 30, {1, 0}), ("fp8_e5m2", 190, 40, {2, 0}),
+    ("fp8_e5m2", 64, 400, {4, 0}), ("fp8_e5m2", 256, 100, {1, 0}), ("fp8_e5m2", 200, 60, {1, 0})])
+def test_pairs_instead_of_flat(kv, batch, others, seen):
+    """Few workgroups: the fewest splits whose longest chunk is within its share, on both sides of the line."""
+    def fits(splits, longest):
+        share, more = (PACKED_SHARE_ONE_EACH if batch * splits <= 256 else PACKED_SHARE)[kv]
         most = share * (longest + (batch - 1) * others) / 256 + more - (PACKED_MERGE_TILES[kv] if splits > 1 else 0)
-        fits = -(-longest // splits) <= most
-        assert packed(lens, kv) == (splits if fits else 0), longest
-        seen.add(fits)
-    assert seen == {True, False}
+        uniform = longest <= 1.25 * (longest + (batch - 1) * others) / batch
+        return -(-longest // splits) <= max(most, PACKED_SHORT_CHUNK_TILES if uniform else 0)
+
+    got = set()
+    for longest in range(others, 9 * others // 4):
+        lens = [32 * longest] + [32 * others] * (batch - 1)
+        choices = [s for s in (1, 2, 4) if batch * s >= 192 and (s == 1 or batch * s // 2 < 256)]
+        want = next((s for s in choices if fits(s, longest)), 0)
+        assert packed(lens, kv) == want, longest
+        got.add(want)
+    assert got >= seen
 
 
 def test_pairs_limits():
@@ -180,7 +188,7 @@ def test_pairs_limits():
     assert packed([32 * 200] + [32 * 100] * 174, "int8", 8) == 1
     # 1-byte types only; the fewest splits, as a power of two, that give every CU a workgroup of pairs
     assert packed([8192] * 256, "fp16") == packed([8192] * 256, "bf16") == 0
-    assert [packed([8192] * b) for b in (256, 250, 128, 120, 64, 60)] == [1, 2, 2, 4, 4, 8]
+    assert [packed([8192] * b) for b in (256, 250, 191, 128, 120, 95, 64, 60)] == [1, 1, 2, 2, 2, 4, 4, 4]
     # an unsplit launch with too few workgroups for pairs is cut in two from PACKED_SPLIT_MIN_TILES on
     t = 32 * PACKED_SPLIT_MIN_TILES
     assert packed([t] * 132) == 2 and packed([t - 32] * 132) == 0 and packed([t] * 127) == 0 and packed([t] * 192) == 0
@@ -243,17 +251,20 @@ def test_few_split_ragged_batches(kv, hkv, group):
     assert seen == {(4, 4), (4, 0), (1, 1), (1, 0)}
 
 
-def test_batches_with_little_work():
+@pytest.mark.parametrize("batch,others", [(20, 5), (10, 8)])  # 160 and 80 workgroups unsplit
+def test_batches_with_little_work(batch, others):
     """Too little for the flat split: few_splits, or the splits of plan_num_splits where the longest chunk
     is known to be far over a CU's share; without lengths few_splits."""
     seen = set()
-    for longest in range(9, 200):
-        lens = [32 * longest] + [32 * 5] * 19  # 160 workgroups unsplit, under 512 tiles
-        fits = longest <= FEW_SPLIT_SHARE * (longest + 95) * 8 / 256 + FEW_SPLIT_SHARE_TILES
-        want = few_splits(20, max(lens), 8, 4, 256) if fits else plan_num_splits(lens, 8, 4, 256)[0]
+    for longest in range(2 * others, 300):
+        lens = [32 * longest] + [32 * others] * (batch - 1)
+        few = few_splits(batch, max(lens), 8, 4, 256)
+        more = FEW_UNSPLIT_SHARE_TILES if few == 1 else FEW_SPLIT_SHARE_TILES
+        fits = -(-longest // few) <= FEW_SPLIT_SHARE * (longest + (batch - 1) * others) * 8 / 256 + more
+        want = few if fits else plan_num_splits(lens, 8, 4, 256)[0]
         assert classic(lens, "fp16", 8, 4, 128) == want, longest
-        seen.add((fits, want))
-    assert seen >= {(True, 1), (False, 2), (False, 3)}
+        seen.add((fits, want != few))
+    assert seen >= {(True, False), (False, True)}
     assert classic([32 * 25] * 20, "fp16", 8, 4, 128, False) == few_splits(20, 800, 8, 4, 256) == 1
 
 
@@ -287,21 +298,21 @@ def test_ordered_batches_by_size():
     def ordered(lens, hkv=8, group=8, cus=256, head_dim=128):
         return ordered_batch_runs_unsplit(lens, hkv, group, cus, "fp16", head_dim)
 
-    # K/V a CU between the limits (8 heads of 256 bytes, K and V: 16 bytes a token and CU)
+    # K/V a CU between the limits of the number of q heads (8 kv heads of 256 bytes, K and V: 16 bytes a
+    # token and CU)
+    def batch(tokens, longest, others):
+        lens = [longest] + [others] * ((tokens - longest) // others)
+        lens[1] += tokens - sum(lens)
+        return lens
+
+    for group, least, most in ((8, 256, 6144), (16, 256, 6144), (7, 512, 2048), (4, 512, 2048)):
+        small, large = batch(least << 6, 90, 40), batch(most << 6, 900, 400)
+        assert ordered(small, group=group) and ordered(large, group=group)
+        small[2] -= 1
+        large[2] += 1
+        assert not ordered(small, group=group) and not ordered(large, group=group)
     lens = [600] + [200] * 400
-    assert ordered(lens)
-    small = [90] + [40] * 817
-    small[1] += 32768 - sum(small)
-    assert 16 * sum(small) == 512 << 10 and ordered(small)
-    small[2] -= 1
-    assert not ordered(small)
-    large = [600] + [250] * 520
-    large[1] += 131072 - sum(large)
-    assert 16 * sum(large) == 2 << 20 and ordered(large)
-    large[2] += 1
-    assert not ordered(large)
-    # few q heads a kv head
-    assert ordered(lens, group=4) and not ordered(lens, group=3)
+    assert ordered(lens, group=4) and not ordered(lens, group=3) and not ordered(lens, group=1)
     # two workgroups a CU or fewer, and no fewer than the library orders on a smaller device
     few = [300] + [130] * 99
     assert not ordered(few[:64], cus=64) and ordered(few[:65], cus=64)
