@@ -192,6 +192,8 @@ def test_pairs_limits():
     # an unsplit launch with too few workgroups for pairs is cut in two from PACKED_SPLIT_MIN_TILES on
     t = 32 * PACKED_SPLIT_MIN_TILES
     assert packed([t] * 132) == 2 and packed([t - 32] * 132) == 0 and packed([t] * 127) == 0 and packed([t] * 192) == 0
+    # where the flat split stands, pairs come before the few-workgroup classic split
+    assert packed([5090] * 32) == 8 and classic([5090] * 32, "int8", 2, 7, 64) == 0
 
 
 def classic(lens, kv, hkv, group, head_dim, known=True, cus=256):
